@@ -17,6 +17,7 @@
 // LDS, double-buffered, one global load per workgroup per tile; column sums accumulate
 // in-lane over the wave's 16 queries, then in an LDS ring of 16 tiles that is added to the
 // scores once per ring. Query blocks are dispatched heaviest (longest causal range) first.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -28,16 +29,16 @@ namespace pf {
 constexpr int D = 64;
 constexpr int GROUP = 8;
 constexpr int QB = 64;          // queries per workgroup
-// Row-blocks (2 queries each) per wave: pass 1 keeps a running maximum and sum per row, so it
-// runs 8 waves of 4 row-blocks; pass 2 keeps one normaliser per row and runs 4 waves of 8.
-template <int PASS> constexpr int rows_per_wave() { return PASS == 1 ? 4 : 8; }
-template <int PASS> constexpr int waves() { return QB / (2 * rows_per_wave<PASS>()); }
+constexpr int RB2 = 8;          // pass 2: row-blocks (2 queries each) per wave
+constexpr int WAVES = QB / (2 * RB2);
 constexpr int KT = 64;          // keys per tile (4 key-blocks of 16)
 constexpr int KROW = D + 8;     // padded bf16 row of a staged key
 constexpr int RING = 16;        // tiles of column sums held before they are added to the scores
-// A row's reference moves (to the tile's maximum) when a sum of four of its terms passes 2^8,
-// which a key more than 8 above the reference always causes.
-constexpr float kRescaleSum = 256.f;
+// A row's reference follows its sums: past kMoveSum it moves up by a power of two (exponents near
+// zero keep the exponential's argument exact), past kRescaleSum, near the overflow, to the tile's
+// maximum.
+constexpr float kMoveSum = 64.f;
+constexpr float kRescaleSum = 0x1p64f;
 }  // namespace pf
 
 struct PrefillArgs {
@@ -59,7 +60,301 @@ struct PrefillArgs {
   float* norm2;  // [count, q_heads] row normalisers in log2 units (sink included)
   int delay;     // pass 2 credits query i's keys k <= prefix_len + i - delay only
   int block_shift;  // kind 4: log2 of the block size
+  // Pass 1's key ranges: at most `splits`, of at most `tiles` 64-key tiles; part[(range * count + query) *
+  // q_heads + head] = (reference, sum of 2^(x - reference)) of the row over that range.
+  float2* part;
+  int splits, tiles;
 };
+
+// ---------------------------------------------------------------------------
+// Pass 1: row normalisers
+// ---------------------------------------------------------------------------
+// S^T = K . Q^T in 32x32x16 MFMAs: a lane holds 16 keys of one (query, head) row, so a row needs
+// one reference and one sum per lane, and its terms add up in the lane. A workgroup (8 waves x 8
+// queries) takes one KV head, 64 queries and a range of at most `tiles` 64-key tiles of what
+// they see; prefill_merge_kernel joins the ranges' (reference, sum) pairs and the sink. Per logit the
+// walk issues one FMA, one exponential and one add, all on vector registers, 4 waves per SIMD
+// (128 VGPRs). Bound by vector issue: 329 cycles per 1024 logits and SIMD over a long walk where the
+// instructions alone take 283, and by the card's power there (1.9 GHz). Against 16x16x32 MFMAs with
+// 2 waves per SIMD and whole causal ranges: 87 -> 43 us for the first 2048 tokens of a prompt, 816
+// -> 665 us for 1896 tokens after 30,720, 3.36 -> 2.75 ms for 8192 after 28,672.
+namespace p1 {
+constexpr int QW = 8;                // queries per wave: two column blocks of 4 queries x 8 heads
+constexpr int WAVES = 8;
+constexpr int THREADS = 64 * WAVES;
+static_assert(QW * WAVES == pf::QB, "a workgroup's queries");
+// Work items of a launch: enough for several rounds of the 512 workgroups the chip holds (2 per
+// CU), at least MIN_TILES tiles each, which keeps an item's start (query and first key loads)
+// below a third of its time.
+constexpr int ITEMS = 3072;
+constexpr int MIN_TILES = 4;
+}  // namespace p1
+
+// Key ranges of a query block that sees ntiles tiles (equal ones, of at most `tiles` tiles).
+GSE_DEVICE int key_ranges(int ntiles, int tiles) { return (ntiles + tiles - 1) / tiles; }
+
+GSE_DEVICE float sum16(const f32x16_t& p) {
+  return (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]))) +
+         (((p[8] + p[9]) + (p[10] + p[11])) + ((p[12] + p[13]) + (p[14] + p[15])));
+}
+
+// Key block kb's fragments of a staged K tile (lane: key 32*kb + lane%32, dims 16*ks + 8*(lane/32)).
+GSE_DEVICE void k_fragments(const uint16_t* kt, int kb, int lane, bf16x8_t (&ka)[4]) {
+  const uint16_t* kr = kt + (32 * kb + (lane & 31)) * pf::KROW + 8 * (lane >> 5);
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) ka[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(kr + 16 * ks));
+}
+
+GSE_DEVICE f32x16_t dot64(const bf16x8_t (&a)[4], const bf16x8_t (&b)[4]) {
+  f32x16_t d = {};
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) d = mfma32x32x16(a[ks], b[ks], d);
+  return d;
+}
+
+// Logits of keys past a lane's causal bound become -inf: register i of a block holds key
+// first + 8*(i/4) + i%4, dead when past `bound` (both relative to the same origin).
+GSE_DEVICE void mask_keys(f32x16_t& d, int first, int bound) {
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (first + 8 * (i / 4) + i % 4 > bound) d[i] = -INFINITY;
+}
+
+// One tile of a wave: ts[rb] = the lane's sum of 2^(x * scale2 + nref[rb]) over its 32 keys, nref
+// the negated reference, a whole number. When a sum passes kMoveSum, its row's reference takes the
+// sum's exponent and both sums are scaled by that power of two (exact); when one passes kRescaleSum
+// (rows whose first keys were all masked, or logits over 40 above them) the references of the
+// wave's rows move to their tile maximum and the tile is formed again.
+// MASKED: key 32*kb + 8*(i/4) + i%4 of the tile is dead past bound + 4*rb.
+template <bool MASKED>
+GSE_DEVICE void row_sum_tile(const uint16_t* kt, const bf16x8_t (&qf)[2][4], float (&nref)[2], float (&sum)[2],
+                             float scale2, int bound, int lane) {
+  using namespace pf;
+  float ts[2];
+  {
+    bf16x8_t ka[4];
+    k_fragments(kt, 0, lane, ka);
+    f32x16_t dn = dot64(ka, qf[0]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {  // (key block, column block) pairs, the next one's MFMAs issued ahead
+      const int kb = u >> 1, rb = u & 1;
+      f32x16_t d = dn;
+      if (u == 1) k_fragments(kt, 1, lane, ka);
+      if (u < 3) dn = dot64(ka, qf[(u + 1) & 1]);
+      if (MASKED) mask_keys(d, 32 * kb, bound + 4 * rb);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) d[i] = fast_exp2(fmaf(d[i], scale2, nref[rb]));
+      ts[rb] = kb == 0 ? sum16(d) : ts[rb] + sum16(d);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  const float tsmax = fmaxf(ts[0], ts[1]);
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(tsmax > kMoveSum) == 0, 1)) {
+    sum[0] += ts[0];
+    sum[1] += ts[1];
+    return;
+  }
+  if (__builtin_amdgcn_ballot_w64(tsmax > kRescaleSum)) {
+#pragma unroll 1
+    for (int rb = 0; rb < 2; ++rb) {
+      bf16x8_t q[4];
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) q[ks] = rb == 0 ? qf[0][ks] : qf[1][ks];
+      const float old = rb == 0 ? nref[0] : nref[1];
+      float tmax = -INFINITY;
+#pragma unroll 1
+      for (int kb = 0; kb < 2; ++kb) {
+        bf16x8_t ka[4];
+        k_fragments(kt, kb, lane, ka);
+        f32x16_t d = dot64(ka, q);
+        if (MASKED) mask_keys(d, 32 * kb, bound + 4 * rb);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, d[i]);
+      }
+      const float nr = fminf(old, -rintf(tmax * scale2));
+      float t = 0.f;
+#pragma unroll 1
+      for (int kb = 0; kb < 2; ++kb) {
+        bf16x8_t ka[4];
+        k_fragments(kt, kb, lane, ka);
+        f32x16_t d = dot64(ka, q);
+        if (MASKED) mask_keys(d, 32 * kb, bound + 4 * rb);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) d[i] = fast_exp2(fmaf(d[i], scale2, nr));
+        t += sum16(d);
+      }
+      const float keep = fast_exp2(nr - old);
+      if (rb == 0) {
+        sum[0] *= keep;
+        nref[0] = nr;
+        ts[0] = t;
+      } else {
+        sum[1] *= keep;
+        nref[1] = nr;
+        ts[1] = t;
+      }
+    }
+  }
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const int e = ts[rb] > kMoveSum && ts[rb] <= kRescaleSum ? __builtin_amdgcn_frexp_expf(ts[rb]) : 0;
+    nref[rb] -= float(e);
+    sum[rb] = ldexpf(sum[rb] + ts[rb], -e);
+  }
+}
+
+__global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArgs a) {
+  using namespace pf;
+  using p1::QW;
+  __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Block i: KV head i % kv_heads, then the query block from the end (the longest causal ranges
+  // first), then the key range. Blocks go to an XCD's shader engines in turn, whatever these have
+  // left to do, so ranges of different lengths must not alternate with the block index.
+  const int nqb = int((a.count + QB - 1) / QB);
+  const int g = blockIdx.x % a.kv_heads;
+  const int item = blockIdx.x / a.kv_heads;
+  const int split = item / nqb;
+  const int64_t qb0 = int64_t(nqb - 1 - item % nqb) * QB;
+  const int last_q = int((qb0 + QB < a.count ? qb0 + QB : a.count) - 1);
+  const int kend = int(a.prefix_len) + last_q + 1;  // keys any query of the workgroup sees
+  const int ntiles = (kend + KT - 1) / KT;
+  const int ranges = key_ranges(ntiles, a.tiles);
+  if (split >= ranges) return;
+  const int ti0 = int(int64_t(ntiles) * split / ranges), ti1 = int(int64_t(ntiles) * (split + 1) / ranges);
+  const int i0 = int(qb0) + QW * wave;  // this wave's first query
+  const bool wave_live = i0 < a.count;
+  const int wave_kend = int(a.prefix_len) + min(i0 + QW - 1, int(a.count) - 1) + 1;
+
+  // B fragments: column lane%32 of block rb is query i0 + 4*rb + (lane%32)/8, head g*8 + lane%8.
+  bf16x8_t qf[2][4];
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const int64_t qi = i0 + 4 * rb + ((lane & 31) >> 3);
+    const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * GROUP + (lane & 7)) * a.q_sh + 8 * (lane >> 5);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      qf[rb][ks] = qi < a.count ? as_bf16x8(*reinterpret_cast<const uint4*>(qp + 16 * ks)) : bf16x8_t{};
+  }
+  float nref[2] = {1e30f, 1e30f};  // finite, so fully masked rows give 2^(-inf) = 0, never NaN
+  float sum[2] = {0.f, 0.f};
+  const float scale2 = in_vgpr(a.scale2);
+
+  // Tile load: thread t stages 16 bytes of key t/8. Tile t's K rows are loaded into registers
+  // during tile t - 2 and stored to LDS at the end of tile t - 1, and its slot indices are read
+  // two tiles before that, in two register sets alternating by tile parity (the loop is unrolled
+  // by two: copying one into the other would wait for the loads in flight into it). Keys past
+  // kend read slot 0's row (any valid row) and are masked.
+  const int lk = threadIdx.x >> 3, lp = threadIdx.x & 7;
+  auto slot_at = [&](int ti) -> int32_t {
+    const int key = ti * KT + lk;
+    return key < kend ? int32_t(load_index_dyn(a.slots, a.slots_dtype, key)) : 0;
+  };
+  const auto kbase = as_global(a.k) + int64_t(g) * a.kv_sh + 8 * lp;
+  auto load_row = [&](int32_t s) { return gload16(kbase + int64_t(s) * a.kv_ss); };
+  auto store_row = [&](int p, const uint4& x) { *reinterpret_cast<uint4*>(&ktile[p][lk * KROW + 8 * lp]) = x; };
+  uint4 xk[2];    // xk[p]: K rows of the tile of offset parity p in flight
+  int32_t sk[2];  // sk[p]: slot of the next tile of parity p whose rows are not yet loaded
+  {
+    const int32_t s0 = slot_at(ti0), s1 = slot_at(ti0 + 1);
+    sk[0] = slot_at(ti0 + 2);
+    sk[1] = slot_at(ti0 + 3);
+    const uint4 y = load_row(s0);
+    xk[1] = load_row(s1);
+    store_row(0, y);
+  }
+  // The query fragments are in registers before the walk starts: a wait for them inside the
+  // loop would also wait for every load in flight at the top of each tile.
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) landed(qf[rb][ks]);
+  __syncthreads();
+
+  const int qpos = int(a.prefix_len) + i0 + ((lane & 31) >> 3) - 4 * (lane >> 5);  // the lane's causal bound
+  {  // Each row's reference: the maximum over the lane's keys of the range's first 32.
+    bf16x8_t ka[4];
+    k_fragments(ktile[0], 0, lane, ka);
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+      f32x16_t d = dot64(ka, qf[rb]);
+      mask_keys(d, 0, qpos + 4 * rb - ti0 * KT);
+      float m = d[0];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) m = fmaxf(m, d[i]);
+      nref[rb] = fminf(nref[rb], -rintf(m * scale2));
+    }
+  }
+
+  // The tiles every wave sees whole (below the workgroup's first query) run in a loop of their
+  // own with no causal mask (a wave past the chunk's end computes rows nobody reads, with zero
+  // queries); the rest choose per wave.
+  auto tile_step = [&](int ti, auto general, auto parity) {
+    constexpr bool GENERAL = decltype(general)::value;
+    constexpr int P = decltype(parity)::value;  // (ti - ti0) & 1
+    xk[P] = load_row(sk[P]);
+    sk[P] = slot_at(ti + 4);
+    const int t0 = ti * KT;
+    if (!GENERAL)
+      row_sum_tile<false>(ktile[P], qf, nref, sum, scale2, 0, lane);
+    else if (wave_live && t0 < wave_kend)
+      row_sum_tile<true>(ktile[P], qf, nref, sum, scale2, qpos - t0, lane);
+    if (ti + 1 < ti1) store_row(1 - P, xk[1 - P]);
+    __syncthreads();
+  };
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+  const int whole = int((a.prefix_len + qb0 + 1) / KT);  // tiles whose keys the first query sees
+  const int common = ti0 + (max(min(ti1, whole) - ti0, 0) & ~1);
+  int ti = ti0;
+#pragma unroll 1
+  for (; ti < common; ti += 2) {
+    tile_step(ti, std::false_type{}, P0{});
+    tile_step(ti + 1, std::false_type{}, P1{});
+  }
+#pragma unroll 1
+  for (; ti < ti1; ti += 2) {
+    tile_step(ti, std::true_type{}, P0{});
+    if (ti + 1 < ti1) tile_step(ti + 1, std::true_type{}, P1{});
+  }
+
+  // The row's pair over both lane halves.
+#pragma unroll
+  for (int rb = 0; rb < 2; ++rb) {
+    const float other = lane_xor32(nref[rb]);
+    const float nr = fminf(nref[rb], other);
+    const float total = xor32_sum(sum[rb] * fast_exp2(nr - nref[rb]));
+    const int64_t qi = i0 + 4 * rb + ((lane & 31) >> 3);
+    if (lane < 32 && qi < a.count)
+      a.part[(split * a.count + qi) * a.q_heads + g * GROUP + (lane & 7)] = float2{-nr, total};
+  }
+}
+
+// Row normalisers in log2 units: thread = (query, head), joining the key ranges that hold keys of
+// the row's query block and the sink.
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t n = a.count * a.q_heads;
+  if (t >= n) return;
+  const int64_t qb0 = t / a.q_heads / pf::QB * pf::QB;
+  const int64_t kend = a.prefix_len + (qb0 + pf::QB < a.count ? qb0 + pf::QB : a.count);
+  const int ranges = key_ranges(int((kend + pf::KT - 1) / pf::KT), a.tiles);
+  float m = load_float_dyn(a.sinks, a.sinks_dtype, t % a.q_heads) * kLog2e, l = 1.f;
+  for (int s0 = 0; s0 < ranges; s0 += 8) {  // eight ranges' loads in flight together
+    float2 p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = a.part[int64_t(min(s0 + j, ranges - 1)) * n + t];
+    float mn = m;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) mn = fmaxf(mn, p[j].x);
+    l *= fast_exp2(m - mn);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) l += s0 + j < ranges ? p[j].y * fast_exp2(p[j].x - mn) : 0.f;
+    m = mn;
+  }
+  a.norm2[t] = m + __log2f(l);
+}
 
 // Row-block rb's logits of a 64-key tile: D = Q . K^T for four 16-key blocks (MFMA rows are
 // (query, head) pairs, a lane's four values of block kb are rows 4*(grp%2)..+3 of query
@@ -78,59 +373,13 @@ GSE_DEVICE void prefill_mask(f32x4_t (&d)[4], int rb, int64_t rel, int grp) {
   }
 }
 
-// Pass 1's row sums of one row-block over a tile: ts[r] = sum over this lane's four keys of
-// 2^(x * scale2 - ref[r]).
-GSE_DEVICE void prefill_row_sums(const f32x4_t (&d)[4], const float (&ref)[4], float scale2, float (&ts)[4]) {
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float e0 = fast_exp2(fmaf(d[0][r], scale2, -ref[r]));
-    const float e1 = fast_exp2(fmaf(d[1][r], scale2, -ref[r]));
-    const float e2 = fast_exp2(fmaf(d[2][r], scale2, -ref[r]));
-    const float e3 = fast_exp2(fmaf(d[3][r], scale2, -ref[r]));
-    ts[r] = (e0 + e1) + (e2 + e3);
-  }
-}
-
-// Pass 1's rare path: some row sum of the tile passed kRescaleSum, so a key may lie more than
-// 8 above its row's reference. Every row's reference moves up to its maximum over the tile
-// (its sum rescaled: exact), so keys near that maximum send no later tile here, and the
-// tile's row sums are formed again (the logits again from the MFMAs).
-template <bool MASKED, int RB>
-GSE_DEVICE void prefill_rescale(const bf16x8_t (&qa)[RB][2], const bf16x8_t (&kb0)[4], const bf16x8_t (&kb1)[4],
-                                float (&ref)[RB][4], float (&sum)[RB][4], float (&ts)[RB][4], float scale2,
-                                int64_t rel, int grp) {
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    f32x4_t d[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      d[kb] = mfma16x16x32(qa[rb][0], kb0[kb], f32x4_t{0.f, 0.f, 0.f, 0.f});
-      d[kb] = mfma16x16x32(qa[rb][1], kb1[kb], d[kb]);
-    }
-    prefill_mask<MASKED>(d, rb, rel, grp);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float tmax = fmaxf(fmaxf(d[0][r], d[1][r]), fmaxf(d[2][r], d[3][r])) * scale2;
-      const float nr = fmaxf(ref[rb][r], tmax);
-      sum[rb][r] *= fast_exp2(ref[rb][r] - nr);
-      ref[rb][r] = nr;
-    }
-    prefill_row_sums(d, ref[rb], scale2, ts[rb]);
-  }
-}
-
 // One 64-key tile of a wave: row-block rb's MFMAs for four 16-key blocks, then per logit one
-// FMA + exp2 (+ the add). Row-block rb + 1's MFMAs are issued before rb's exponentials. Pass 1
-// tests its row sums once per tile (one branch per tile, not per row-block: a branch on a
-// vector result waits for the exponentials behind it), through their running maximum (two
-// v_max3 per row-block in place of four compares).
-template <int PASS, bool MAX_MODE, bool MASKED, int RB>
+// FMA + exp2 (+ the add). Row-block rb + 1's MFMAs are issued before rb's exponentials.
+template <bool MAX_MODE, bool MASKED, int RB>
 GSE_DEVICE void prefill_tile(const bf16x8_t (&qa)[RB][2], const bf16x8_t (&kb0)[4], const bf16x8_t (&kb1)[4],
-                             float (&ref)[RB][4], float (&sum)[RB][4], float (&cs)[4], float scale2,
+                             const float (&ref)[RB][4], float (&cs)[4], float scale2,
                              int64_t rel, int grp) {
   using namespace pf;
-  float ts[RB][4];
-  float tsmax = 0.f;  // the tile's largest row sum (sums are in [0, +inf]: never NaN)
   f32x4_t dn[4];
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
@@ -150,26 +399,18 @@ GSE_DEVICE void prefill_tile(const bf16x8_t (&qa)[RB][2], const bf16x8_t (&kb0)[
       }
     }
     prefill_mask<MASKED>(d, rb, rel, grp);
-    if (PASS == 1) {
-      // Row sums of 2^(x - ref) over this lane's four keys; a sum past kRescaleSum may hide a
-      // key more than 8 above the reference.
-      prefill_row_sums(d, ref[rb], scale2, ts[rb]);
-      tsmax = fmaxf(fmaxf(tsmax, ts[rb][0]), ts[rb][1]);  // two v_max3 per row-block
-      tsmax = fmaxf(fmaxf(tsmax, ts[rb][2]), ts[rb][3]);
-    } else {
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        if (MAX_MODE) {  // the largest probability is 2^(largest exponent): one exponential
-          const float y = fmaxf(fmaxf(fmaf(d[kb][0], scale2, -ref[rb][0]), fmaf(d[kb][1], scale2, -ref[rb][1])),
-                                fmaxf(fmaf(d[kb][2], scale2, -ref[rb][2]), fmaf(d[kb][3], scale2, -ref[rb][3])));
-          cs[kb] += fast_exp2(xor16_max(y));
-        } else {
-          const float p0 = fast_exp2(fmaf(d[kb][0], scale2, -ref[rb][0]));
-          const float p1 = fast_exp2(fmaf(d[kb][1], scale2, -ref[rb][1]));
-          const float p2 = fast_exp2(fmaf(d[kb][2], scale2, -ref[rb][2]));
-          const float p3 = fast_exp2(fmaf(d[kb][3], scale2, -ref[rb][3]));
-          cs[kb] += (p0 + p1) + (p2 + p3);
-        }
+    for (int kb = 0; kb < 4; ++kb) {
+      if (MAX_MODE) {  // the largest probability is 2^(largest exponent): one exponential
+        const float y = fmaxf(fmaxf(fmaf(d[kb][0], scale2, -ref[rb][0]), fmaf(d[kb][1], scale2, -ref[rb][1])),
+                              fmaxf(fmaf(d[kb][2], scale2, -ref[rb][2]), fmaf(d[kb][3], scale2, -ref[rb][3])));
+        cs[kb] += fast_exp2(xor16_max(y));
+      } else {
+        const float p0 = fast_exp2(fmaf(d[kb][0], scale2, -ref[rb][0]));
+        const float p1 = fast_exp2(fmaf(d[kb][1], scale2, -ref[rb][1]));
+        const float p2 = fast_exp2(fmaf(d[kb][2], scale2, -ref[rb][2]));
+        const float p3 = fast_exp2(fmaf(d[kb][3], scale2, -ref[rb][3]));
+        cs[kb] += (p0 + p1) + (p2 + p3);
       }
     }
     // Alternate the next row-block's 8 MFMAs with this one's vector work (1 MFMA, then 6 vector
@@ -184,25 +425,17 @@ GSE_DEVICE void prefill_tile(const bf16x8_t (&qa)[RB][2], const bf16x8_t (&kb0)[
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (PASS == 1) {
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(tsmax > kRescaleSum) != 0, 0))
-      prefill_rescale<MASKED, RB>(qa, kb0, kb1, ref, sum, ts, scale2, rel, grp);
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) sum[rb][r] += ts[rb][r];
-  }
 }
 
-template <int PASS, bool MAX_MODE>
-__global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(PrefillArgs a) {
+template <bool MAX_MODE>
+__global__ __launch_bounds__(64 * pf::WAVES) void prefill_kernel(PrefillArgs a) {
   using namespace pf;
-  constexpr int RB = rows_per_wave<PASS>();
+  constexpr int RB = RB2;
   __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
-  __shared__ float ring[PASS == 2 ? RING * KT : 1];
+  __shared__ float ring[RING * KT];
   // Slots of the keys of two rings of tiles (the one being summed and the next), for the ring's
   // score atomics.
-  __shared__ int32_t ring_slot[PASS == 2 ? 2 * RING * KT : 1];
+  __shared__ int32_t ring_slot[2 * RING * KT];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -213,7 +446,7 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
   const int64_t i0 = qb0 + 2 * RB * wave;  // this wave's first query
   const int64_t last_q = (qb0 + QB < a.count ? qb0 + QB : a.count) - 1;
   // Pass 2 credits keys up to `shift` entries before each query's causal bound.
-  const int64_t shift = PASS == 2 ? a.delay : 0;
+  const int64_t shift = a.delay;
   const int64_t kend = a.prefix_len + last_q + 1 - shift;  // keys any query of the workgroup sees (scores)
   const bool wave_live = i0 < a.count;
   const int64_t wave_kend = a.prefix_len + (i0 + 2 * RB - 1 < a.count ? i0 + 2 * RB - 1 : a.count - 1) + 1 - shift;
@@ -234,21 +467,17 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
   }
   // This lane's output rows in row-block rb: query i0 + 2*rb + grp/2, heads hq0 + r.
   const int hq0 = g * GROUP + 4 * (grp & 1);
-  // Pass 1: per-row reference maximum (log2 units) and the sum of 2^(x - ref) over this lane's
-  // keys. Pass 2: the rows' normalisers (+inf for rows past the chunk: their terms are 0).
-  float ref[RB][4], sum[RB][4];
+  // The rows' normalisers (+inf for rows past the chunk: their terms are 0).
+  float ref[RB][4];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const int64_t qi = i0 + 2 * rb + (grp >> 1);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      ref[rb][r] = -1e30f;  // finite, so fully masked rows give 2^(-inf) = 0, never NaN
-      sum[rb][r] = 0.f;
-      if (PASS == 2) ref[rb][r] = qi < a.count ? a.norm2[qi * a.q_heads + hq0 + r] : INFINITY;
+      ref[rb][r] = qi < a.count ? a.norm2[qi * a.q_heads + hq0 + r] : INFINITY;
     }
   }
-  if (PASS == 2)
-    for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) ring[t] = 0.f;
+  for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) ring[t] = 0.f;
 
   // Cooperative tile load: thread t < 256 stages key t/4, dims [16*(t%4), +16). Tile t's K rows
   // are loaded into registers during tile t - 2 and stored to LDS at the end of tile t - 1, and
@@ -257,7 +486,7 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
   // tile parity (the loop is unrolled by two), so nothing is copied between them: a copy would
   // wait for the loads in flight into its source. Keys past kend read slot 0's row (any valid
   // row) and are never used.
-  const bool loader = threadIdx.x < 256;
+  constexpr bool loader = true;
   const int lk = (threadIdx.x >> 2) & 63, lp = threadIdx.x & 3;
   auto slot_at = [&](int64_t t0) -> int32_t {
     const int64_t key = t0 + lk;
@@ -276,7 +505,7 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
   // Pass 2 keeps each staged key's slot for its ring's score atomics: positions of tile t are
   // (t mod 2*RING) * KT, so the ring being summed and the next one never share them.
   auto keep_slot = [&](int ti, int32_t s) {
-    if (PASS == 2 && lp == 0) ring_slot[(ti % (2 * RING)) * KT + lk] = s;
+    if (lp == 0) ring_slot[(ti % (2 * RING)) * KT + lk] = s;
   };
   const int ntiles = int((kend + KT - 1) / KT);
   uint4 xk[2][2] = {};     // xk[p]: K rows of the tile of parity p in flight
@@ -300,21 +529,13 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
     landed(qa[rb][1]);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-      if (PASS == 2) landed(ref[rb][r]);
+      landed(ref[rb][r]);
   }
   __syncthreads();
 
-  // One tile of the walk. In pass 1 the tiles every wave sees whole (below the workgroup's
-  // first query) run in a loop of their own with no causal mask and no test of the wave's
-  // range (a wave past the chunk's end computes rows nobody reads, with zero queries): a loop
-  // whose body chooses between the masked and unmasked forms keeps each row's reference and
-  // sum in different registers on the two sides and copies them back every tile (a quarter
-  // of pass 1's vector instructions). Pass 2 keeps the one loop: its own copy of the unmasked
-  // loop is scheduled with every MFMA of the tile up front, which takes 256 VGPRs (one wave
-  // per SIMD, a third slower).
+  // One tile of the walk.
   const int64_t qpos0 = a.prefix_len + i0 - shift;  // the wave's first query's causal bound
-  auto tile_step = [&](int ti, auto general, auto parity) {
-    constexpr bool GENERAL = decltype(general)::value;
+  auto tile_step = [&](int ti, auto parity) {
     constexpr int P = decltype(parity)::value;  // ti & 1
     const int64_t t0 = int64_t(ti) * KT;
     // Tile ti + 2's rows (into the set tile ti's rows left) and tile ti + 4's slots go out.
@@ -323,7 +544,7 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
       keep_slot(ti + 2, sk[P]);
       sk[P] = slot_at(t0 + 4 * KT);
     }
-    if (!GENERAL || (wave_live && t0 < wave_kend)) {
+    if (wave_live && t0 < wave_kend) {
       const uint16_t* kt = ktile[ti & 1];
       bf16x8_t kb0[4], kb1[4];
 #pragma unroll
@@ -334,31 +555,29 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
       }
       // Keys past the wave's first query need the causal mask (at most the last two tiles).
       float cs[4] = {0.f, 0.f, 0.f, 0.f};
-      if (GENERAL && t0 + KT - 1 > qpos0)
-        prefill_tile<PASS, MAX_MODE, true, RB>(qa, kb0, kb1, ref, sum, cs, a.scale2, t0 + col - qpos0, grp);
+      if (t0 + KT - 1 > qpos0)
+        prefill_tile<MAX_MODE, true, RB>(qa, kb0, kb1, ref, cs, a.scale2, t0 + col - qpos0, grp);
       else
-        prefill_tile<PASS, MAX_MODE, false, RB>(qa, kb0, kb1, ref, sum, cs, a.scale2, 0, grp);
-      if (PASS == 2) {
-        // Sum mode: every lane group holds partial sums; max mode: groups 0/1 hold the even
-        // queries' (twice), 2/3 the odd ones'.
-        float* rt = ring + (ti % RING) * KT;
+        prefill_tile<MAX_MODE, false, RB>(qa, kb0, kb1, ref, cs, a.scale2, 0, grp);
+      // Sum mode: every lane group holds partial sums; max mode: groups 0/1 hold the even
+      // queries' (twice), 2/3 the odd ones'.
+      float* rt = ring + (ti % RING) * KT;
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-          const float tot = MAX_MODE ? xor32_sum(cs[kb]) : xor32_sum(xor16_sum(cs[kb]));
-          if (grp == 0) atomicAdd(&rt[16 * kb + col], tot);
-        }
+      for (int kb = 0; kb < 4; ++kb) {
+        const float tot = MAX_MODE ? xor32_sum(cs[kb]) : xor32_sum(xor16_sum(cs[kb]));
+        if (grp == 0) atomicAdd(&rt[16 * kb + col], tot);
       }
     }
     if (loader && ti + 1 < ntiles) store_rows(ti + 1, xk[1 - P]);
     __syncthreads();
-    if (PASS == 2 && ((ti + 1) % RING == 0 || ti + 1 == ntiles)) {
+    if ((ti + 1) % RING == 0 || ti + 1 == ntiles) {
       // Add the ring's tiles to the scores, one atomic per key per workgroup (the keys' slots
       // were kept in LDS when their rows were loaded).
       const int r0 = ((ti - ti % RING) % (2 * RING)) * KT;
       const int64_t base = int64_t(ti - ti % RING) * KT;
 #pragma unroll
-      for (int u = 0; u < RING * KT / (64 * waves<PASS>()); ++u) {
-        const int t = threadIdx.x + u * 64 * waves<PASS>();
+      for (int u = 0; u < RING * KT / (64 * WAVES); ++u) {
+        const int t = threadIdx.x + u * 64 * WAVES;
         if (base + t < kend)
           unsafeAtomicAdd(&a.scores[int64_t(g) * a.ssg + int64_t(ring_slot[r0 + t]) * a.sss], ring[t]);
         ring[t] = 0.f;
@@ -369,44 +588,10 @@ __global__ __launch_bounds__(64 * pf::waves<PASS>()) void prefill_kernel(Prefill
   using P0 = std::integral_constant<int, 0>;
   using P1 = std::integral_constant<int, 1>;
   int ti = 0;
-  if constexpr (PASS == 1) {
-    // Tiles whole for every wave: keys up to the workgroup's first query's causal bound (an
-    // even count, for the unrolled pairs).
-    const int64_t first_bound = a.prefix_len + qb0 - shift;
-    const int n_common = (first_bound + 1 >= KT ? int(min(int64_t(ntiles), (first_bound + 1) / KT)) : 0) & ~1;
-#pragma unroll 1
-    for (; ti < n_common; ti += 2) {
-      tile_step(ti, std::false_type{}, P0{});
-      tile_step(ti + 1, std::false_type{}, P1{});
-    }
-  }
 #pragma unroll 1
   for (; ti < ntiles; ti += 2) {
-    tile_step(ti, std::true_type{}, P0{});
-    if (ti + 1 < ntiles) tile_step(ti + 1, std::true_type{}, P1{});
-  }
-
-  if (PASS == 1 && wave_live) {
-    // Combine each row's (ref, sum) over the 16 key columns, then fold in the sink.
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float mm = ref[rb][r], ll = sum[rb][r];
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) {
-          const float mo = __shfl_xor(mm, o, kWave), lo = __shfl_xor(ll, o, kWave);
-          const float mn = fmaxf(mm, mo);
-          ll = ll * fast_exp2(mm - mn) + lo * fast_exp2(mo - mn);
-          mm = mn;
-        }
-        const int64_t qi = i0 + 2 * rb + (grp >> 1);
-        if (col == 0 && qi < a.count) {
-          const float sink2 = load_float_dyn(a.sinks, a.sinks_dtype, hq0 + r) * kLog2e;
-          const float mx = fmaxf(mm, sink2);
-          a.norm2[qi * a.q_heads + hq0 + r] = mx + __log2f(ll * fast_exp2(mm - mx) + fast_exp2(sink2 - mx));
-        }
-      }
+    tile_step(ti, P0{});
+    if (ti + 1 < ntiles) tile_step(ti + 1, P1{});
   }
 }
 
@@ -660,10 +845,10 @@ struct DiagArgs {
 // keys the spec has evicted, summed over keys and KV heads, times lost_scale. Geometry as pass 1
 // (8 waves x 4 row-blocks per workgroup of 64 queries); K tiles through LDS, column sums through
 // two LDS rings.
-__global__ __launch_bounds__(64 * pf::waves<1>()) void diagnose_kernel(DiagArgs da) {
+__global__ __launch_bounds__(64 * 8) void diagnose_kernel(DiagArgs da) {
   using namespace pf;
   const PrefillArgs& a = da.p;
-  constexpr int RB = rows_per_wave<1>();
+  constexpr int RB = 4;
   __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
   __shared__ float ring_sum[RING * KT], ring_max[RING * KT];
   const int lane = threadIdx.x & 63;
@@ -846,8 +1031,41 @@ __global__ __launch_bounds__(64 * pf::waves<1>()) void diagnose_kernel(DiagArgs 
 
 using namespace gse;
 
+// Upper bound of pass 1's key ranges for a chunk of `count` queries: row_plan's item count divides
+// by the mean tiles of a query block, at least half of the last one's.
+static int64_t max_splits(int64_t count, int kv_heads) {
+  const int64_t blocks = (count + pf::QB - 1) / pf::QB * kv_heads;
+  return blocks > 0 ? 2 * p1::ITEMS / blocks + 2 : 0;
+}
+
+static int64_t norm_bytes(int64_t count, int q_heads) { return ((count * q_heads * 4 + 255) / 256) * 256; }
+
 extern "C" int64_t gse_prefill_workspace_bytes(int64_t count, int q_heads) {
-  return ((count * q_heads * 4 + 255) / 256) * 256;
+  // The normalisers, then pass 1's (reference, sum) pairs.
+  const int64_t pairs = max_splits(count, q_heads / pf::GROUP) * count * q_heads * int64_t(sizeof(float2));
+  return norm_bytes(count, q_heads) + ((pairs + 255) / 256) * 256;
+}
+
+// Pass 1 and the merge: row normalisers of a chunk into a.norm2. Fills in a's workspace pointers
+// and the key ranges.
+static int launch_norms(PrefillArgs& a, void* workspace, hipStream_t s) {
+  a.norm2 = static_cast<float*>(workspace);
+  a.part = reinterpret_cast<float2*>(static_cast<char*>(workspace) + norm_bytes(a.count, a.q_heads));
+  const int64_t nqb = (a.count + pf::QB - 1) / pf::QB;
+  const int64_t first = (a.prefix_len + (a.count < pf::QB ? a.count : pf::QB) + pf::KT - 1) / pf::KT;
+  const int64_t last = (a.total + pf::KT - 1) / pf::KT;
+  const int64_t work = (first + last + 1) / 2 * nqb * a.kv_heads;  // tiles of the launch
+  const int64_t tiles = std::max<int64_t>(p1::MIN_TILES, (work + p1::ITEMS - 1) / p1::ITEMS);
+  a.tiles = int(tiles);
+  a.splits = int((last + tiles - 1) / tiles);
+  if (a.splits > max_splits(a.count, a.kv_heads)) return gse_fail(GSE_EINVAL, "prefill: key ranges past the workspace");
+  const int64_t blocks = nqb * a.kv_heads * a.splits;
+  if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
+  hipLaunchKernelGGL(prefill_norm_kernel, dim3(uint32_t(blocks)), dim3(p1::THREADS), 0, s, a);
+  if (int rc = gse_launch_check("prefill pass 1")) return rc;
+  const int64_t rows = a.count * a.q_heads;
+  hipLaunchKernelGGL(prefill_merge_kernel, dim3(uint32_t((rows + 255) / 256)), dim3(256), 0, s, a);
+  return gse_launch_check("prefill normalisers");
 }
 
 extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_stride_h, int64_t count,
@@ -882,10 +1100,10 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
   const int64_t blocks = (count + pf::QB - 1) / pf::QB * kv_heads;
   if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
   const dim3 grid{static_cast<uint32_t>(blocks)};
+  if (kind == GSE_SCORE_KIND_BLOCK_STEP && kv_heads > pb::WAVES)
+    return gse_fail(GSE_ESHAPE, "prefill: block counters need kv_heads <= 8");
+  if (int rc = launch_norms(a, workspace, s)) return rc;
   if (kind == GSE_SCORE_KIND_BLOCK_STEP) {
-    if (kv_heads > pb::WAVES) return gse_fail(GSE_ESHAPE, "prefill: block counters need kv_heads <= 8");
-    hipLaunchKernelGGL((prefill_kernel<1, false>), grid, dim3(64 * pf::waves<1>()), 0, s, a);
-    if (int rc = gse_launch_check("prefill pass 1")) return rc;
     const dim3 bgrid(static_cast<uint32_t>((count + pb::QB - 1) / pb::QB));
     if (slots_dtype == GSE_I64)
       hipLaunchKernelGGL(prefill_block_kernel<int64_t>, bgrid, dim3(pb::THREADS), 0, s, a);
@@ -894,13 +1112,9 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
     return gse_launch_check("prefill block counters");
   }
   if (kind == 2) {
-    hipLaunchKernelGGL((prefill_kernel<1, true>), grid, dim3(64 * pf::waves<1>()), 0, s, a);
-    if (int rc = gse_launch_check("prefill pass 1")) return rc;
-    hipLaunchKernelGGL((prefill_kernel<2, true>), grid, dim3(64 * pf::waves<2>()), 0, s, a);
+    hipLaunchKernelGGL((prefill_kernel<true>), grid, dim3(64 * pf::WAVES), 0, s, a);
   } else {
-    hipLaunchKernelGGL((prefill_kernel<1, false>), grid, dim3(64 * pf::waves<1>()), 0, s, a);
-    if (int rc = gse_launch_check("prefill pass 1")) return rc;
-    hipLaunchKernelGGL((prefill_kernel<2, false>), grid, dim3(64 * pf::waves<2>()), 0, s, a);
+    hipLaunchKernelGGL((prefill_kernel<false>), grid, dim3(64 * pf::WAVES), 0, s, a);
   }
   return gse_launch_check("prefill pass 2");
 }
@@ -944,8 +1158,7 @@ extern "C" int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_s
   const int64_t blocks = (count + pf::QB - 1) / pf::QB * kv_heads;
   if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "diagnose: chunk too large");
   const dim3 grid{static_cast<uint32_t>(blocks)};
-  hipLaunchKernelGGL((prefill_kernel<1, false>), grid, dim3(64 * pf::waves<1>()), 0, s, da.p);
-  if (int rc = gse_launch_check("diagnose pass 1")) return rc;
-  hipLaunchKernelGGL(diagnose_kernel, grid, dim3(64 * pf::waves<1>()), 0, s, da);
+  if (int rc = launch_norms(da.p, workspace, s)) return rc;
+  hipLaunchKernelGGL(diagnose_kernel, grid, dim3(64 * 8), 0, s, da);
   return gse_launch_check("diagnose pass 3");
 }

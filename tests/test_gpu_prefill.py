@@ -54,6 +54,42 @@ def test_prefill_scores_match_oracle(count, prefix_len, mode, delay):
     torch.testing.assert_close(st.scores, expected, rtol=1e-3, atol=1e-6)
 
 
+def _exact_scores(mode, q, keys, sinks, slots, prefix_len):
+    """[KV head, list entry] column sums or maxima of the exact probabilities, in 64 bits."""
+    count, total = q.shape[0], slots.numel()
+    hidden = torch.arange(total, device="cuda") > prefix_len + torch.arange(count, device="cuda")[:, None]
+    out = torch.zeros((8, total), dtype=torch.float64, device="cuda")
+    for g in range(8):
+        qg = q[:, 8 * g:8 * g + 8].double().transpose(0, 1)
+        x = (torch.matmul(qg, keys[slots, g].double().t().contiguous()) * 0.125).masked_fill(hidden, -torch.inf)
+        sink = sinks[8 * g:8 * g + 8].double().view(8, 1, 1)
+        p = torch.exp(x - torch.logaddexp(torch.logsumexp(x, -1, keepdim=True), sink))
+        out[g] = p.sum((0, 1)) if mode == 1 else p.amax(0).sum(0)
+    return out
+
+
+# Edges of the query blocks (8 per wave, 64 per workgroup), of the 64-key tiles and of the key
+# ranges (4 tiles or more), and logits that move a row's reference: by a factor over 2^6 from tile
+# to tile (scale 3), and past 2^64 (scale 40).
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("count,prefix_len,scale", [
+    (1, 255, 1), (1, 256, 1), (7, 0, 1), (8, 63, 1), (9, 64, 1), (63, 449, 1), (64, 512, 1), (65, 1, 1),
+    (129, 3000, 1), (513, 700, 1), (2, 9000, 1), (70, 1500, 3), (70, 1500, 40)])
+def test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, scale, mode):
+    b, st, q, sinks, prefix, new = _case(count, prefix_len, seed=7 * count + prefix_len)
+    keys = b.token_to_kv_pool.get_key_buffer(1)
+    slots = torch.cat((prefix, new)).long()
+    # Keys grow along the list, so later tiles hold larger logits.
+    ramp = torch.linspace(0.1, scale, slots.numel(), device="cuda")[:, None, None]
+    keys[slots] = (keys[slots].float() * ramp).to(keys.dtype)
+    st.scores.zero_()
+    ge._prefill_scores(st, 0, mode, layer(1), q, keys, sinks, prefix, new)
+    want = _exact_scores(mode, q, keys, sinks, slots, prefix_len)
+    # 32-bit logits: an absolute error of |x| * 2^-22 (64 products) is a relative error of p.
+    largest = 1.5 * 8 * scale * 0.125 * 8 * 8
+    torch.testing.assert_close(st.scores[0][:, slots].double(), want, rtol=1e-5 + largest * 2 ** -22, atol=1e-7)
+
+
 def test_after_extend_scores_chunks_of_two_requests():
     """The hook path: CSR prefix per request, zeroed new slots, sum and max rows in one batch."""
     g = torch.Generator().manual_seed(21)
