@@ -75,6 +75,14 @@ GSE_DEVICE float in_vgpr(float x) {
   return x;
 }
 
+// fmaxf as one instruction: the compiler quiets operands it cannot trace to an arithmetic
+// instruction (a lane swap's results) with a v_max each, which this instruction does itself.
+GSE_DEVICE float vmax(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 GSE_DEVICE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // The wave's loaded registers are in use here: the compiler waits for exactly these loads.

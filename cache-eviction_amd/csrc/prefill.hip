@@ -2,21 +2,16 @@
 // sink in the normaliser, reduced per KV head over its query heads (sum or
 // max) and over the chunk's queries, added to each key's slot score.
 //
-// A workgroup owns one KV head and 64 queries (4 waves x 16). Its MFMA rows
-// are (query, head) pairs: row-block rb of a wave holds queries 2*rb and
-// 2*rb + 1 with the KV head's 8 query heads each, so no row is padding:
-//   S = Q . K^T   [16 rows x 16 keys] per row-block and key-block (16x16x32 bf16)
-// Pass 1 streams the visible keys once to get each row's log-sum-exp (with the
-// sink); pass 2 streams them again, turns logits into probabilities with that
-// normaliser and accumulates column sums (with a score delay d, only of the keys
-// at least d entries before each query: the causal bound of pass 2 moves back by d).
+// Pass 1 (prefill_norm_kernel, prefill_merge_kernel) streams the visible keys past each query
+// block once to get every (query, head) row's log-sum-exp, with the sink; pass 2
+// (prefill_score_kernel) streams the queries past each key block, turns logits into probabilities
+// with that normaliser and accumulates each key's sum (with a score delay d, only over the queries
+// at least d entries after it). MFMA rows or columns are (query, head) pairs, the KV head's 8 query
+// heads each, so none is padding.
 //
-// Work per (query head, key) is one exp2 per pass, which bounds the kernel (v_exp_f32 runs
-// at half the rate of an FMA): pass 1 keeps a lazily rescaled running maximum per row (one
-// FMA + exp2 + add per logit), pass 2 one FMA + exp2 + add. K tiles of 64 keys go through
-// LDS, double-buffered, one global load per workgroup per tile; column sums accumulate
-// in-lane over the wave's 16 queries, then in an LDS ring of 16 tiles that is added to the
-// scores once per ring. Query blocks are dispatched heaviest (longest causal range) first.
+// Work per (query head, key) is one exp2 per pass, which bounds the kernels: v_exp_f32 takes 8.6
+// cycles per wave instruction, FMA and add 2 to 4, and the card's power limit lowers the clock
+// (1.9 GHz) over a launch of milliseconds.
 #include <algorithm>
 #include <type_traits>
 
@@ -29,8 +24,6 @@ namespace pf {
 constexpr int D = 64;
 constexpr int GROUP = 8;
 constexpr int QB = 64;          // queries per workgroup
-constexpr int RB2 = 8;          // pass 2: row-blocks (2 queries each) per wave
-constexpr int WAVES = QB / (2 * RB2);
 constexpr int KT = 64;          // keys per tile (4 key-blocks of 16)
 constexpr int KROW = D + 8;     // padded bf16 row of a staged key
 constexpr int RING = 16;        // tiles of column sums held before they are added to the scores
@@ -64,6 +57,7 @@ struct PrefillArgs {
   // q_heads + head] = (reference, sum of 2^(x - reference)) of the row over that range.
   float2* part;
   int splits, tiles;
+  int qblock;  // pass 2: queries per workgroup
 };
 
 // ---------------------------------------------------------------------------
@@ -83,11 +77,13 @@ constexpr int QW = 8;                // queries per wave: two column blocks of 4
 constexpr int WAVES = 8;
 constexpr int THREADS = 64 * WAVES;
 static_assert(QW * WAVES == pf::QB, "a workgroup's queries");
-// Work items of a launch: enough for several rounds of the 512 workgroups the chip holds (2 per
-// CU), at least MIN_TILES tiles each, which keeps an item's start (query and first key loads)
-// below a third of its time.
-constexpr int ITEMS = 3072;
-constexpr int MIN_TILES = 4;
+// Work items of a launch: about three rounds of the 512 workgroups the chip holds (2 per CU), at
+// least MIN_TILES tiles each (an item's start, its query and first key loads, costs some 3 us).
+// Both passes, 2048 tokens without a prefix: 97 us; twice the items or half the tiles 117, a third
+// fewer items 94. 190 tokens after 7000: 59 against 64. Past 2048 tokens after 28,672 the split no
+// longer matters (1231 us, 1241 with twice the items, 1271 with a third fewer).
+constexpr int ITEMS = 1536;
+constexpr int MIN_TILES = 8;
 }  // namespace p1
 
 // Key ranges of a query block that sees ntiles tiles (equal ones, of at most `tiles` tiles).
@@ -356,243 +352,231 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   a.norm2[t] = m + __log2f(l);
 }
 
-// Row-block rb's logits of a 64-key tile: D = Q . K^T for four 16-key blocks (MFMA rows are
-// (query, head) pairs, a lane's four values of block kb are rows 4*(grp%2)..+3 of query
-// 2*rb + grp/2 against key 16*kb + col). MASKED: key (t0 + 16*kb + col) is dead for this
-// lane's query when rel + 16*kb > 2*rb + grp/2, with rel = t0 + col - (position of the wave's
-// first query); its logit becomes -inf.
+// ---------------------------------------------------------------------------
+// Pass 2: column sums
+// ---------------------------------------------------------------------------
+// A workgroup owns one KV head, 256 keys (4 waves x 64, their K fragments in registers) and
+// a.qblock queries, which stream through LDS 8 at a time: a key's sum stays in a register over the
+// whole walk and reaches the score table with one atomic per (key, query block), and no key index
+// is read inside it. Sum mode forms S^T = K . Q^T (a lane holds 16 keys of one row: one normaliser,
+// a sum per key), max mode S = Q . K^T (a lane holds 4 heads of 4 queries for one key: the maximum
+// over the heads is in the lane and its other half). 3 (sum: 32 sums and 32 K registers) and 4 (max)
+// waves per SIMD. Against query blocks of 64 walking the keys (column sums through LDS rings, two
+// waves per SIMD): sums 77 -> 52 us for the first 2048 tokens of a prompt, 3.4 -> 2.5 ms for 8192
+// tokens after 28,672; maxima 1120 -> 480 us for 1896 after 30,720.
+namespace p2 {
+constexpr int KW = 64;  // keys per wave: two 32-key blocks
+constexpr int WAVES = 4;
+constexpr int KB = KW * WAVES;
+constexpr int THREADS = 64 * WAVES;
+constexpr int QT = 8;  // queries per tile (64 rows)
+// Work items of a launch (as p1::ITEMS), the fewest queries per item, and the most: a sum takes at
+// most MAX_QUERIES / 4 additions in one register, so its rounding error stays near that of a sum
+// over 64-query blocks.
+constexpr int ITEMS = 2048;
+constexpr int MIN_QUERIES = 64;
+constexpr int MAX_QUERIES = 512;
+}  // namespace p2
+
+// Column block cb (4 queries) of a staged query tile against the wave's keys, sums: cs[kb][i] +=
+// the probability of key 32*kb + 8*(i/4) + 4*(lane/32) + i%4 in row lane%32. MASKED: dead past
+// bound + 4*cb (from the key 4*(lane/32)).
 template <bool MASKED>
-GSE_DEVICE void prefill_mask(f32x4_t (&d)[4], int rb, int64_t rel, int grp) {
-  if (MASKED) {
-    const int64_t qrel = 2 * rb + (grp >> 1);
+GSE_DEVICE void column_sum_tile(const uint16_t* qt, const float* nt, const bf16x8_t (&kf)[2][4],
+                                f32x16_t (&cs)[2], float scale2, int bound, int lane) {
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb)
-      if (rel + 16 * kb > qrel)
+  for (int cb = 0; cb < 2; ++cb) {
+    bf16x8_t qf[4];
+    k_fragments(qt, cb, lane, qf);
+    const float nn = nt[32 * cb + (lane & 31)];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) d[kb][r] = -INFINITY;
+    for (int kb = 0; kb < 2; ++kb) {
+      f32x16_t d = dot64(kf[kb], qf);
+      if (MASKED) mask_keys(d, 32 * kb, bound + 4 * cb);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) cs[kb][i] += fast_exp2(fmaf(d[i], scale2, nn));
+      // The sums are formed here: otherwise the exponentials of all four blocks sink behind the
+      // tile's last MFMA, with their 64 logits.
+#pragma unroll
+      for (int i = 0; i < 16; ++i) cs[kb][i] = in_vgpr(cs[kb][i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
 }
 
-// One 64-key tile of a wave: row-block rb's MFMAs for four 16-key blocks, then per logit one
-// FMA + exp2 (+ the add). Row-block rb + 1's MFMAs are issued before rb's exponentials.
-template <bool MAX_MODE, bool MASKED, int RB>
-GSE_DEVICE void prefill_tile(const bf16x8_t (&qa)[RB][2], const bf16x8_t (&kb0)[4], const bf16x8_t (&kb1)[4],
-                             const float (&ref)[RB][4], float (&cs)[4], float scale2,
-                             int64_t rel, int grp) {
-  using namespace pf;
-  f32x4_t dn[4];
+// The same, maxima over the KV head's query heads: cs[kb] += the sum over this lane half's two
+// queries of each column block (0 and 2, or 1 and 3) of key 32*kb + lane%32's largest probability.
+// The largest probability is 2^(largest exponent): one exponential per (query, key). MASKED: key
+// 32*kb is dead past bound + query.
+template <bool MASKED>
+GSE_DEVICE void column_max_tile(const uint16_t* qt, const float* nt, const bf16x8_t (&kf)[2][4], float (&cs)[2],
+                                float scale2, int bound, int lane) {
 #pragma unroll
-  for (int kb = 0; kb < 4; ++kb) {
-    dn[kb] = mfma16x16x32(qa[0][0], kb0[kb], f32x4_t{0.f, 0.f, 0.f, 0.f});
-    dn[kb] = mfma16x16x32(qa[0][1], kb1[kb], dn[kb]);
+  for (int cb = 0; cb < 2; ++cb) {
+    bf16x8_t qf[4];
+    k_fragments(qt, cb, lane, qf);
+    f32x4_t nn[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      nn[b] = *reinterpret_cast<const f32x4_t*>(nt + 32 * cb + 8 * b + 4 * (lane >> 5));
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const f32x16_t d = dot64(qf, kf[kb]);
+      float y[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        float x[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[r] = fmaf(d[4 * b + r], scale2, nn[b][r]);
+        y[b] = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+        if (MASKED && 32 * kb > bound + 4 * cb + b) y[b] = -INFINITY;
+      }
+#pragma unroll
+      for (int b = 0; b < 4; b += 2) {  // lower lanes take query b, upper lanes query b + 1
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[b]), __float_as_uint(y[b + 1]), false, false);
+        cs[kb] += fast_exp2(vmax(__uint_as_float(r[0]), __uint_as_float(r[1])));
+      }
+      cs[kb] = in_vgpr(cs[kb]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
+}
+
+// One value per lane out of N: lane bits select it, log2(N) exchanges (lane l ends with the sum over
+// its exchange group of value l % N; N is 2^k, the group the N lanes around it).
+template <int N>
+GSE_DEVICE float scatter_sum(float (&v)[N], int lane) {
+  if constexpr (N == 1) {
+    return v[0];
+  } else {
+    float w[N / 2];
+    const bool upper = lane & (N / 2);
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    f32x4_t d[4];
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) d[kb] = dn[kb];
-    if (rb + 1 < RB) {
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        dn[kb] = mfma16x16x32(qa[rb + 1][0], kb0[kb], f32x4_t{0.f, 0.f, 0.f, 0.f});
-        dn[kb] = mfma16x16x32(qa[rb + 1][1], kb1[kb], dn[kb]);
-      }
+    for (int i = 0; i < N / 2; ++i) {
+      const float keep = upper ? v[i + N / 2] : v[i], send = upper ? v[i] : v[i + N / 2];
+      w[i] = keep + __shfl_xor(send, N / 2, kWave);
     }
-    prefill_mask<MASKED>(d, rb, rel, grp);
-#pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      if (MAX_MODE) {  // the largest probability is 2^(largest exponent): one exponential
-        const float y = fmaxf(fmaxf(fmaf(d[kb][0], scale2, -ref[rb][0]), fmaf(d[kb][1], scale2, -ref[rb][1])),
-                              fmaxf(fmaf(d[kb][2], scale2, -ref[rb][2]), fmaf(d[kb][3], scale2, -ref[rb][3])));
-        cs[kb] += fast_exp2(xor16_max(y));
-      } else {
-        const float p0 = fast_exp2(fmaf(d[kb][0], scale2, -ref[rb][0]));
-        const float p1 = fast_exp2(fmaf(d[kb][1], scale2, -ref[rb][1]));
-        const float p2 = fast_exp2(fmaf(d[kb][2], scale2, -ref[rb][2]));
-        const float p3 = fast_exp2(fmaf(d[kb][3], scale2, -ref[rb][3]));
-        cs[kb] += (p0 + p1) + (p2 + p3);
-      }
-    }
-    // Alternate the next row-block's 8 MFMAs with this one's vector work (1 MFMA, then 6 vector
-    // instructions): a SIMD overlaps an MFMA only with the independent vector instructions its
-    // own wave issues behind it (the waves' MFMA and vector work do not overlap each other).
-    if (rb + 1 < RB) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // six vector ALU instructions
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    return scatter_sum(w, lane);
   }
 }
 
 template <bool MAX_MODE>
-__global__ __launch_bounds__(64 * pf::WAVES) void prefill_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(p2::THREADS, MAX_MODE ? 4 : 3) void prefill_score_kernel(PrefillArgs a) {
   using namespace pf;
-  constexpr int RB = RB2;
-  __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
-  __shared__ float ring[RING * KT];
-  // Slots of the keys of two rings of tiles (the one being summed and the next), for the ring's
-  // score atomics.
-  __shared__ int32_t ring_slot[2 * RING * KT];
+  using namespace p2;
+  __shared__ __attribute__((aligned(16))) uint16_t qtile[2][QT * GROUP * KROW];
+  __shared__ __attribute__((aligned(16))) float ntile[2][QT * GROUP];  // negated normalisers
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col = lane & 15, grp = lane >> 4;
-  // Heaviest query blocks first: linear block i -> KV head i % kv_heads, query block from the end.
-  const int64_t nqb = (a.count + QB - 1) / QB;
+  // Block i: KV head i % kv_heads, then the query block, then the key block (the first keys are
+  // credited by most queries; the last by few).
+  const int count = int(a.count);
+  const int nqb = (count + a.qblock - 1) / a.qblock;
   const int g = blockIdx.x % a.kv_heads;
-  const int64_t qb0 = (nqb - 1 - int64_t(blockIdx.x / a.kv_heads)) * QB;
-  const int64_t i0 = qb0 + 2 * RB * wave;  // this wave's first query
-  const int64_t last_q = (qb0 + QB < a.count ? qb0 + QB : a.count) - 1;
-  // Pass 2 credits keys up to `shift` entries before each query's causal bound.
-  const int64_t shift = a.delay;
-  const int64_t kend = a.prefix_len + last_q + 1 - shift;  // keys any query of the workgroup sees (scores)
-  const bool wave_live = i0 < a.count;
-  const int64_t wave_kend = a.prefix_len + (i0 + 2 * RB - 1 < a.count ? i0 + 2 * RB - 1 : a.count - 1) + 1 - shift;
+  const int item = blockIdx.x / a.kv_heads;
+  const int k0 = item / nqb * KB, kw = k0 + KW * wave;
+  const int qb0 = item % nqb * a.qblock;
+  const int q1 = min(qb0 + a.qblock, count);
+  const int bound0 = int(a.prefix_len) - a.delay;  // query i credits keys up to bound0 + i
+  const int q0 = max(qb0, max(k0 - bound0, 0) / QT * QT);
+  if (q0 >= q1) return;
+  const int kend = min(int(a.total), bound0 + q1);  // keys the item credits
 
-  // A fragments: row col of row-block rb is query i0 + 2*rb + col/8, head g*8 + col%8;
-  // lane supplies dims [16*grp, 16*grp + 16) as two 8-dim MFMA halves.
-  bf16x8_t qa[RB][2];
+  // The wave's keys: lane holds dims [16*ks + 8*(lane/32), +8) of keys kw + 32*kb + lane%32 (past
+  // the list: its last key, never credited).
+  bf16x8_t kf[2][4];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int64_t qi = i0 + 2 * rb + col / 8;
-    qa[rb][0] = bf16x8_t{};
-    qa[rb][1] = bf16x8_t{};
-    if (qi < a.count) {
-      const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * GROUP + col % 8) * a.q_sh + 16 * grp;
-      qa[rb][0] = as_bf16x8(*reinterpret_cast<const uint4*>(qp));
-      qa[rb][1] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 8));
-    }
+  for (int kb = 0; kb < 2; ++kb) {
+    const int key = min(kw + 32 * kb + (lane & 31), int(a.total) - 1);
+    const int64_t s = load_index_dyn(a.slots, a.slots_dtype, key);
+    const auto kp = as_global(a.k) + s * a.kv_ss + int64_t(g) * a.kv_sh + 8 * (lane >> 5);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) kf[kb][ks] = as_bf16x8(gload16(kp + 16 * ks));
   }
-  // This lane's output rows in row-block rb: query i0 + 2*rb + grp/2, heads hq0 + r.
-  const int hq0 = g * GROUP + 4 * (grp & 1);
-  // The rows' normalisers (+inf for rows past the chunk: their terms are 0).
-  float ref[RB][4];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int64_t qi = i0 + 2 * rb + (grp >> 1);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      ref[rb][r] = qi < a.count ? a.norm2[qi * a.q_heads + hq0 + r] : INFINITY;
-    }
-  }
-  for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) ring[t] = 0.f;
-
-  // Cooperative tile load: thread t < 256 stages key t/4, dims [16*(t%4), +16). Tile t's K rows
-  // are loaded into registers during tile t - 2 and stored to LDS at the end of tile t - 1, and
-  // its slot indices are read two tiles before that: a load's latency is hidden behind two tiles
-  // of compute, and no K load waits on an index load. Two register sets of each alternate by
-  // tile parity (the loop is unrolled by two), so nothing is copied between them: a copy would
-  // wait for the loads in flight into its source. Keys past kend read slot 0's row (any valid
-  // row) and are never used.
-  constexpr bool loader = true;
-  const int lk = (threadIdx.x >> 2) & 63, lp = threadIdx.x & 3;
-  auto slot_at = [&](int64_t t0) -> int32_t {
-    const int64_t key = t0 + lk;
-    return key < kend ? int32_t(load_index_dyn(a.slots, a.slots_dtype, key)) : 0;
+  // Query tile load: thread t stages 16 bytes of rows t/8 (query q + row/8, head row%8) and t/8 + 32
+  // (four queries on); the next tile is in flight while one computes. Rows past the chunk are zero
+  // with normaliser +inf: probability 0.
+  static_assert(THREADS * 2 == QT * GROUP * 8, "two pieces per thread");
+  const int lr = threadIdx.x >> 3, lp = threadIdx.x & 7;
+  const auto qbase = as_global(a.q) + int64_t(g * GROUP + (lr & 7)) * a.q_sh + 8 * lp;
+  const auto nbase = as_global(a.norm2) + g * GROUP + (threadIdx.x & 7);
+  auto load_q = [&](int q) {
+    const int qi = q + (lr >> 3);
+    return qi < count ? gload16(qbase + int64_t(qi) * a.q_st) : uint4{};
   };
-  auto load_rows = [&](int32_t s, uint4 (&x)[2]) {
-    const auto kp = as_global(a.k) + int64_t(s) * a.kv_ss + int64_t(g) * a.kv_sh + 16 * lp;
-    x[0] = gload16(kp);
-    x[1] = gload16(kp + 8);
+  auto load_n = [&](int q) {
+    const int qi = q + int(threadIdx.x >> 3);
+    return threadIdx.x < QT * GROUP && qi < count ? -nbase[int64_t(qi) * a.q_heads] : -INFINITY;
   };
-  auto store_rows = [&](int ti, const uint4 (&x)[2]) {
-    uint16_t* dst = &ktile[ti & 1][lk * KROW + 16 * lp];
-    *reinterpret_cast<uint4*>(dst) = x[0];
-    *reinterpret_cast<uint4*>(dst + 8) = x[1];
+  auto store_tile = [&](int p, const uint4& x0, const uint4& x1, float n) {
+    *reinterpret_cast<uint4*>(&qtile[p][lr * KROW + 8 * lp]) = x0;
+    *reinterpret_cast<uint4*>(&qtile[p][(lr + 32) * KROW + 8 * lp]) = x1;
+    if (threadIdx.x < QT * GROUP) ntile[p][threadIdx.x] = n;
   };
-  // Pass 2 keeps each staged key's slot for its ring's score atomics: positions of tile t are
-  // (t mod 2*RING) * KT, so the ring being summed and the next one never share them.
-  auto keep_slot = [&](int ti, int32_t s) {
-    if (lp == 0) ring_slot[(ti % (2 * RING)) * KT + lk] = s;
-  };
-  const int ntiles = int((kend + KT - 1) / KT);
-  uint4 xk[2][2] = {};     // xk[p]: K rows of the tile of parity p in flight
-  int32_t sk[2] = {0, 0};  // sk[p]: slot of the next tile of parity p whose rows are not yet loaded
-  if (loader) {
-    const int32_t s0 = slot_at(0), s1 = slot_at(KT);
-    sk[0] = slot_at(2 * KT);
-    sk[1] = slot_at(3 * KT);
-    uint4 y[2];
-    load_rows(s0, y);
-    load_rows(s1, xk[1]);
-    keep_slot(0, s0);
-    keep_slot(1, s1);
-    store_rows(0, y);
-  }
-  // The query fragments and normalisers are in registers before the walk starts: a wait for
-  // them inside the loop would also wait for every load in flight at the top of each tile.
+  store_tile(0, load_q(q0), load_q(q0 + QT / 2), load_n(q0));
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    landed(qa[rb][0]);
-    landed(qa[rb][1]);
+  for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      landed(ref[rb][r]);
-  }
+    for (int ks = 0; ks < 4; ++ks) landed(kf[kb][ks]);
   __syncthreads();
 
-  // One tile of the walk.
-  const int64_t qpos0 = a.prefix_len + i0 - shift;  // the wave's first query's causal bound
-  auto tile_step = [&](int ti, auto parity) {
-    constexpr int P = decltype(parity)::value;  // ti & 1
-    const int64_t t0 = int64_t(ti) * KT;
-    // Tile ti + 2's rows (into the set tile ti's rows left) and tile ti + 4's slots go out.
-    if (loader) {
-      load_rows(sk[P], xk[P]);
-      keep_slot(ti + 2, sk[P]);
-      sk[P] = slot_at(t0 + 4 * KT);
-    }
-    if (wave_live && t0 < wave_kend) {
-      const uint16_t* kt = ktile[ti & 1];
-      bf16x8_t kb0[4], kb1[4];
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const uint16_t* kr = kt + (16 * kb + col) * KROW + 16 * grp;
-        kb0[kb] = as_bf16x8(*reinterpret_cast<const uint4*>(kr));
-        kb1[kb] = as_bf16x8(*reinterpret_cast<const uint4*>(kr + 8));
-      }
-      // Keys past the wave's first query need the causal mask (at most the last two tiles).
-      float cs[4] = {0.f, 0.f, 0.f, 0.f};
-      if (t0 + KT - 1 > qpos0)
-        prefill_tile<MAX_MODE, true, RB>(qa, kb0, kb1, ref, cs, a.scale2, t0 + col - qpos0, grp);
+  f32x16_t sums[2] = {};
+  float maxes[2] = {0.f, 0.f};
+  const float scale2 = in_vgpr(a.scale2);
+  // The wave's bound of query q, relative to the lane's first key.
+  const int rel = bound0 - kw - (MAX_MODE ? lane & 31 : 4 * (lane >> 5));
+  auto tile_step = [&](int q, int p, auto whole) {
+    constexpr bool WHOLE = decltype(whole)::value;
+    const uint4 x0 = load_q(q + QT), x1 = load_q(q + QT + QT / 2);
+    const float n = load_n(q + QT);
+    // The lane's bound of the first query (sum mode: of its own row's).
+    const int bound = rel + q + (MAX_MODE ? 0 : (lane & 31) >> 3);
+    auto compute = [&](auto masked) {
+      constexpr bool MASKED = decltype(masked)::value;
+      if constexpr (MAX_MODE)
+        column_max_tile<MASKED>(qtile[p], ntile[p], kf, maxes, scale2, bound, lane);
       else
-        prefill_tile<MAX_MODE, false, RB>(qa, kb0, kb1, ref, cs, a.scale2, 0, grp);
-      // Sum mode: every lane group holds partial sums; max mode: groups 0/1 hold the even
-      // queries' (twice), 2/3 the odd ones'.
-      float* rt = ring + (ti % RING) * KT;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const float tot = MAX_MODE ? xor32_sum(cs[kb]) : xor32_sum(xor16_sum(cs[kb]));
-        if (grp == 0) atomicAdd(&rt[16 * kb + col], tot);
-      }
+        column_sum_tile<MASKED>(qtile[p], ntile[p], kf, sums, scale2, bound, lane);
+    };
+    if constexpr (WHOLE) {
+      compute(std::false_type{});
+    } else if (kw + KW - 1 <= bound0 + q) {
+      compute(std::false_type{});
+    } else if (kw <= bound0 + q + QT - 1) {
+      compute(std::true_type{});
     }
-    if (loader && ti + 1 < ntiles) store_rows(ti + 1, xk[1 - P]);
+    if (q + QT < q1) store_tile(p ^ 1, x0, x1, n);
     __syncthreads();
-    if ((ti + 1) % RING == 0 || ti + 1 == ntiles) {
-      // Add the ring's tiles to the scores, one atomic per key per workgroup (the keys' slots
-      // were kept in LDS when their rows were loaded).
-      const int r0 = ((ti - ti % RING) % (2 * RING)) * KT;
-      const int64_t base = int64_t(ti - ti % RING) * KT;
-#pragma unroll
-      for (int u = 0; u < RING * KT / (64 * WAVES); ++u) {
-        const int t = threadIdx.x + u * 64 * WAVES;
-        if (base + t < kend)
-          unsafeAtomicAdd(&a.scores[int64_t(g) * a.ssg + int64_t(ring_slot[r0 + t]) * a.sss], ring[t]);
-        ring[t] = 0.f;
-      }
-      __syncthreads();
-    }
   };
-  using P0 = std::integral_constant<int, 0>;
-  using P1 = std::integral_constant<int, 1>;
-  int ti = 0;
+  // Queries that credit every key of the workgroup run in a loop of their own.
+  const int qw = min(q1, max(q0, (max(k0 + KB - 1 - bound0, 0) + QT - 1) / QT * QT));
+  int q = q0, p = 0;
 #pragma unroll 1
-  for (; ti < ntiles; ti += 2) {
-    tile_step(ti, P0{});
-    if (ti + 1 < ntiles) tile_step(ti + 1, P1{});
+  for (; q < qw; q += QT, p ^= 1) tile_step(q, p, std::false_type{});
+#pragma unroll 1
+  for (; q < q1; q += QT, p ^= 1) tile_step(q, p, std::true_type{});
+
+  // One lane per key, one atomic per lane.
+  float total;
+  int key;
+  if constexpr (MAX_MODE) {
+    const float t0 = xor32_sum(maxes[0]), t1 = xor32_sum(maxes[1]);
+    total = lane < 32 ? t0 : t1;
+    key = kw + lane;
+  } else {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {  // lane bit 4 selects the key block
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(sums[0][i]), __float_as_uint(sums[1][i]), false,
+                                                      false);
+      v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    total = scatter_sum(v, lane);  // lane % 16 selects the register
+    const int i = lane & 15;
+    key = kw + 32 * ((lane >> 4) & 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
   }
+  if (key < kend)
+    unsafeAtomicAdd(&a.scores[int64_t(g) * a.ssg + load_index_dyn(a.slots, a.slots_dtype, key) * a.sss], total);
 }
 
 // ---------------------------------------------------------------------------
@@ -1097,9 +1081,6 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
                    prefix_len, sinks, sinks_dtype, kind, scores, scores_stride_g, scores_stride_s, q_heads, kv_heads,
                    sm_scale * kLog2e, static_cast<float*>(workspace), delay, block_shift};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int64_t blocks = (count + pf::QB - 1) / pf::QB * kv_heads;
-  if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
-  const dim3 grid{static_cast<uint32_t>(blocks)};
   if (kind == GSE_SCORE_KIND_BLOCK_STEP && kv_heads > pb::WAVES)
     return gse_fail(GSE_ESHAPE, "prefill: block counters need kv_heads <= 8");
   if (int rc = launch_norms(a, workspace, s)) return rc;
@@ -1111,11 +1092,16 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
       hipLaunchKernelGGL(prefill_block_kernel<int32_t>, bgrid, dim3(pb::THREADS), 0, s, a);
     return gse_launch_check("prefill block counters");
   }
-  if (kind == 2) {
-    hipLaunchKernelGGL((prefill_kernel<true>), grid, dim3(64 * pf::WAVES), 0, s, a);
-  } else {
-    hipLaunchKernelGGL((prefill_kernel<false>), grid, dim3(64 * pf::WAVES), 0, s, a);
-  }
+  const int64_t nkb = (total + p2::KB - 1) / p2::KB;
+  const int64_t want = std::max<int64_t>(1, p2::ITEMS / (nkb * kv_heads));
+  const int64_t nq = std::min(want, (count + p2::MIN_QUERIES - 1) / p2::MIN_QUERIES);
+  a.qblock = int(std::min<int64_t>(((count + nq - 1) / nq + p2::QT - 1) / p2::QT * p2::QT, p2::MAX_QUERIES));
+  const int64_t items = nkb * ((count + a.qblock - 1) / a.qblock) * kv_heads;
+  if (items >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
+  if (kind == 2)
+    hipLaunchKernelGGL(prefill_score_kernel<true>, dim3(uint32_t(items)), dim3(p2::THREADS), 0, s, a);
+  else
+    hipLaunchKernelGGL(prefill_score_kernel<false>, dim3(uint32_t(items)), dim3(p2::THREADS), 0, s, a);
   return gse_launch_check("prefill pass 2");
 }
 
