@@ -9,7 +9,6 @@
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
 // Wavefront size on CDNA is 64.
 constexpr int kWave = 64;
@@ -60,17 +59,8 @@ GSE_DEVICE f32x4_t mfma16x16x32(bf16x8_t a, bf16x8_t b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// 32x32x16 bf16 MFMA, fp32 accumulate. Lane l supplies A[l%32][8*(l/32)+e] and
-// B[8*(l/32)+e][l%32] for e = 0..7, and holds D[8*(i/4)+4*(l/32)+i%4][l%32] for i = 0..15. Half the
-// issue slots of the 16x16x32 form per product, at the same rate.
-GSE_DEVICE f32x16_t mfma32x32x16(bf16x8_t a, bf16x8_t b, f32x16_t c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// A uniform value in a vector register: a vector instruction with a scalar operand issues in 4
-// cycles, FMA, multiply and add on vector registers alone in 2 (measured with 4 waves per SIMD:
-// 4.6 and 2.6 cycles per instruction, v_exp_f32 8.6).
-GSE_DEVICE float in_vgpr(float x) {
+// x, formed here: the compiler cannot move its computation past this point.
+GSE_DEVICE float formed(float x) {
   asm volatile("" : "+v"(x));
   return x;
 }

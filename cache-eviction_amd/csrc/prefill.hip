@@ -7,7 +7,7 @@
 // (prefill_score_kernel) streams the queries past each key block, turns logits into probabilities
 // with that normaliser and accumulates each key's sum (with a score delay d, only over the queries
 // at least d entries after it). MFMA rows or columns are (query, head) pairs, the KV head's 8 query
-// heads each, so none is padding.
+// heads each, so none is padding: a 16-wide block holds two queries.
 //
 // Work per (query head, key) is one exp2 per pass, which bounds the kernels: v_exp_f32 takes 8.6
 // cycles per wave instruction, FMA and add 2 to 4, and the card's power limit lowers the clock
@@ -63,15 +63,17 @@ struct PrefillArgs {
 // ---------------------------------------------------------------------------
 // Pass 1: row normalisers
 // ---------------------------------------------------------------------------
-// S^T = K . Q^T in 32x32x16 MFMAs: a lane holds 16 keys of one (query, head) row, so a row needs
-// one reference and one sum per lane, and its terms add up in the lane. A workgroup (8 waves x 8
-// queries) takes one KV head, 64 queries and a range of at most `tiles` 64-key tiles of what
-// they see; prefill_merge_kernel joins the ranges' (reference, sum) pairs and the sink. Per logit the
-// walk issues one FMA, one exponential and one add, all on vector registers, 4 waves per SIMD
-// (128 VGPRs). Bound by vector issue: 329 cycles per 1024 logits and SIMD over a long walk where the
-// instructions alone take 283, and by the card's power there (1.9 GHz). Against 16x16x32 MFMAs with
-// 2 waves per SIMD and whole causal ranges: 87 -> 43 us for the first 2048 tokens of a prompt, 816
-// -> 665 us for 1896 tokens after 30,720, 3.36 -> 2.75 ms for 8192 after 28,672.
+// S^T = K . Q^T in 16x16x32 MFMAs: a lane holds 4 keys per key block of one (query, head) row, so a
+// row needs one reference and one sum per lane, and its terms add up in the lane. A workgroup (8
+// waves x 8 queries) takes one KV head, 64 queries and a range of at most `tiles` 64-key tiles of
+// what they see; prefill_merge_kernel joins the ranges' (reference, sum) pairs and the sink.
+// Bound by vector issue (one FMA, one exponential and one add per logit: 305 cycles per 1024
+// logits and SIMD with their MFMAs) and, over a launch of milliseconds, by the card's power: that
+// mix alone runs at 2.2 GHz, 139 ns per 1024 logits; 32x32x16 MFMAs take fewer issue slots but
+// more power (156 ns), and the FMA with a vector instead of a scalar scale 147 ns. Against rows
+// spread over 16 lanes (a running maximum per row and lane) with 2 waves per SIMD and whole causal
+// ranges: 87 -> 42 us for the first 2048 tokens of a prompt, 816 -> 640 us for 1896 tokens after
+// 30,720, 3.36 -> 2.75 ms for 8192 after 28,672.
 namespace p1 {
 constexpr int QW = 8;                // queries per wave: two column blocks of 4 queries x 8 heads
 constexpr int WAVES = 8;
@@ -89,110 +91,108 @@ constexpr int MIN_TILES = 8;
 // Key ranges of a query block that sees ntiles tiles (equal ones, of at most `tiles` tiles).
 GSE_DEVICE int key_ranges(int ntiles, int tiles) { return (ntiles + tiles - 1) / tiles; }
 
-GSE_DEVICE float sum16(const f32x16_t& p) {
-  return (((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]))) +
-         (((p[8] + p[9]) + (p[10] + p[11])) + ((p[12] + p[13]) + (p[14] + p[15])));
+// Row block rb's fragments of a staged tile of 16-row blocks: lane (col, grp) holds dims [8*grp, +8)
+// and [32 + 8*grp, +8) of row 16*rb + col.
+GSE_DEVICE void fragments(const uint16_t* tile, int rb, int lane, bf16x8_t (&f)[2]) {
+  const uint16_t* r = tile + (16 * rb + (lane & 15)) * pf::KROW + 8 * (lane >> 4);
+  f[0] = as_bf16x8(*reinterpret_cast<const uint4*>(r));
+  f[1] = as_bf16x8(*reinterpret_cast<const uint4*>(r + 32));
 }
 
-// Key block kb's fragments of a staged K tile (lane: key 32*kb + lane%32, dims 16*ks + 8*(lane/32)).
-GSE_DEVICE void k_fragments(const uint16_t* kt, int kb, int lane, bf16x8_t (&ka)[4]) {
-  const uint16_t* kr = kt + (32 * kb + (lane & 31)) * pf::KROW + 8 * (lane >> 5);
+GSE_DEVICE f32x4_t dot64(const bf16x8_t (&a)[2], const bf16x8_t (&b)[2]) {
+  return mfma16x16x32(a[1], b[1], mfma16x16x32(a[0], b[0], f32x4_t{0.f, 0.f, 0.f, 0.f}));
+}
+
+// Logits of keys past a lane's causal bound become -inf: register r of a block holds key first + r,
+// dead when past `bound` (both relative to the same origin).
+GSE_DEVICE void mask_keys(f32x4_t& d, int first, int bound) {
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) ka[ks] = as_bf16x8(*reinterpret_cast<const uint4*>(kr + 16 * ks));
+  for (int r = 0; r < 4; ++r)
+    if (first + r > bound) d[r] = -INFINITY;
 }
 
-GSE_DEVICE f32x16_t dot64(const bf16x8_t (&a)[4], const bf16x8_t (&b)[4]) {
-  f32x16_t d = {};
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) d = mfma32x32x16(a[ks], b[ks], d);
-  return d;
-}
+GSE_DEVICE float sum4(const f32x4_t& p) { return (p[0] + p[1]) + (p[2] + p[3]); }
 
-// Logits of keys past a lane's causal bound become -inf: register i of a block holds key
-// first + 8*(i/4) + i%4, dead when past `bound` (both relative to the same origin).
-GSE_DEVICE void mask_keys(f32x16_t& d, int first, int bound) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i)
-    if (first + 8 * (i / 4) + i % 4 > bound) d[i] = -INFINITY;
-}
-
-// One tile of a wave: ts[rb] = the lane's sum of 2^(x * scale2 + nref[rb]) over its 32 keys, nref
+// One tile of a wave: ts[rb] = the lane's sum of 2^(x * scale2 + nref[rb]) over its 16 keys, nref
 // the negated reference, a whole number. When a sum passes kMoveSum, its row's reference takes the
 // sum's exponent and both sums are scaled by that power of two (exact); when one passes kRescaleSum
 // (rows whose first keys were all masked, or logits over 40 above them) the references of the
 // wave's rows move to their tile maximum and the tile is formed again.
-// MASKED: key 32*kb + 8*(i/4) + i%4 of the tile is dead past bound + 4*rb.
+// MASKED: key 16*kb + r of the tile is dead past bound + 2*rb.
 template <bool MASKED>
-GSE_DEVICE void row_sum_tile(const uint16_t* kt, const bf16x8_t (&qf)[2][4], float (&nref)[2], float (&sum)[2],
+GSE_DEVICE void row_sum_tile(const uint16_t* kt, const bf16x8_t (&qf)[4][2], float (&nref)[4], float (&sum)[4],
                              float scale2, int bound, int lane) {
   using namespace pf;
-  float ts[2];
+  float ts[4];
   {
-    bf16x8_t ka[4];
-    k_fragments(kt, 0, lane, ka);
-    f32x16_t dn = dot64(ka, qf[0]);
+    // Units of two key blocks against one column block (2 queries); the next unit's MFMAs are
+    // issued ahead of this one's vector work.
+    bf16x8_t ka[2][2];
+    f32x4_t dn[2];
+    fragments(kt, 0, lane, ka[0]);
+    fragments(kt, 1, lane, ka[1]);
+    dn[0] = dot64(ka[0], qf[0]);
+    dn[1] = dot64(ka[1], qf[0]);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {  // (key block, column block) pairs, the next one's MFMAs issued ahead
-      const int kb = u >> 1, rb = u & 1;
-      f32x16_t d = dn;
-      if (u == 1) k_fragments(kt, 1, lane, ka);
-      if (u < 3) dn = dot64(ka, qf[(u + 1) & 1]);
-      if (MASKED) mask_keys(d, 32 * kb, bound + 4 * rb);
+    for (int u = 0; u < 8; ++u) {
+      const int kp = u >> 2, rb = u & 3;
+      f32x4_t d[2] = {dn[0], dn[1]};
+      if (u == 3) {
+        fragments(kt, 2, lane, ka[0]);
+        fragments(kt, 3, lane, ka[1]);
+      }
+      if (u < 7) {
+        dn[0] = dot64(ka[0], qf[(u + 1) & 3]);
+        dn[1] = dot64(ka[1], qf[(u + 1) & 3]);
+      }
 #pragma unroll
-      for (int i = 0; i < 16; ++i) d[i] = fast_exp2(fmaf(d[i], scale2, nref[rb]));
-      ts[rb] = kb == 0 ? sum16(d) : ts[rb] + sum16(d);
+      for (int h = 0; h < 2; ++h) {
+        if (MASKED) mask_keys(d[h], 32 * kp + 16 * h, bound + 2 * rb);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[h][r] = fast_exp2(fmaf(d[h][r], scale2, nref[rb]));
+      }
+      const float t = sum4(d[0]) + sum4(d[1]);
+      ts[rb] = kp == 0 ? t : ts[rb] + t;
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  const float tsmax = fmaxf(ts[0], ts[1]);
+  const float tsmax = fmaxf(fmaxf(ts[0], ts[1]), fmaxf(ts[2], ts[3]));
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(tsmax > kMoveSum) == 0, 1)) {
-    sum[0] += ts[0];
-    sum[1] += ts[1];
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) sum[rb] += ts[rb];
     return;
   }
   if (__builtin_amdgcn_ballot_w64(tsmax > kRescaleSum)) {
-#pragma unroll 1
-    for (int rb = 0; rb < 2; ++rb) {
-      bf16x8_t q[4];
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) q[ks] = rb == 0 ? qf[0][ks] : qf[1][ks];
-      const float old = rb == 0 ? nref[0] : nref[1];
+    for (int rb = 0; rb < 4; ++rb) {
       float tmax = -INFINITY;
 #pragma unroll 1
-      for (int kb = 0; kb < 2; ++kb) {
-        bf16x8_t ka[4];
-        k_fragments(kt, kb, lane, ka);
-        f32x16_t d = dot64(ka, q);
-        if (MASKED) mask_keys(d, 32 * kb, bound + 4 * rb);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, d[i]);
+      for (int kb = 0; kb < 4; ++kb) {
+        bf16x8_t ka[2];
+        fragments(kt, kb, lane, ka);
+        f32x4_t d = dot64(ka, qf[rb]);
+        if (MASKED) mask_keys(d, 16 * kb, bound + 2 * rb);
+        tmax = fmaxf(fmaxf(tmax, fmaxf(d[0], d[1])), fmaxf(d[2], d[3]));
       }
-      const float nr = fminf(old, -rintf(tmax * scale2));
+      const float nr = fminf(nref[rb], -rintf(tmax * scale2));
       float t = 0.f;
 #pragma unroll 1
-      for (int kb = 0; kb < 2; ++kb) {
-        bf16x8_t ka[4];
-        k_fragments(kt, kb, lane, ka);
-        f32x16_t d = dot64(ka, q);
-        if (MASKED) mask_keys(d, 32 * kb, bound + 4 * rb);
+      for (int kb = 0; kb < 4; ++kb) {
+        bf16x8_t ka[2];
+        fragments(kt, kb, lane, ka);
+        f32x4_t d = dot64(ka, qf[rb]);
+        if (MASKED) mask_keys(d, 16 * kb, bound + 2 * rb);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) d[i] = fast_exp2(fmaf(d[i], scale2, nr));
-        t += sum16(d);
+        for (int r = 0; r < 4; ++r) d[r] = fast_exp2(fmaf(d[r], scale2, nr));
+        t += sum4(d);
       }
-      const float keep = fast_exp2(nr - old);
-      if (rb == 0) {
-        sum[0] *= keep;
-        nref[0] = nr;
-        ts[0] = t;
-      } else {
-        sum[1] *= keep;
-        nref[1] = nr;
-        ts[1] = t;
-      }
+      sum[rb] *= fast_exp2(nr - nref[rb]);
+      nref[rb] = nr;
+      ts[rb] = t;
     }
   }
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
+  for (int rb = 0; rb < 4; ++rb) {
     const int e = ts[rb] > kMoveSum && ts[rb] <= kRescaleSum ? __builtin_amdgcn_frexp_expf(ts[rb]) : 0;
     nref[rb] -= float(e);
     sum[rb] = ldexpf(sum[rb] + ts[rb], -e);
@@ -223,19 +223,20 @@ __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArg
   const bool wave_live = i0 < a.count;
   const int wave_kend = int(a.prefix_len) + min(i0 + QW - 1, int(a.count) - 1) + 1;
 
-  // B fragments: column lane%32 of block rb is query i0 + 4*rb + (lane%32)/8, head g*8 + lane%8.
-  bf16x8_t qf[2][4];
+  // B fragments: column col = lane%16 of block rb is query i0 + 2*rb + col/8, head g*8 + col%8.
+  bf16x8_t qf[4][2];
+  float nref[4], sum[4];
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const int64_t qi = i0 + 4 * rb + ((lane & 31) >> 3);
-    const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * GROUP + (lane & 7)) * a.q_sh + 8 * (lane >> 5);
+  for (int rb = 0; rb < 4; ++rb) {
+    const int64_t qi = i0 + 2 * rb + ((lane & 15) >> 3);
+    const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * GROUP + (lane & 7)) * a.q_sh + 8 * (lane >> 4);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      qf[rb][ks] = qi < a.count ? as_bf16x8(*reinterpret_cast<const uint4*>(qp + 16 * ks)) : bf16x8_t{};
+    for (int h = 0; h < 2; ++h)
+      qf[rb][h] = qi < a.count ? as_bf16x8(*reinterpret_cast<const uint4*>(qp + 32 * h)) : bf16x8_t{};
+    nref[rb] = 1e30f;  // finite, so fully masked rows give 2^(-inf) = 0, never NaN
+    sum[rb] = 0.f;
   }
-  float nref[2] = {1e30f, 1e30f};  // finite, so fully masked rows give 2^(-inf) = 0, never NaN
-  float sum[2] = {0.f, 0.f};
-  const float scale2 = in_vgpr(a.scale2);
+  const float scale2 = a.scale2;
 
   // Tile load: thread t stages 16 bytes of key t/8. Tile t's K rows are loaded into registers
   // during tile t - 2 and stored to LDS at the end of tile t - 1, and its slot indices are read
@@ -263,22 +264,28 @@ __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArg
   // The query fragments are in registers before the walk starts: a wait for them inside the
   // loop would also wait for every load in flight at the top of each tile.
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) landed(qf[rb][ks]);
+  for (int rb = 0; rb < 4; ++rb) {
+    landed(qf[rb][0]);
+    landed(qf[rb][1]);
+  }
   __syncthreads();
 
-  const int qpos = int(a.prefix_len) + i0 + ((lane & 31) >> 3) - 4 * (lane >> 5);  // the lane's causal bound
-  {  // Each row's reference: the maximum over the lane's keys of the range's first 32.
-    bf16x8_t ka[4];
-    k_fragments(ktile[0], 0, lane, ka);
+  // The causal bound of the lane's row of block 0, from the lane's first key (4*grp) on.
+  const int qpos = int(a.prefix_len) + i0 + ((lane & 15) >> 3) - 4 * (lane >> 4);
+  {  // Each row's reference: the maximum over the range's first 32 keys.
+    bf16x8_t ka[2][2];
+    fragments(ktile[0], 0, lane, ka[0]);
+    fragments(ktile[0], 1, lane, ka[1]);
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      f32x16_t d = dot64(ka, qf[rb]);
-      mask_keys(d, 0, qpos + 4 * rb - ti0 * KT);
-      float m = d[0];
+    for (int rb = 0; rb < 4; ++rb) {
+      float m = -INFINITY;
 #pragma unroll
-      for (int i = 1; i < 16; ++i) m = fmaxf(m, d[i]);
+      for (int h = 0; h < 2; ++h) {
+        f32x4_t d = dot64(ka[h], qf[rb]);
+        mask_keys(d, 16 * h, qpos + 2 * rb - ti0 * KT);
+        m = fmaxf(m, fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3])));
+      }
+      m = xor32_max(xor16_max(m));
       nref[rb] = fminf(nref[rb], -rintf(m * scale2));
     }
   }
@@ -315,14 +322,13 @@ __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArg
     if (ti + 1 < ti1) tile_step(ti + 1, std::true_type{}, P1{});
   }
 
-  // The row's pair over both lane halves.
+  // The row's pair over the four lane groups.
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const float other = lane_xor32(nref[rb]);
-    const float nr = fminf(nref[rb], other);
-    const float total = xor32_sum(sum[rb] * fast_exp2(nr - nref[rb]));
-    const int64_t qi = i0 + 4 * rb + ((lane & 31) >> 3);
-    if (lane < 32 && qi < a.count)
+  for (int rb = 0; rb < 4; ++rb) {
+    const float nr = -xor32_max(xor16_max(-nref[rb]));
+    const float total = xor32_sum(xor16_sum(sum[rb] * fast_exp2(nr - nref[rb])));
+    const int64_t qi = i0 + 2 * rb + ((lane & 15) >> 3);
+    if (lane < 16 && qi < a.count)
       a.part[(split * a.count + qi) * a.q_heads + g * GROUP + (lane & 7)] = float2{-nr, total};
   }
 }
@@ -359,11 +365,11 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 // a.qblock queries, which stream through LDS 8 at a time: a key's sum stays in a register over the
 // whole walk and reaches the score table with one atomic per (key, query block), and no key index
 // is read inside it. Sum mode forms S^T = K . Q^T (a lane holds 16 keys of one row: one normaliser,
-// a sum per key), max mode S = Q . K^T (a lane holds 4 heads of 4 queries for one key: the maximum
-// over the heads is in the lane and its other half). 3 (sum: 32 sums and 32 K registers) and 4 (max)
-// waves per SIMD. Against query blocks of 64 walking the keys (column sums through LDS rings, two
+// a sum per key), max mode S = Q . K^T (a lane holds 4 heads of a query for one key: the maximum
+// over the heads is in the lane and its neighbouring group). 4 waves per SIMD. Bound as pass 1;
+// max mode takes one exponential per (query, key). Against query blocks of 64 walking the keys (column sums through LDS rings, two
 // waves per SIMD): sums 77 -> 52 us for the first 2048 tokens of a prompt, 3.4 -> 2.5 ms for 8192
-// tokens after 28,672; maxima 1120 -> 480 us for 1896 after 30,720.
+// tokens after 28,672; maxima 1120 -> 450 us for 1896 after 30,720.
 namespace p2 {
 constexpr int KW = 64;  // keys per wave: two 32-key blocks
 constexpr int WAVES = 4;
@@ -378,67 +384,71 @@ constexpr int MIN_QUERIES = 64;
 constexpr int MAX_QUERIES = 512;
 }  // namespace p2
 
-// Column block cb (4 queries) of a staged query tile against the wave's keys, sums: cs[kb][i] +=
-// the probability of key 32*kb + 8*(i/4) + 4*(lane/32) + i%4 in row lane%32. MASKED: dead past
-// bound + 4*cb (from the key 4*(lane/32)).
+// A staged query tile against the wave's keys, sums: cs[kb][r] += the probabilities of key
+// 16*kb + 4*(lane/16) + r in rows lane%16 of the column blocks (2 queries each). MASKED: key
+// 16*kb + r is dead past bound + 2*cb.
 template <bool MASKED>
-GSE_DEVICE void column_sum_tile(const uint16_t* qt, const float* nt, const bf16x8_t (&kf)[2][4],
-                                f32x16_t (&cs)[2], float scale2, int bound, int lane) {
+GSE_DEVICE void column_sum_tile(const uint16_t* qt, const float* nt, const bf16x8_t (&kf)[4][2], f32x4_t (&cs)[4],
+                                float scale2, int bound, int lane) {
 #pragma unroll
-  for (int cb = 0; cb < 2; ++cb) {
-    bf16x8_t qf[4];
-    k_fragments(qt, cb, lane, qf);
-    const float nn = nt[32 * cb + (lane & 31)];
+  for (int c2 = 0; c2 < 4; c2 += 2) {
+    bf16x8_t qf[2][2];
+    float nn[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      f32x16_t d = dot64(kf[kb], qf);
-      if (MASKED) mask_keys(d, 32 * kb, bound + 4 * cb);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) cs[kb][i] += fast_exp2(fmaf(d[i], scale2, nn));
-      // The sums are formed here: otherwise the exponentials of all four blocks sink behind the
-      // tile's last MFMA, with their 64 logits.
-#pragma unroll
-      for (int i = 0; i < 16; ++i) cs[kb][i] = in_vgpr(cs[kb][i]);
-      __builtin_amdgcn_sched_barrier(0);
+    for (int j = 0; j < 2; ++j) {
+      fragments(qt, c2 + j, lane, qf[j]);
+      nn[j] = nt[16 * (c2 + j) + (lane & 15)];
     }
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      f32x4_t d[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) d[j] = dot64(kf[kb], qf[j]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        if (MASKED) mask_keys(d[j], 16 * kb, bound + 2 * (c2 + j));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[j][r] = fast_exp2(fmaf(d[j][r], scale2, nn[j]));
+      }
+      // The sums are formed here: otherwise the exponentials sink behind the tile's last MFMA, with
+      // their logits.
+#pragma unroll
+      for (int r = 0; r < 4; ++r) cs[kb][r] = formed(cs[kb][r] + (d[0][r] + d[1][r]));
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// The same, maxima over the KV head's query heads: cs[kb] += the sum over this lane half's two
-// queries of each column block (0 and 2, or 1 and 3) of key 32*kb + lane%32's largest probability.
-// The largest probability is 2^(largest exponent): one exponential per (query, key). MASKED: key
-// 32*kb is dead past bound + query.
+// The same, maxima over the KV head's query heads: a lane holds heads 4*(grp%2) + r of query grp/2
+// of a row block (2 queries) for key col of a key block; the other four heads are in the
+// neighbouring lane group. One swap joins them for two key blocks: cs[kp] += the largest probability
+// of key 32*kp + 16*(grp%2) + col over the tile's queries of parity grp/2. The largest probability
+// is 2^(largest exponent): one exponential per (query, key). MASKED: key 16*kb is dead past
+// bound + 2*rb.
 template <bool MASKED>
-GSE_DEVICE void column_max_tile(const uint16_t* qt, const float* nt, const bf16x8_t (&kf)[2][4], float (&cs)[2],
+GSE_DEVICE void column_max_tile(const uint16_t* qt, const float* nt, const bf16x8_t (&kf)[4][2], float (&cs)[2],
                                 float scale2, int bound, int lane) {
 #pragma unroll
-  for (int cb = 0; cb < 2; ++cb) {
-    bf16x8_t qf[4];
-    k_fragments(qt, cb, lane, qf);
-    f32x4_t nn[4];
+  for (int rb = 0; rb < 4; ++rb) {
+    bf16x8_t qf[2];
+    fragments(qt, rb, lane, qf);
+    const f32x4_t nn = *reinterpret_cast<const f32x4_t*>(nt + 16 * rb + 4 * (lane >> 4));
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
-      nn[b] = *reinterpret_cast<const f32x4_t*>(nt + 32 * cb + 8 * b + 4 * (lane >> 5));
+    for (int kp = 0; kp < 2; ++kp) {
+      float y[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      const f32x16_t d = dot64(qf, kf[kb]);
-      float y[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
+      for (int h = 0; h < 2; ++h) {
+        const f32x4_t d = dot64(qf, kf[2 * kp + h]);
         float x[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x[r] = fmaf(d[4 * b + r], scale2, nn[b][r]);
-        y[b] = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
-        if (MASKED && 32 * kb > bound + 4 * cb + b) y[b] = -INFINITY;
+        for (int r = 0; r < 4; ++r) x[r] = fmaf(d[r], scale2, nn[r]);
+        y[h] = fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3]));
+        if (MASKED && 32 * kp + 16 * h > bound + 2 * rb) y[h] = -INFINITY;
       }
-#pragma unroll
-      for (int b = 0; b < 4; b += 2) {  // lower lanes take query b, upper lanes query b + 1
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[b]), __float_as_uint(y[b + 1]), false, false);
-        cs[kb] += fast_exp2(vmax(__uint_as_float(r[0]), __uint_as_float(r[1])));
-      }
-      cs[kb] = in_vgpr(cs[kb]);
-      __builtin_amdgcn_sched_barrier(0);
+      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y[0]), __float_as_uint(y[1]), false, false);
+      cs[kp] = formed(cs[kp] + fast_exp2(vmax(__uint_as_float(r[0]), __uint_as_float(r[1]))));
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
@@ -461,7 +471,7 @@ GSE_DEVICE float scatter_sum(float (&v)[N], int lane) {
 }
 
 template <bool MAX_MODE>
-__global__ __launch_bounds__(p2::THREADS, MAX_MODE ? 4 : 3) void prefill_score_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(p2::THREADS, 4) void prefill_score_kernel(PrefillArgs a) {
   using namespace pf;
   using namespace p2;
   __shared__ __attribute__((aligned(16))) uint16_t qtile[2][QT * GROUP * KROW];
@@ -482,16 +492,16 @@ __global__ __launch_bounds__(p2::THREADS, MAX_MODE ? 4 : 3) void prefill_score_k
   if (q0 >= q1) return;
   const int kend = min(int(a.total), bound0 + q1);  // keys the item credits
 
-  // The wave's keys: lane holds dims [16*ks + 8*(lane/32), +8) of keys kw + 32*kb + lane%32 (past
-  // the list: its last key, never credited).
-  bf16x8_t kf[2][4];
+  // The wave's keys: lane (col, grp) holds dims [8*grp, +8) and [32 + 8*grp, +8) of keys
+  // kw + 16*kb + col (past the list: its last key, never credited).
+  bf16x8_t kf[4][2];
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    const int key = min(kw + 32 * kb + (lane & 31), int(a.total) - 1);
+  for (int kb = 0; kb < 4; ++kb) {
+    const int key = min(kw + 16 * kb + (lane & 15), int(a.total) - 1);
     const int64_t s = load_index_dyn(a.slots, a.slots_dtype, key);
-    const auto kp = as_global(a.k) + s * a.kv_ss + int64_t(g) * a.kv_sh + 8 * (lane >> 5);
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) kf[kb][ks] = as_bf16x8(gload16(kp + 16 * ks));
+    const auto kp = as_global(a.k) + s * a.kv_ss + int64_t(g) * a.kv_sh + 8 * (lane >> 4);
+    kf[kb][0] = as_bf16x8(gload16(kp));
+    kf[kb][1] = as_bf16x8(gload16(kp + 32));
   }
   // Query tile load: thread t stages 16 bytes of rows t/8 (query q + row/8, head row%8) and t/8 + 32
   // (four queries on); the next tile is in flight while one computes. Rows past the chunk are zero
@@ -515,22 +525,22 @@ __global__ __launch_bounds__(p2::THREADS, MAX_MODE ? 4 : 3) void prefill_score_k
   };
   store_tile(0, load_q(q0), load_q(q0 + QT / 2), load_n(q0));
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) landed(kf[kb][ks]);
+  for (int kb = 0; kb < 4; ++kb) {
+    landed(kf[kb][0]);
+    landed(kf[kb][1]);
+  }
   __syncthreads();
 
-  f32x16_t sums[2] = {};
+  f32x4_t sums[4] = {};
   float maxes[2] = {0.f, 0.f};
-  const float scale2 = in_vgpr(a.scale2);
-  // The wave's bound of query q, relative to the lane's first key.
-  const int rel = bound0 - kw - (MAX_MODE ? lane & 31 : 4 * (lane >> 5));
+  const float scale2 = a.scale2;
+  // The bound of the lane's row of a tile at query 0, from the lane's first key on.
+  const int rel = bound0 - kw + (MAX_MODE ? (lane >> 5) - (lane & 15) : ((lane & 15) >> 3) - 4 * (lane >> 4));
   auto tile_step = [&](int q, int p, auto whole) {
     constexpr bool WHOLE = decltype(whole)::value;
     const uint4 x0 = load_q(q + QT), x1 = load_q(q + QT + QT / 2);
     const float n = load_n(q + QT);
-    // The lane's bound of the first query (sum mode: of its own row's).
-    const int bound = rel + q + (MAX_MODE ? 0 : (lane & 31) >> 3);
+    const int bound = rel + q;
     auto compute = [&](auto masked) {
       constexpr bool MASKED = decltype(masked)::value;
       if constexpr (MAX_MODE)
@@ -560,20 +570,15 @@ __global__ __launch_bounds__(p2::THREADS, MAX_MODE ? 4 : 3) void prefill_score_k
   float total;
   int key;
   if constexpr (MAX_MODE) {
-    const float t0 = xor32_sum(maxes[0]), t1 = xor32_sum(maxes[1]);
+    const float t0 = xor32_sum(maxes[0]), t1 = xor32_sum(maxes[1]);  // both query parities
     total = lane < 32 ? t0 : t1;
     key = kw + lane;
   } else {
     float v[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {  // lane bit 4 selects the key block
-      const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(sums[0][i]), __float_as_uint(sums[1][i]), false,
-                                                      false);
-      v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    }
+    for (int i = 0; i < 16; ++i) v[i] = sums[i / 4][i % 4];
     total = scatter_sum(v, lane);  // lane % 16 selects the register
-    const int i = lane & 15;
-    key = kw + 32 * ((lane >> 4) & 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    key = kw + 16 * ((lane & 15) >> 2) + 4 * (lane >> 4) + (lane & 3);
   }
   if (key < kend)
     unsafeAtomicAdd(&a.scores[int64_t(g) * a.ssg + load_index_dyn(a.slots, a.slots_dtype, key) * a.sss], total);
