@@ -26,7 +26,6 @@ constexpr int GROUP = 8;
 constexpr int QB = 64;          // queries per workgroup
 constexpr int KT = 64;          // keys per tile (4 key-blocks of 16)
 constexpr int KROW = D + 8;     // padded bf16 row of a staged key
-constexpr int RING = 16;        // tiles of column sums held before they are added to the scores
 // A row's reference follows its sums: past kMoveSum it moves up by a power of two (exponents near
 // zero keep the exponential's argument exact), past kRescaleSum, near the overflow, to the tile's
 // maximum.
@@ -199,10 +198,49 @@ GSE_DEVICE void row_sum_tile(const uint16_t* kt, const bf16x8_t (&qf)[4][2], flo
   }
 }
 
+// Staging of a walk over 64-key tiles by 512 threads: thread t brings 16 bytes of key t/8. Tile t's
+// K rows are loaded into registers during tile t - 2 and stored to LDS at the end of tile t - 1,
+// and its slot indices are read two tiles before that, in two register sets alternating by tile
+// parity (the walks are unrolled by two: copying one into the other would wait for the loads in
+// flight into it). Keys past kend read slot 0's row (any valid row) and are masked.
+struct KeyTiles {
+  typedef uint16_t Tile[pf::KT * pf::KROW];
+  const PrefillArgs& a;
+  const int kend, lk, lp;
+  const global_ptr<const uint16_t> base;
+  uint4 row[2];     // row[p]: K rows of the tile of offset parity p in flight
+  int32_t slot[2];  // slot[p]: slot of the next tile of parity p whose rows are not yet loaded
+
+  GSE_DEVICE KeyTiles(const PrefillArgs& a_, int g, int kend_)
+      : a(a_), kend(kend_), lk(threadIdx.x >> 3), lp(threadIdx.x & 7),
+        base(as_global(a_.k) + int64_t(g) * a_.kv_sh + 8 * (threadIdx.x & 7)) {}
+  GSE_DEVICE int32_t slot_at(int ti) const {
+    const int key = ti * pf::KT + lk;
+    return key < kend ? int32_t(load_index_dyn(a.slots, a.slots_dtype, key)) : 0;
+  }
+  GSE_DEVICE uint4 load(int32_t s) const { return gload16(base + int64_t(s) * a.kv_ss); }
+  GSE_DEVICE void store(Tile& tile, const uint4& x) const { *reinterpret_cast<uint4*>(&tile[lk * pf::KROW + 8 * lp]) = x; }
+  // Tile ti0 to LDS, the next ones on their way.
+  GSE_DEVICE void start(int ti0, Tile (&tiles)[2]) {
+    const int32_t s0 = slot_at(ti0), s1 = slot_at(ti0 + 1);
+    slot[0] = slot_at(ti0 + 2);
+    slot[1] = slot_at(ti0 + 3);
+    const uint4 y = load(s0);
+    row[1] = load(s1);
+    store(tiles[0], y);
+  }
+  // At the start of tile ti, of parity p: tile ti + 2's rows and tile ti + 4's slots go out.
+  GSE_DEVICE void ahead(int ti, int p) {
+    row[p] = load(slot[p]);
+    slot[p] = slot_at(ti + 4);
+  }
+  GSE_DEVICE void stage(int p, Tile (&tiles)[2]) { store(tiles[p], row[p]); }
+};
+
 __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArgs a) {
   using namespace pf;
   using p1::QW;
-  __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
+  __shared__ __attribute__((aligned(16))) KeyTiles::Tile ktile[2];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Block i: KV head i % kv_heads, then the query block from the end (the longest causal ranges
@@ -238,29 +276,8 @@ __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArg
   }
   const float scale2 = a.scale2;
 
-  // Tile load: thread t stages 16 bytes of key t/8. Tile t's K rows are loaded into registers
-  // during tile t - 2 and stored to LDS at the end of tile t - 1, and its slot indices are read
-  // two tiles before that, in two register sets alternating by tile parity (the loop is unrolled
-  // by two: copying one into the other would wait for the loads in flight into it). Keys past
-  // kend read slot 0's row (any valid row) and are masked.
-  const int lk = threadIdx.x >> 3, lp = threadIdx.x & 7;
-  auto slot_at = [&](int ti) -> int32_t {
-    const int key = ti * KT + lk;
-    return key < kend ? int32_t(load_index_dyn(a.slots, a.slots_dtype, key)) : 0;
-  };
-  const auto kbase = as_global(a.k) + int64_t(g) * a.kv_sh + 8 * lp;
-  auto load_row = [&](int32_t s) { return gload16(kbase + int64_t(s) * a.kv_ss); };
-  auto store_row = [&](int p, const uint4& x) { *reinterpret_cast<uint4*>(&ktile[p][lk * KROW + 8 * lp]) = x; };
-  uint4 xk[2];    // xk[p]: K rows of the tile of offset parity p in flight
-  int32_t sk[2];  // sk[p]: slot of the next tile of parity p whose rows are not yet loaded
-  {
-    const int32_t s0 = slot_at(ti0), s1 = slot_at(ti0 + 1);
-    sk[0] = slot_at(ti0 + 2);
-    sk[1] = slot_at(ti0 + 3);
-    const uint4 y = load_row(s0);
-    xk[1] = load_row(s1);
-    store_row(0, y);
-  }
+  KeyTiles keys(a, g, kend);
+  keys.start(ti0, ktile);
   // The query fragments are in registers before the walk starts: a wait for them inside the
   // loop would also wait for every load in flight at the top of each tile.
 #pragma unroll
@@ -296,14 +313,13 @@ __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArg
   auto tile_step = [&](int ti, auto general, auto parity) {
     constexpr bool GENERAL = decltype(general)::value;
     constexpr int P = decltype(parity)::value;  // (ti - ti0) & 1
-    xk[P] = load_row(sk[P]);
-    sk[P] = slot_at(ti + 4);
+    keys.ahead(ti, P);
     const int t0 = ti * KT;
     if (!GENERAL)
       row_sum_tile<false>(ktile[P], qf, nref, sum, scale2, 0, lane);
     else if (wave_live && t0 < wave_kend)
       row_sum_tile<true>(ktile[P], qf, nref, sum, scale2, qpos - t0, lane);
-    if (ti + 1 < ti1) store_row(1 - P, xk[1 - P]);
+    if (ti + 1 < ti1) keys.stage(1 - P, ktile);
     __syncthreads();
   };
   using P0 = std::integral_constant<int, 0>;
@@ -816,6 +832,8 @@ __global__ __launch_bounds__(pb::THREADS) void prefill_block_kernel(PrefillArgs 
 // Static regret diagnostic (pass 3)
 // ---------------------------------------------------------------------------
 constexpr int DIAG_MAX_SPECS = 8;
+constexpr int FOLD = 4;  // tiles per fold of the waves' column sums: a key and table per thread
+static_assert(2 * FOLD * pf::KT == p1::THREADS, "one (table, key) per thread");
 
 struct DiagArgs {
   PrefillArgs p;         // q, keys, slots, sinks, scale, row normalisers of pass 1
@@ -828,183 +846,194 @@ struct DiagArgs {
   float lost_scale;      // 1 / (query heads * full layers)
 };
 
+// Bit masks of the diagnostic's specs: words[(s * kv_heads + g) * n_words ..], bit k%32 of word k/32
+// set when key k < n is not resident. One wave per 64 keys of a (spec, KV head).
+__global__ __launch_bounds__(256) void pack_evicted_kernel(const uint8_t* resident, int64_t res_ss, int64_t res_sg,
+                                                           int kv_heads, int64_t n, uint32_t* words,
+                                                           int64_t n_words) {
+  const int sg = blockIdx.y, s = sg / kv_heads, g = sg % kv_heads;
+  const int64_t key = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  const bool gone = key < n && !resident[s * res_ss + g * res_sg + key];
+  const uint64_t bits = __builtin_amdgcn_ballot_w64(gone);
+  const int lane = threadIdx.x & 63;
+  const int64_t w = (key >> 6) * 2 + lane;
+  if (lane < 2 && w < n_words) words[sg * n_words + w] = uint32_t(bits >> (32 * lane));
+}
+
 // Pass 3 of a diagnostic chunk: the exact probabilities of pass 1's normalisers, added to two
 // position-indexed score tables (sum and max over each KV head's query heads, summed over the
 // chunk's queries), and every spec's lost mass per query: the group-summed probability on
-// keys the spec has evicted, summed over keys and KV heads, times lost_scale. Geometry as pass 1
-// (8 waves x 4 row-blocks per workgroup of 64 queries); K tiles through LDS, column sums through
-// two LDS rings.
-__global__ __launch_bounds__(64 * 8) void diagnose_kernel(DiagArgs da) {
+// keys the spec has evicted, summed over keys and KV heads, times lost_scale. Items as pass 1 (64
+// queries, a range of key tiles), S = Q . K^T: a lane holds 4 heads of one query for one key, so a
+// spec costs one FMA (with its 0/1 bit of the key) per 4 logits; column sums and maxima meet by lane
+// swaps, then through a column per wave in LDS (float atomics there took 194 cycles each, half the
+// kernel). NS, the number of specs, is a template argument: a run-time bound on
+// the unrolled spec loop cost a branch per (spec, 16x16 block). Vector issue bound as pass 1; 2048
+// queries after 14,336 keys, 4 specs: 1292 -> 684 us, 65 % of the cycles issuing (2 waves per SIMD).
+template <int NS>
+__global__ __launch_bounds__(p1::THREADS, NS == 0 ? 4 : 2) void diagnose_kernel(DiagArgs da) {
   using namespace pf;
+  using p1::QW;
   const PrefillArgs& a = da.p;
-  constexpr int RB = 4;
-  __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
-  __shared__ float ring_sum[RING * KT], ring_max[RING * KT];
+  __shared__ __attribute__((aligned(16))) KeyTiles::Tile ktile[2];
+  // Column sums and maxima of each wave, two rings of FOLD tiles: one fills while the other folds.
+  __shared__ float cols[2][2][p1::WAVES][FOLD * KT];
+  __shared__ uint32_t evicted[2][2 * DIAG_MAX_SPECS];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int64_t nqb = (a.count + QB - 1) / QB;
+  const int nqb = int((a.count + QB - 1) / QB);
   const int g = blockIdx.x % a.kv_heads;
-  const int64_t qb0 = (nqb - 1 - int64_t(blockIdx.x / a.kv_heads)) * QB;
-  const int64_t i0 = qb0 + 2 * RB * wave;
-  const int64_t last_q = (qb0 + QB < a.count ? qb0 + QB : a.count) - 1;
-  const int64_t kend = a.prefix_len + last_q + 1;
+  const int item = blockIdx.x / a.kv_heads;
+  const int split = item / nqb;
+  const int64_t qb0 = int64_t(nqb - 1 - item % nqb) * QB;
+  const int last_q = int((qb0 + QB < a.count ? qb0 + QB : a.count) - 1);
+  const int kend = int(a.prefix_len) + last_q + 1;
+  const int ntiles = (kend + KT - 1) / KT;
+  const int ranges = key_ranges(ntiles, a.tiles);
+  if (split >= ranges) return;
+  const int ti0 = int(int64_t(ntiles) * split / ranges), ti1 = int(int64_t(ntiles) * (split + 1) / ranges);
+  const int i0 = int(qb0) + QW * wave;
   const bool wave_live = i0 < a.count;
-  const int64_t wave_kend = a.prefix_len + (i0 + 2 * RB - 1 < a.count ? i0 + 2 * RB - 1 : a.count - 1) + 1;
+  const int wave_kend = int(a.prefix_len) + min(i0 + QW - 1, int(a.count) - 1) + 1;
 
-  bf16x8_t qa[RB][2];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int64_t qi = i0 + 2 * rb + col / 8;
-    qa[rb][0] = bf16x8_t{};
-    qa[rb][1] = bf16x8_t{};
-    if (qi < a.count) {
-      const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * GROUP + col % 8) * a.q_sh + 16 * grp;
-      qa[rb][0] = as_bf16x8(*reinterpret_cast<const uint4*>(qp));
-      qa[rb][1] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 8));
-    }
-  }
+  // A fragments: row col of block rb is query i0 + 2*rb + col/8, head g*8 + col%8. The lane's D
+  // rows: query i0 + 2*rb + grp/2, heads hq0 + r.
   const int hq0 = g * GROUP + 4 * (grp & 1);
-  float nrm[RB][4];
-  float lost[DIAG_MAX_SPECS][RB];
+  bf16x8_t qf[4][2];
+  f32x4_t nn[4];  // negated normalisers (-inf past the chunk: probability 0)
+  float lost[NS > 0 ? NS : 1][4];
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int64_t qi = i0 + 2 * rb + (grp >> 1);
+  for (int rb = 0; rb < 4; ++rb) {
+    const int64_t qi = i0 + 2 * rb + (col >> 3), qd = i0 + 2 * rb + (grp >> 1);
+    const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * GROUP + (col & 7)) * a.q_sh + 8 * grp;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) nrm[rb][r] = qi < a.count ? a.norm2[qi * a.q_heads + hq0 + r] : INFINITY;
+    for (int h = 0; h < 2; ++h)
+      qf[rb][h] = qi < a.count ? as_bf16x8(*reinterpret_cast<const uint4*>(qp + 32 * h)) : bf16x8_t{};
 #pragma unroll
-    for (int sp = 0; sp < DIAG_MAX_SPECS; ++sp) lost[sp][rb] = 0.f;
+    for (int r = 0; r < 4; ++r) nn[rb][r] = qd < a.count ? -a.norm2[qd * a.q_heads + hq0 + r] : -INFINITY;
+#pragma unroll
+    for (int sp = 0; sp < NS; ++sp) lost[sp][rb] = 0.f;
   }
-  for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) {
-    ring_sum[t] = 0.f;
-    ring_max[t] = 0.f;
-  }
-
-  const bool loader = threadIdx.x < 256;
-  const int lk = (threadIdx.x >> 2) & 63, lp = threadIdx.x & 3;
-  auto load_tile = [&](int64_t t0, uint4& x0, uint4& x1) {
-    const int64_t key = t0 + lk;
-    const int64_t s = key < kend ? load_index_dyn(a.slots, a.slots_dtype, key) : 0;
-    const auto kp = as_global(a.k) + s * a.kv_ss + int64_t(g) * a.kv_sh + 16 * lp;
-    x0 = gload16(kp);
-    x1 = gload16(kp + 8);
+  KeyTiles keys(a, g, kend);
+  // The specs' words of a tile travel with its K rows (as KeyTiles): thread t < 2 * NS brings half
+  // t%2 of spec t/2. Loaded where they are used they would cost a memory latency per tile.
+  const auto words = as_global(da.evicted) + int64_t(g) * da.ev_sg +
+                     (int(threadIdx.x) < 2 * NS ? (threadIdx.x >> 1) * da.ev_ss + (threadIdx.x & 1) : 0);
+  const int last_tile = ntiles - 1;
+  auto load_words = [&](int ti) { return NS > 0 ? words[2 * min(ti, last_tile)] : 0u; };
+  auto stage_words = [&](int p, uint32_t w) {
+    if (int(threadIdx.x) < 2 * NS) evicted[p][threadIdx.x] = w;
   };
-  auto store_tile = [&](int buf, uint4 x0, uint4 x1) {
-    uint16_t* dst = &ktile[buf][lk * KROW + 16 * lp];
-    *reinterpret_cast<uint4*>(dst) = x0;
-    *reinterpret_cast<uint4*>(dst + 8) = x1;
-  };
-  const int ntiles = int((kend + KT - 1) / KT);
-  uint4 x0 = {}, x1 = {};
-  if (loader) {
-    load_tile(0, x0, x1);
-    store_tile(0, x0, x1);
+  uint32_t word[2] = {0u, load_words(ti0 + 1)};
+  stage_words(0, load_words(ti0));
+  keys.start(ti0, ktile);
+#pragma unroll
+  for (int rb = 0; rb < 4; ++rb) {
+    landed(qf[rb][0]);
+    landed(qf[rb][1]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) landed(nn[rb][r]);
   }
   __syncthreads();
 
-#pragma unroll 1
-  for (int ti = 0; ti < ntiles; ++ti) {
-    const int64_t t0 = int64_t(ti) * KT;
-    if (loader && ti + 1 < ntiles) load_tile(t0 + KT, x0, x1);
+  const int qpos = int(a.prefix_len) + i0 + (grp >> 1) - col;  // causal bound of block 0, from the lane's key
+  const float scale2 = a.scale2;
+  auto tile_step = [&](int ti, auto parity) {
+    constexpr int P = decltype(parity)::value;  // (ti - ti0) & 1
+    word[P] = load_words(ti + 2);
+    keys.ahead(ti, P);
+    const int t0 = ti * KT;
+    float tsum = 0.f, tmax = 0.f;  // of key t0 + lane
     if (wave_live && t0 < wave_kend) {
-      const uint16_t* kt = ktile[ti & 1];
-      bf16x8_t kb0[4], kb1[4];
+      float cs[4] = {0.f, 0.f, 0.f, 0.f}, cm[2] = {0.f, 0.f};
+      auto rows = [&](auto masked) {
+        constexpr bool MASKED = decltype(masked)::value;
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const uint16_t* kr = kt + (16 * kb + col) * KROW + 16 * grp;
-        kb0[kb] = as_bf16x8(*reinterpret_cast<const uint4*>(kr));
-        kb1[kb] = as_bf16x8(*reinterpret_cast<const uint4*>(kr + 8));
-      }
-      // Evicted bits of this lane's four keys, per spec (bit kb of ev[sp]).
-      uint32_t ev[DIAG_MAX_SPECS];
+        for (int kp = 0; kp < 2; ++kp) {
+          bf16x8_t kf[2][2];
+          float gone[NS > 0 ? NS : 1][2];  // 1 for the specs that evicted the lane's keys
 #pragma unroll
-      for (int sp = 0; sp < DIAG_MAX_SPECS; ++sp) {
-        ev[sp] = 0;
-        if (sp < da.n_specs) {
-          const uint32_t* w = da.evicted + sp * da.ev_ss + int64_t(g) * da.ev_sg + (t0 >> 5);
-          const uint32_t w0 = w[0], w1 = w[1];
-          ev[sp] = ((w0 >> col) & 1u) | (((w0 >> (16 + col)) & 1u) << 1) | (((w1 >> col) & 1u) << 2) |
-                   (((w1 >> (16 + col)) & 1u) << 3);
-        }
-      }
-      const int64_t rel = t0 + col - (a.prefix_len + i0);
-      float cs[4] = {0.f, 0.f, 0.f, 0.f}, cm[4] = {0.f, 0.f, 0.f, 0.f};
-      // The causal mask only on the tiles that reach past the wave's first query.
-      auto rows = [&](auto masked_tag) {
-        constexpr bool MASKED = decltype(masked_tag)::value;
+          for (int h = 0; h < 2; ++h) fragments(ktile[P], 2 * kp + h, lane, kf[h]);
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          f32x4_t d[4];
+          for (int sp = 0; sp < NS; ++sp) {
+            const uint32_t w = evicted[P][2 * sp + kp];
 #pragma unroll
-          for (int kb = 0; kb < 4; ++kb) {
-            d[kb] = mfma16x16x32(qa[rb][0], kb0[kb], f32x4_t{0.f, 0.f, 0.f, 0.f});
-            d[kb] = mfma16x16x32(qa[rb][1], kb1[kb], d[kb]);
-          }
-          if (MASKED) {
-            const int64_t qrel = 2 * rb + (grp >> 1);
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
-              if (rel + 16 * kb > qrel)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) d[kb][r] = -INFINITY;
+            for (int h = 0; h < 2; ++h) gone[sp][h] = float((w >> (16 * h + col)) & 1u);
           }
 #pragma unroll
-          for (int kb = 0; kb < 4; ++kb) {
-            const float p0 = fast_exp2(fmaf(d[kb][0], a.scale2, -nrm[rb][0]));
-            const float p1 = fast_exp2(fmaf(d[kb][1], a.scale2, -nrm[rb][1]));
-            const float p2 = fast_exp2(fmaf(d[kb][2], a.scale2, -nrm[rb][2]));
-            const float p3 = fast_exp2(fmaf(d[kb][3], a.scale2, -nrm[rb][3]));
-            const float psum = (p0 + p1) + (p2 + p3);
-            cs[kb] += psum;
-            cm[kb] += xor16_max(fmaxf(fmaxf(p0, p1), fmaxf(p2, p3)));
+          for (int rb = 0; rb < 4; ++rb) {
+            float y[2];
 #pragma unroll
-            for (int sp = 0; sp < DIAG_MAX_SPECS; ++sp)
-              if (sp < da.n_specs) lost[sp][rb] += (ev[sp] >> kb) & 1u ? psum : 0.f;
+            for (int h = 0; h < 2; ++h) {
+              f32x4_t d = dot64(qf[rb], kf[h]);
+              if (MASKED && 32 * kp + 16 * h > qpos - t0 + 2 * rb) d = f32x4_t{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+              for (int r = 0; r < 4; ++r) d[r] = fast_exp2(fmaf(d[r], scale2, nn[rb][r]));
+              const float psum = sum4(d);
+              cs[2 * kp + h] += psum;
+              y[h] = fmaxf(fmaxf(d[0], d[1]), fmaxf(d[2], d[3]));
+#pragma unroll
+              for (int sp = 0; sp < NS; ++sp) lost[sp][rb] = fmaf(psum, gone[sp][h], lost[sp][rb]);
+            }
+            // The maximum over all 8 heads, for the two key blocks at once (as column_max_tile).
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y[0]), __float_as_uint(y[1]), false, false);
+            cm[kp] = formed(cm[kp] + vmax(__uint_as_float(r[0]), __uint_as_float(r[1])));
+            __builtin_amdgcn_sched_barrier(0);
           }
-          __builtin_amdgcn_sched_barrier(0);
         }
       };
-      if (t0 + KT - 1 > a.prefix_len + i0)
+      if (t0 + KT - 1 > int(a.prefix_len) + i0)
         rows(std::true_type{});
       else
         rows(std::false_type{});
-      float* rs = ring_sum + (ti % RING) * KT;
-      float* rm = ring_max + (ti % RING) * KT;
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) {
-        const float tsum = xor32_sum(xor16_sum(cs[kb]));
-        const float tmax = xor32_sum(cm[kb]);
-        if (grp == 0) {
-          atomicAdd(&rs[16 * kb + col], tsum);
-          atomicAdd(&rm[16 * kb + col], tmax);
-        }
-      }
+      // Lane l ends with key l: lane bit 4 selects the key block of a pair, bit 5 the pair.
+      auto join16 = [](float x, float y) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      };
+      auto join32 = [](float x, float y) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+      };
+      tsum = join32(join16(cs[0], cs[1]), join16(cs[2], cs[3]));
+      tmax = join32(cm[0], cm[1]);
     }
-    if (loader && ti + 1 < ntiles) store_tile((ti + 1) & 1, x0, x1);
+    const int n = ti - ti0, ring = (n / FOLD) & 1, slot = n % FOLD;
+    cols[ring][0][wave][slot * KT + lane] = tsum;
+    cols[ring][1][wave][slot * KT + lane] = tmax;
+    if (ti + 1 < ti1) {
+      stage_words(1 - P, word[1 - P]);
+      keys.stage(1 - P, ktile);
+    }
     __syncthreads();
-    if ((ti + 1) % RING == 0 || ti + 1 == ntiles) {
-      const int64_t base = int64_t(ti - ti % RING) * KT;
-      for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) {
-        const int64_t key = base + t;
-        if (key < kend) {
-          // Diagnostic score tables are indexed by position (the chunk's CSR column).
-          unsafeAtomicAdd(&a.scores[int64_t(g) * a.ssg + key * a.sss], ring_sum[t]);
-          unsafeAtomicAdd(&da.score_max[int64_t(g) * a.ssg + key * a.sss], ring_max[t]);
-        }
-        ring_sum[t] = 0.f;
-        ring_max[t] = 0.f;
+    if (slot == FOLD - 1 || ti + 1 == ti1) {
+      // One thread per key and table. Diagnostic score tables are indexed by position (the chunk's
+      // CSR column).
+      const int table = threadIdx.x / (FOLD * KT), at = threadIdx.x % (FOLD * KT);
+      const int key = (ti - slot) * KT + at;
+      if (at < (slot + 1) * KT && key < kend) {
+        float total = 0.f;
+#pragma unroll
+        for (int w = 0; w < p1::WAVES; ++w) total += cols[ring][table][w][at];
+        unsafeAtomicAdd((table ? da.score_max : a.scores) + int64_t(g) * a.ssg + key * a.sss, total);
       }
-      __syncthreads();
     }
+  };
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
+#pragma unroll 1
+  for (int ti = ti0; ti < ti1; ti += 2) {
+    tile_step(ti, P0{});
+    if (ti + 1 < ti1) tile_step(ti + 1, P1{});
   }
 
-  if (wave_live) {
-    // Per spec and query: the lane sums over its key columns (16 lanes) and the two head halves.
+  if (NS > 0 && wave_live) {
+    // Per spec and query: the lane's sum over its key columns (16 lanes) and the two head halves.
 #pragma unroll
-    for (int sp = 0; sp < DIAG_MAX_SPECS; ++sp) {
-      if (sp >= da.n_specs) break;
+    for (int sp = 0; sp < NS; ++sp)
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
+      for (int rb = 0; rb < 4; ++rb) {
         float v = lost[sp][rb];
 #pragma unroll
         for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, kWave);
@@ -1012,7 +1041,6 @@ __global__ __launch_bounds__(64 * 8) void diagnose_kernel(DiagArgs da) {
         const int64_t qi = i0 + 2 * rb + (grp >> 1);
         if (col == 0 && (grp & 1) == 0 && qi < a.count) atomicAdd(&da.lost[sp * da.lost_ss + qi], v * da.lost_scale);
       }
-    }
   }
 }
 
@@ -1146,10 +1174,29 @@ extern "C" int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_s
   da.lost_ss = lost_stride_s;
   da.lost_scale = lost_scale;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int64_t blocks = (count + pf::QB - 1) / pf::QB * kv_heads;
-  if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "diagnose: chunk too large");
-  const dim3 grid{static_cast<uint32_t>(blocks)};
   if (int rc = launch_norms(da.p, workspace, s)) return rc;
-  hipLaunchKernelGGL(diagnose_kernel, grid, dim3(64 * 8), 0, s, da);
+  // launch_norms has set the key ranges and checked the grid.
+  const dim3 grid{static_cast<uint32_t>((count + pf::QB - 1) / pf::QB * kv_heads * da.p.splits)};
+  static void (*const kernels[])(DiagArgs) = {diagnose_kernel<0>, diagnose_kernel<1>, diagnose_kernel<2>,
+                                              diagnose_kernel<3>, diagnose_kernel<4>, diagnose_kernel<5>,
+                                              diagnose_kernel<6>, diagnose_kernel<7>, diagnose_kernel<8>};
+  static_assert(sizeof(kernels) / sizeof(kernels[0]) == DIAG_MAX_SPECS + 1, "one instance per spec count");
+  hipLaunchKernelGGL(kernels[n_specs], grid, dim3(p1::THREADS), 0, s, da);
   return gse_launch_check("diagnose pass 3");
+}
+
+extern "C" int gse_pack_evicted(const void* resident, int64_t resident_stride_s, int64_t resident_stride_g,
+                                int n_specs, int kv_heads, int64_t n, uint32_t* words, int64_t n_words,
+                                gse_stream_t stream) {
+  if (n_specs < 0 || n_specs > DIAG_MAX_SPECS || kv_heads < 1 || kv_heads > 1024 || n < 0)
+    return gse_fail(GSE_EINVAL, "pack: 0..8 policy specs, kv_heads in 1..1024");
+  if (n_words < (n + 63) / 64 * 2) return gse_fail(GSE_EINVAL, "pack: words must cover the keys rounded up to 64");
+  if (!n_specs || !n_words) return GSE_OK;
+  if (!resident || !words) return gse_fail(GSE_EINVAL, "pack: null pointer");
+  const int64_t blocks = (n_words + 7) / 8;  // 256 keys each
+  if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "pack: too many keys");
+  hipLaunchKernelGGL(pack_evicted_kernel, dim3(uint32_t(blocks), n_specs * kv_heads), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), static_cast<const uint8_t*>(resident), resident_stride_s,
+                     resident_stride_g, kv_heads, n, words, n_words);
+  return gse_launch_check("pack evicted");
 }

@@ -529,6 +529,11 @@ int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_stride_h, in
                        int64_t evicted_stride_s, int64_t evicted_stride_g, float* lost, int64_t lost_stride_s,
                        float lost_scale, int q_heads, int kv_heads, int head_dim, float sm_scale,
                        void* workspace, int64_t workspace_bytes, gse_stream_t stream);
+/* A diagnostic's bit masks: words[(s * kv_heads + g) * n_words + k/32], bit k%32 set when
+ * resident[s, g, k] (bytes, unit stride over k < n) is zero; 0 past n. n_words (even)
+ * covers n rounded up to 64. */
+int gse_pack_evicted(const void* resident, int64_t resident_stride_s, int64_t resident_stride_g, int n_specs,
+                     int kv_heads, int64_t n, uint32_t* words, int64_t n_words, gse_stream_t stream);
 
 /*
  * replay_layer_difference — static replay's per-query error of the first full

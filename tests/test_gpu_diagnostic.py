@@ -135,3 +135,47 @@ def test_hooks_write_the_diagnostic_payload(runtime, tmp_path, monkeypatch):
     assert np.array_equal(payload["lost"], entry["lost"].cpu().numpy())
     assert payload["lost"][:, :2048].sum() == 0 and payload["lost"][:, 2048:].min() > 0
     assert row not in st.entries
+
+
+# One kernel instance per spec count; edges of the query blocks, the 64-key tiles, the folds of four
+# tiles and the masks' words; every spec holds other positions of a table that does not start at a
+# word's first byte.
+@pytest.mark.parametrize("specs,count,start", [
+    (1, 1, 0), (2, 37, 0), (3, 64, 255), (4, 65, 256), (5, 130, 1000), (6, 9, 2049), (7, 200, 31), (8, 100, 4100)])
+def test_chunk_of_any_spec_count_against_64_bits(runtime, specs, count, start):
+    from gstar_evict import diagnostics
+    ge = runtime
+    total = start + count
+    g = torch.Generator(device="cuda").manual_seed(100 * specs + count)
+    b = backend(rows=2, width=64, slots=total + 8, gen=torch.Generator().manual_seed(count))
+    st = ge.state(b)
+    keys = b.token_to_kv_pool.get_key_buffer(1)
+    slots = torch.randperm(total, generator=g, device="cuda") + 1
+    q = torch.randn((count, 64, 64), generator=g, device="cuda").to(torch.bfloat16)
+    sinks = torch.randn(64, generator=g, device="cuda")
+    held = torch.rand((specs, len(FULL), 8, total + 77), generator=g, device="cuda") < 0.5
+    tables = {name: torch.zeros((len(FULL), 8, total + 77), device="cuda") for name in ("score_sum", "score_max")}
+    entry = dict(tables, resident=held, lost=torch.zeros((specs, total + 77), device="cuda"), frontier=start,
+                 layers_seen=set(), specs=[])
+    chunks = [(0, count)] if start // 2048 == (total - 1) // 2048 else [(0, 2048 - start % 2048),
+                                                                       (2048 - start % 2048, count)]
+    entry["frontier"] = 1 << 30  # no boundary of its own
+    for lo, hi in chunks:
+        diagnostics.diagnose(st, entry, 0, layer(1), q[lo:hi], keys, sinks, slots[:start + hi], start + lo)
+    assert not entry.get("error")
+    lost = torch.zeros((specs, total + 77), dtype=torch.float64, device="cuda")
+    sums, maxes = (torch.zeros((8, total + 77), dtype=torch.float64, device="cuda") for _ in range(2))
+    hidden = torch.arange(total, device="cuda") > start + torch.arange(count, device="cuda")[:, None]
+    for h in range(8):
+        x = torch.matmul(q[:, 8 * h:8 * h + 8].double().transpose(0, 1), keys[slots, h].double().t().contiguous())
+        x = (x * 0.125).masked_fill(hidden, -torch.inf)
+        sink = sinks[8 * h:8 * h + 8].double().view(8, 1, 1)
+        p = torch.exp(x - torch.logaddexp(torch.logsumexp(x, -1, keepdim=True), sink))
+        sums[h, :total], maxes[h, :total] = p.sum((0, 1)), p.amax(0).sum(0)
+        for s in range(specs):
+            lost[s, start:total] += p[..., ~held[s, 0, h, :total]].sum((0, 2)) / (64 * len(FULL))
+    # 32-bit probabilities (logits up to about 8: 2^-20) and sums of up to 200 * 8 of them.
+    tol = dict(rtol=1e-5, atol=1e-7)
+    torch.testing.assert_close(entry["score_sum"][0].double(), sums, **tol)
+    torch.testing.assert_close(entry["score_max"][0].double(), maxes, **tol)
+    torch.testing.assert_close(entry["lost"].double(), lost, **tol)
