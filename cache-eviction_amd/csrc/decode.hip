@@ -661,178 +661,209 @@ struct ScoreArgs {
   int64_t kv_ss, kv_sh;
   const int32_t* indptr;
   const void* indices;
-  const float* norm;  // [bs, q_heads], natural log
+  const float* norm;  // [bs, q_heads], natural log; null: from the split log-sum-exps below
   const int32_t* mode;
   const void* rows;
   int rows_dtype;
   float* scores;
   int64_t scores_sg, scores_ss;
-  int kv_heads, q_heads, chunk;
+  int kv_heads, q_heads, bs;
   float scale2;
-};
-
-constexpr int SCORE_MAX_CHUNK = 1024;  // keys per workgroup of decode_score_kernel
-constexpr int SCORE_STEPS = 4;  // 16-key steps of decode_score_kernel whose loads issue together
-
-// Kind 4's fold of kmax[g][key - k0] (keys [k0, k_end), k_end - k0 a multiple of the block):
-// thread t takes keys k0 + t + 512 i; a 64-lane wave covers 64 aligned entries, so a block's
-// maximum is a butterfly over the low `shift` lane bits.
-template <typename IdxT>
-GSE_DEVICE void block_step_reduce(const ScoreArgs& a, const float (*kmax)[SCORE_MAX_CHUNK], const IdxT* idx, int k0,
-                                  int k_end, int shift) {
-  const int lane = threadIdx.x & 63;
-  for (int base = 0; base < k_end - k0; base += blockDim.x) {
-    const int key = base + int(threadIdx.x);
-    // k_end - k0 is a multiple of the block, so a block's lanes are all live or all idle.
-    const bool live = key < k_end - k0;
-    float m = 0.f;
-    if (live)
-      for (int g = 0; g < a.kv_heads; ++g) m = fmaxf(m, kmax[g][key]);
-    for (int o = 1; o < (1 << shift); o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
-    if (live && (lane & ((1 << shift) - 1)) == 0) {
-      const int32_t s = int32_t(idx[k0 + key]);
-      a.scores[uint64_t(uint32_t(s)) * a.scores_ss] += m;
-    }
-  }
-}
-
-// Grid (splits, bs), 512 threads: wave g = KV head g over keys [split*chunk, +chunk) of
-// sequence b (the list's first len - delay entries). Per 16 keys, Sp = Q . K^T ([16 heads x
-// 16 keys], heads 8-15 padding), so a lane holds 4 heads of one key: sum / max over heads is
-// in-lane plus one lane swap.
-// Kind 4 (block counters): each wave leaves its keys' maxima over its query heads in LDS; then
-// per key the maximum over the KV heads and per block the maximum over its keys (lane swaps:
-// blocks of at most 64 entries are aligned lane groups of a wave), added to KV head 0's score
-// of the block's first slot. chunk is a multiple of 64, so no block spans two workgroups.
-template <typename IdxT>
-__global__ __launch_bounds__(512) void decode_score_kernel(ScoreArgs a) {
-  __shared__ float kmax[MAX_KVH][SCORE_MAX_CHUNK];
-  const int b = blockIdx.y;
-  const int lane = threadIdx.x & 63;
-  const int g = threadIdx.x >> 6;
-  const int col = lane & 15;
-  const int grp = lane >> 4;
-  const int64_t row = load_index_dyn(a.rows, a.rows_dtype, b);
-  const int word = a.mode[row];
-  const int md = score_kind(word);
-  if (!scoring_kind(md)) return;
-  const bool blocks = md == GSE_SCORE_KIND_BLOCK_STEP;
-  if (g >= a.kv_heads && !blocks) return;
-  const bool max_mode = md != 1;
-  const int base = a.indptr[b];
-  const int full = a.indptr[b + 1] - base;
-  const int len = blocks ? block_step_limit(full, score_delay(word), score_block_shift(word))
-                         : full - score_delay(word);  // keys the query scores
-  const int k0 = blockIdx.x * a.chunk;
-  const int k_end = k0 + a.chunk < len ? k0 + a.chunk : len;
-  if (k0 >= k_end) return;
-  const IdxT* idx = static_cast<const IdxT*>(a.indices) + base;
-  if (blocks && g >= a.kv_heads) {  // idle wave: only the reduction below
-    __syncthreads();
-    block_step_reduce(a, kmax, idx, k0, k_end, score_block_shift(word));
-    return;
-  }
-
-  // A rows: heads g*8 + col (zero for col >= 8), dims [8*grp, +8) and [32 + 8*grp, +8).
-  bf16x8_t qa0 = {}, qa1 = {};
-  if (col < GROUP) {
-    const uint16_t* qp = a.q + int64_t(b) * a.q_sb + int64_t(g * GROUP + col) * a.q_sh + 8 * grp;
-    qa0 = as_bf16x8(ld16(qp));
-    qa1 = as_bf16x8(ld16(qp + 32));
-  }
-  // Normalisers of this lane's rows (heads 4*grp + r; rows 8-15 padding, probability 0).
-  f32x4_t nrm = {INFINITY, INFINITY, INFINITY, INFINITY};
-  if (grp < 2)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) nrm[r] = a.norm[int64_t(b) * a.q_heads + g * GROUP + 4 * grp + r] * kLog2e;
-
-  const uint16_t* kbase = a.k + int64_t(g) * a.kv_sh + 8 * grp;
-  float* srow = a.scores + int64_t(g) * a.scores_sg;
-  // SCORE_STEPS steps of 16 keys at a time: their slot indices load together, then their K rows
-  // and old scores (a bs = 1 chunk of 64 keys is two round trips, not eight). A list holds each
-  // slot once, so no two keys of a batch share a score.
-  for (int t0 = k0; t0 < k_end; t0 += 16 * SCORE_STEPS) {
-    int32_t sl[SCORE_STEPS];
-#pragma unroll
-    for (int e = 0; e < SCORE_STEPS; ++e) {
-      const int key = t0 + 16 * e + col;
-      sl[e] = int32_t(idx[key < k_end ? key : k_end - 1]);
-    }
-    uint4 kl[SCORE_STEPS], kh[SCORE_STEPS];
-    float old[SCORE_STEPS];
-#pragma unroll
-    for (int e = 0; e < SCORE_STEPS; ++e) {
-      const uint16_t* kp = kbase + uint64_t(uint32_t(sl[e])) * uint64_t(a.kv_ss);
-      kl[e] = ld16(kp);
-      kh[e] = ld16(kp + 32);
-      old[e] = blocks ? 0.f : srow[uint64_t(uint32_t(sl[e])) * a.scores_ss];
-    }
-#pragma unroll
-    for (int e = 0; e < SCORE_STEPS; ++e) {
-      const int key = t0 + 16 * e + col;
-      f32x4_t d = {0.f, 0.f, 0.f, 0.f};
-      d = mfma16x16x32(qa0, as_bf16x8(kl[e]), d);
-      d = mfma16x16x32(qa1, as_bf16x8(kh[e]), d);
-      // Heads 0-3 (group 0) with heads 4-7 (group 1); groups 2, 3 carry padding (exactly 0). The
-      // largest probability is 2^(largest exponent): max mode takes one exponential.
-      float tot;
-      if (max_mode) {
-        const float y = fmaxf(fmaxf(fmaf(d[0], a.scale2, -nrm[0]), fmaf(d[1], a.scale2, -nrm[1])),
-                              fmaxf(fmaf(d[2], a.scale2, -nrm[2]), fmaf(d[3], a.scale2, -nrm[3])));
-        tot = fast_exp2(xor16_max(y));
-      } else {
-        const float u0 = fast_exp2(fmaf(d[0], a.scale2, -nrm[0]));
-        const float u1 = fast_exp2(fmaf(d[1], a.scale2, -nrm[1]));
-        const float u2 = fast_exp2(fmaf(d[2], a.scale2, -nrm[2]));
-        const float u3 = fast_exp2(fmaf(d[3], a.scale2, -nrm[3]));
-        tot = xor16_sum((u0 + u1) + (u2 + u3));
-      }
-      if (blocks) {
-        if (grp == 0 && key < k_end) kmax[g][key - k0] = tot;
-      } else if (grp == 0 && key < k_end) {
-        srow[uint64_t(uint32_t(sl[e])) * a.scores_ss] = old[e] + tot;
-      }
-    }
-  }
-  if (blocks) {
-    __syncthreads();
-    block_step_reduce(a, kmax, idx, k0, k_end, score_block_shift(word));
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Normaliser from an external kernel's split log-sum-exps
-// ---------------------------------------------------------------------------
-struct NormArgs {
+  // An external kernel's split log-sum-exps (R:180-188): split i of sequence b covers keys
+  // [i * per, +per), per = its length over num_splits[b], rounded up to min_kv.
   const float* lse;
   int64_t lse_sb, lse_sh;
   const int32_t* num_splits;
-  const int32_t* indptr;
   const void* sinks;
   int sinks_dtype;
-  float* norm;  // [bs, q_heads]
-  int q_heads, max_kv_splits, min_kv;
+  int max_kv_splits, min_kv;
 };
 
-// R:180-188: the normaliser from SGLang's split log-sum-exps, started at (sink, 1).
-__global__ void norm_from_lse_kernel(NormArgs a) {
-  const int b = blockIdx.x;
-  const int h = threadIdx.x;
-  if (h >= a.q_heads) return;
-  const int64_t len = int64_t(a.indptr[b + 1]) - a.indptr[b];
-  const int64_t splits = a.num_splits[b];
-  const int64_t per = ((len + splits - 1) / splits + a.min_kv - 1) / a.min_kv * a.min_kv;
-  float m = load_float_dyn(a.sinks, a.sinks_dtype, h);
-  float s = 1.f;
-  for (int i = 0; i < a.max_kv_splits; ++i) {
-    if (int64_t(i) * per < len) {
-      const float x = a.lse[int64_t(b) * a.lse_sb + int64_t(h) * a.lse_sh + i];
-      const float n = fmaxf(m, x);
-      s = s * expf(m - n) + expf(x - n);
-      m = n;
+constexpr int SCORE_TILE = 64;  // keys per tile of decode_score_kernel: blocks of kind 4 lie within one
+// Workgroups per CU: the two that fit at its registers (8 waves of 92). More of them wait for a
+// second round: 29.0 us at 2, 31.9 at 4, 37.4 at 8 (8 lists, 115 MB), and 4 per CU in 64 registers
+// 45.5 us.
+constexpr int SCORE_WG_PER_CU = 2;
+
+// Normaliser (natural log, sink included) of the wave's heads g*8 + lane/8 of sequence b, whose
+// list holds len keys, from its split log-sum-exps: eight lanes per head.
+GSE_DEVICE float norm_from_lse(const ScoreArgs& a, int b, int g, int len) {
+  const int lane = threadIdx.x & 63;
+  const int h = g * GROUP + (lane >> 3);
+  const int splits = a.num_splits[b];
+  const int64_t per = ((int64_t(len) + splits - 1) / splits + a.min_kv - 1) / a.min_kv * a.min_kv;
+  const float* lse = a.lse + int64_t(b) * a.lse_sb + int64_t(h) * a.lse_sh;
+  const float sink = load_float_dyn(a.sinks, a.sinks_dtype, h);
+  auto at = [&](int i) { return i < a.max_kv_splits && i * per < len ? lse[i] : -INFINITY; };
+  const float x0 = at(lane & 7), x1 = at((lane & 7) + 8);
+  float m = fmaxf(sink, fmaxf(x0, x1));
+  for (int i = (lane & 7) + 16; i < a.max_kv_splits; i += 8) m = fmaxf(m, at(i));
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) m = wave_max_xor(m, o);
+  float s = expf(x0 - m) + expf(x1 - m);
+  for (int i = (lane & 7) + 16; i < a.max_kv_splits; i += 8) s += expf(at(i) - m);
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) s = wave_sum_xor(s, o);
+  return m + logf(s + expf(sink - m));
+}
+
+// Grid of P workgroups of 512 threads: the batch's lists, cut into 64-key tiles, are one range of
+// tiles; workgroup w takes the w-th P-th of it (equal shares whatever the lengths; the host knows
+// only an upper bound of them). Wave g = KV head g: per 16 keys, Sp = Q . K^T ([16 heads x 16 keys],
+// heads 8-15 padding), so a lane holds 4 heads of one key: sum / max over heads is in-lane plus one
+// lane swap. The waves' totals of a tile meet in LDS and thread (key, head) adds one to the score
+// table: a key's heads are one 32-byte row there, read and written once instead of once per wave.
+// Kind 4 (block counters): per key the maximum over the KV heads and per block the maximum over its
+// keys (lane swaps: blocks of at most 64 entries are aligned lane groups of a wave), added to KV
+// head 0's score of the block's first slot.
+// Bound by HBM; 8 lists of 4 to 18 thousand keys (115 MB), with the clearing of the new slots: 46.9
+// us (a kernel of its own for the normalisers, workgroups sized by the batch's longest possible
+// list, a wave's share of a score row at a time) -> 29.0 us; 32 lists, 1.1 GB: 376 -> 235 us.
+template <typename IdxT>
+__global__ __launch_bounds__(512) void decode_score_kernel(ScoreArgs a) {
+  __shared__ float totals[2][SCORE_TILE][MAX_KVH + 1];
+  const int lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15;
+  const int grp = lane >> 4;
+  const bool live_wave = g < a.kv_heads;
+  auto tiles_of = [&](int b) { return (a.indptr[b + 1] - a.indptr[b] + SCORE_TILE - 1) / SCORE_TILE; };
+  // The batch's tiles (64 sequences at a time, a scan over the lanes), then this workgroup's first
+  // sequence and the tiles before it.
+  int tiles = 0;
+  for (int b0 = 0; b0 < a.bs; b0 += kWave) {
+    int n = b0 + lane < a.bs ? tiles_of(b0 + lane) : 0;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) n += __shfl_xor(n, o, kWave);
+    tiles += n;
+  }
+  int t = int(int64_t(tiles) * blockIdx.x / gridDim.x);
+  const int t_end = int(int64_t(tiles) * (blockIdx.x + 1) / gridDim.x);
+  if (t >= t_end) return;
+  int b = 0, before = 0;  // sequence b's first tile is `before`
+  for (int b0 = 0;; b0 += kWave) {
+    const int n = b0 + lane < a.bs ? tiles_of(b0 + lane) : 0;
+    int upto = n;  // tiles of the sequences b0 .. b0 + lane
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int below = __shfl_up(upto, o, kWave);
+      if (lane >= o) upto += below;
+    }
+    const uint64_t past = __builtin_amdgcn_ballot_w64(before + upto > t);
+    if (past) {  // t < tiles: some chunk of 64 sequences holds it
+      const int l = __builtin_ctzll(past);
+      b = b0 + l;
+      before += __shfl(upto - n, l, kWave);
+      break;
+    }
+    before += __shfl(upto, kWave - 1, kWave);
+  }
+  b = __builtin_amdgcn_readfirstlane(b);
+  before = __builtin_amdgcn_readfirstlane(before);
+
+  int parity = 0;
+  for (; t < t_end; ++b) {
+    const int n = tiles_of(b);
+    const int t1 = min(t_end, before + n);  // this workgroup's tiles of sequence b: [t, t1)
+    const int64_t row = load_index_dyn(a.rows, a.rows_dtype, b);
+    const int word = a.mode[row];
+    const int md = score_kind(word);
+    const int base = a.indptr[b];
+    const int full = a.indptr[b + 1] - base;
+    const bool blocks = md == GSE_SCORE_KIND_BLOCK_STEP;
+    // Keys the query scores.
+    const int len = !scoring_kind(md) ? 0
+                    : blocks          ? block_step_limit(full, score_delay(word), score_block_shift(word))
+                                      : full - score_delay(word);
+    const int first = (t - before) * SCORE_TILE;
+    const int last = min((t1 - before) * SCORE_TILE, len);  // this workgroup's keys: [first, last)
+    t = t1;
+    before += n;
+    if (first >= last) continue;
+    const bool max_mode = md != 1;
+    const IdxT* idx = static_cast<const IdxT*>(a.indices) + base;
+
+    // A rows: heads g*8 + col (zero for col >= 8), dims [8*grp, +8) and [32 + 8*grp, +8).
+    bf16x8_t qa0 = {}, qa1 = {};
+    if (live_wave && col < GROUP) {
+      const uint16_t* qp = a.q + int64_t(b) * a.q_sb + int64_t(g * GROUP + col) * a.q_sh + 8 * grp;
+      qa0 = as_bf16x8(ld16(qp));
+      qa1 = as_bf16x8(ld16(qp + 32));
+    }
+    // Normalisers of this lane's rows (heads 4*grp + r; rows 8-15 padding, probability 0).
+    f32x4_t nrm = {INFINITY, INFINITY, INFINITY, INFINITY};
+    if (live_wave && a.lse) {
+      const float own = norm_from_lse(a, b, g, full) * kLog2e;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = __shfl(own, 8 * ((4 * grp + r) & 7), kWave);
+        if (grp < 2) nrm[r] = x;
+      }
+    } else if (live_wave && grp < 2) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) nrm[r] = a.norm[int64_t(b) * a.q_heads + g * GROUP + 4 * grp + r] * kLog2e;
+    }
+    const uint16_t* kbase = a.k + int64_t(live_wave ? g : 0) * a.kv_sh + 8 * grp;
+
+    for (int t0 = first; t0 < last; t0 += SCORE_TILE, parity ^= 1) {
+      // The tile's slot indices load together, then its K rows and old scores. A list holds each
+      // slot once, so no two keys share a score.
+      int32_t sl[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sl[e] = int32_t(idx[min(t0 + 16 * e + col, last - 1)]);
+      const int mine = threadIdx.x >> 3, h = threadIdx.x & 7;  // this thread's (key, KV head) of the tile
+      const uint64_t my_slot = uint32_t(int32_t(idx[min(t0 + mine, last - 1)]));
+      uint4 kl[4], kh[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint16_t* kp = kbase + uint64_t(uint32_t(sl[e])) * uint64_t(a.kv_ss);
+        kl[e] = ld16(kp);
+        kh[e] = ld16(kp + 32);
+      }
+      const bool adds = !blocks && h < a.kv_heads && t0 + mine < last;
+      float* mp = a.scores + int64_t(h) * a.scores_sg + my_slot * a.scores_ss;
+      const float old = adds ? *mp : 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+        d = mfma16x16x32(qa0, as_bf16x8(kl[e]), d);
+        d = mfma16x16x32(qa1, as_bf16x8(kh[e]), d);
+        // Heads 0-3 (group 0) with heads 4-7 (group 1); groups 2, 3 carry padding (exactly 0). The
+        // largest probability is 2^(largest exponent): max mode takes one exponential.
+        float tot;
+        if (max_mode) {
+          const float y = fmaxf(fmaxf(fmaf(d[0], a.scale2, -nrm[0]), fmaf(d[1], a.scale2, -nrm[1])),
+                                fmaxf(fmaf(d[2], a.scale2, -nrm[2]), fmaf(d[3], a.scale2, -nrm[3])));
+          tot = fast_exp2(xor16_max(y));
+        } else {
+          const float u0 = fast_exp2(fmaf(d[0], a.scale2, -nrm[0]));
+          const float u1 = fast_exp2(fmaf(d[1], a.scale2, -nrm[1]));
+          const float u2 = fast_exp2(fmaf(d[2], a.scale2, -nrm[2]));
+          const float u3 = fast_exp2(fmaf(d[3], a.scale2, -nrm[3]));
+          tot = xor16_sum((u0 + u1) + (u2 + u3));
+        }
+        if (live_wave && grp == 0) totals[parity][16 * e + col][g] = tot;
+      }
+      // Two buffers: a wave writes this one again only past the next tile's barrier, which every
+      // thread reaches after its reads here.
+      __syncthreads();
+      if (blocks) {
+        if (g == 0) {
+          const int shift = score_block_shift(word);
+          // last - t0 is a multiple of the block, so a block's lanes are all live or all idle.
+          const bool live = t0 + lane < last;
+          float m = 0.f;
+          if (live)
+            for (int k = 0; k < a.kv_heads; ++k) m = fmaxf(m, totals[parity][lane][k]);
+          for (int o = 1; o < (1 << shift); o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
+          if (live && (lane & ((1 << shift) - 1)) == 0)
+            a.scores[uint64_t(uint32_t(int32_t(idx[t0 + lane]))) * a.scores_ss] += m;
+        }
+      } else if (adds) {
+        *mp = old + totals[parity][mine][h];
+      }
     }
   }
-  a.norm[int64_t(b) * a.q_heads + h] = m + logf(s);
 }
 
 // gse_decode_noalloc's partials and normalisers: one copy per GPU, held until the process ends.
@@ -864,17 +895,12 @@ int check_decode_shape(int q_heads, int kv_heads, int head_dim) {
   return GSE_OK;
 }
 
-// One score-only pass over K; max_len bounds every sequence's length. A workgroup walks its
-// chunk 16 keys per dependent step, so the chunk (64..1024 keys) is sized to give about four
-// workgroups per CU over the batch.
-int score_pass(ScoreArgs s, int indices_dtype, int bs, int max_len, hipStream_t stream) {
-  const int64_t target = 4 * int64_t(fused_workgroups());
-  int64_t chunk = (int64_t(max_len) * bs + target - 1) / target;
-  chunk = (chunk + 63) / 64 * 64;
-  s.chunk = int(chunk < 64 ? 64 : (chunk > 1024 ? 1024 : chunk));
-  const int splits = (max_len + s.chunk - 1) / s.chunk;
-  if (splits <= 0 || bs <= 0) return GSE_OK;
-  const dim3 grid{static_cast<uint32_t>(splits), static_cast<uint32_t>(bs)}, block{FUSED_THREADS};
+// One score-only pass over K; max_len bounds every sequence's length.
+int score_pass(const ScoreArgs& s, int indices_dtype, int max_len, hipStream_t stream) {
+  const int64_t tiles = int64_t(s.bs) * ((int64_t(std::max(max_len, 0)) + SCORE_TILE - 1) / SCORE_TILE);
+  if (tiles <= 0) return GSE_OK;
+  const int64_t blocks = std::min(tiles, SCORE_WG_PER_CU * int64_t(fused_workgroups()));
+  const dim3 grid{static_cast<uint32_t>(blocks)}, block{FUSED_THREADS};
   if (indices_dtype == GSE_I64)
     hipLaunchKernelGGL(decode_score_kernel<int64_t>, grid, block, 0, stream, s);
   else
@@ -1066,9 +1092,9 @@ int decode_run(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void
   if (score_mode == GSE_SCORE_EAGER) {
     // This step's scores need its final normaliser: a second, score-only pass over K.
     ScoreArgs sa = {f.q, q_stride_b, q_stride_h, f.k, kv_stride_s, kv_stride_h, kv_indptr, kv_indices, norm,
-                    mode_by_row, rows, rows_dtype, scores, scores_stride_g, scores_stride_s, kv_heads, q_heads, 0,
+                    mode_by_row, rows, rows_dtype, scores, scores_stride_g, scores_stride_s, kv_heads, q_heads, bs,
                     sm_scale * kLog2e};
-    if ((rc = score_pass(sa, indices_dtype, bs, max_len, s))) return rc;
+    if ((rc = score_pass(sa, indices_dtype, max_len, s))) return rc;
   }
   return GSE_OK;
 }
@@ -1175,13 +1201,10 @@ extern "C" int gse_decode_scores_from_lse(const void* q, int64_t q_stride_b, int
   if ((q_stride_h % 8) || (q_stride_b % 8) || (kv_stride_s % 8) || (kv_stride_h % 8))
     return gse_fail(GSE_EINVAL, "scores_from_lse: strides must be multiples of 8 elements");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  float* norm = static_cast<float*>(workspace);
-  NormArgs n = {attn_lse, lse_stride_b, lse_stride_h, num_kv_splits, kv_indptr, sinks, sinks_dtype,
-                norm, q_heads, max_kv_splits, min_block_kv};
-  hipLaunchKernelGGL(norm_from_lse_kernel, dim3(bs), dim3(64), 0, s, n);
-  if (int rc = gse_launch_check("norm_from_lse")) return rc;
+  // The pass forms each sequence's normaliser itself.
   ScoreArgs sa = {static_cast<const uint16_t*>(q), q_stride_b, q_stride_h, static_cast<const uint16_t*>(k_pool),
-                  kv_stride_s, kv_stride_h, kv_indptr, kv_indices, norm, mode_by_row, rows, rows_dtype, scores,
-                  scores_stride_g, scores_stride_s, kv_heads, q_heads, 0, sm_scale * kLog2e};
-  return score_pass(sa, indices_dtype, bs, max_len, s);
+                  kv_stride_s, kv_stride_h, kv_indptr, kv_indices, nullptr, mode_by_row, rows, rows_dtype, scores,
+                  scores_stride_g, scores_stride_s, kv_heads, q_heads, bs, sm_scale * kLog2e, attn_lse, lse_stride_b,
+                  lse_stride_h, num_kv_splits, sinks, sinks_dtype, max_kv_splits, min_block_kv};
+  return score_pass(sa, indices_dtype, max_len, s);
 }

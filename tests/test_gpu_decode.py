@@ -78,6 +78,7 @@ def _decode_setup(lengths, seed=0, slots=20000):
     bs = len(lengths)
     q = torch.randn((bs, heads, dim), generator=g).to(torch.bfloat16).cuda()
     sinks = torch.randn(heads, generator=g).to(torch.bfloat16).cuda()
+    assert sum(lengths) < slots
     perm = (torch.randperm(slots - 1, generator=g)[:sum(lengths)] + 1).cuda()
     indptr = torch.tensor(np.concatenate(([0], np.cumsum(lengths))), dtype=torch.int32, device="cuda")
     rows = torch.arange(1, bs + 1, device="cuda")
@@ -309,6 +310,42 @@ def test_after_decode_rebuilds_normaliser_from_split_lse(mode, delay):
                              len(rows_keys) - 1, delay)
     torch.testing.assert_close(st.scores[0].cpu(), torch.tensor(expected, dtype=torch.float32), rtol=2e-3, atol=1e-6)
     assert float(st.scores[1:].abs().sum()) == 0.0
+
+
+# The pass cuts all lists into one range of 64-key tiles: lists that are empty, end on a tile's edge
+# or one past it, more than the 64 lists of one scan, unscored rows between, and split counts past
+# the 16 the first loads cover.
+@pytest.mark.parametrize("lengths,splits", [([1], 1), ([64], 2), ([65, 0, 63], 8), ([0, 0, 5000, 0, 1], 17),
+                                            ([130, 64, 0, 1, 65, 300] * 23 + [129], 40)])
+def test_after_decode_over_many_lists(lengths, splits):
+    bs = len(lengths)
+    b, st, q, sinks, perm, indptr, rows = _decode_setup(lengths, seed=bs + splits)
+    b.max_kv_splits = splits
+    kinds = [1, 2, 0]
+    st.mode[:] = 0
+    st.mode[rows.long()] = torch.tensor([kinds[i % 3] for i in range(bs)], dtype=torch.int32, device="cuda")
+    keys = b.token_to_kv_pool.get_key_buffer(1)
+    lse = torch.full((bs, 64, splits), 1e30, device="cuda")  # splits past a list's end are never read
+    want = torch.zeros(tuple(st.scores.shape[1:]), dtype=torch.float64, device="cuda")
+    for i, n in enumerate(lengths):
+        if not n:
+            continue
+        slots = perm[indptr[i]:indptr[i + 1]].long()
+        per = -(-(-(-n // splits)) // 32) * 32
+        x = torch.matmul(q[i].double().view(8, 8, 64), keys[slots].double().permute(1, 2, 0).contiguous()) * 0.125
+        for s in range(-(-n // per)):
+            lse[i, :, s] = torch.logsumexp(x[..., s * per:(s + 1) * per], -1).reshape(64).float()
+        norm = torch.logaddexp(torch.logsumexp(x, -1), sinks.double().view(8, 8))
+        p = torch.exp(x - norm[..., None])
+        if kinds[i % 3]:
+            want[:, slots] += p.sum(1) if kinds[i % 3] == 1 else p.amax(1)
+    b.forward_metadata = SimpleNamespace(attn_lse=lse, kv_indptr=indptr, kv_indices=perm, num_kv_splits=torch.full(
+        (bs,), splits, dtype=torch.int32, device="cuda"))
+    ge.after_decode(b, q.reshape(bs, -1), layer(1), SimpleNamespace(
+        out_cache_loc=torch.zeros(bs, dtype=torch.int64, device="cuda"), req_pool_indices=rows,
+        seq_lens_cpu=torch.tensor(lengths)), sinks)
+    # 32-bit logits and log-sum-exps of magnitude up to about 16: 2^-20 each.
+    torch.testing.assert_close(st.scores[0].double(), want, rtol=1e-5, atol=1e-8)
 
 
 def test_rows_without_a_policy_get_no_scores_and_sliding_layers_are_skipped():
