@@ -603,228 +603,219 @@ __global__ __launch_bounds__(p2::THREADS, 4) void prefill_score_kernel(PrefillAr
 // ---------------------------------------------------------------------------
 // Block counters of a chunk (score kind 4)
 // ---------------------------------------------------------------------------
-// The second pass for score kind 4 (TEX:197's block counters; no reference code). A
-// workgroup owns 16 queries and every KV head: wave g = KV head g, its MFMA rows (query,
-// head of g) as in pass 2, 8 row-blocks of 2 queries. Per 64-key tile the wave loads K_g of
-// the tile's keys straight into registers (the next tile's loads in flight during this one),
-// turns D = Q . K_g^T into probabilities with pass 1's normalisers and folds each (query,
-// key)'s maximum over g's heads into qk[query][key] in LDS with an unsigned max
-// (probabilities are non-negative, so their bit patterns order as the values do). At the
-// start of the next tile each wave reduces two queries of that tile: per (query, block) the
-// maximum over the block's keys (a butterfly over the low lanes: blocks of at most 64 aligned
-// keys lie in one wave), added to the block's credit in an LDS ring; the ring's credits go to
-// the block counters (KV head 0's score of a block's first slot) with one atomic per block and
-// workgroup. qk alternates between two buffers by tile parity, so a tile needs one barrier.
-// Query i credits the whole blocks of keys < prefix_len + i + 1 - delay. The maximum over heads
-// is taken over the exponents (one exponential per (query, key)); the tiles that every query
-// credits whole run in a loop of their own, without limit checks and with the next row-block's
-// MFMAs interleaved with this one's vector work.
+// The second pass for score kind 4 (TEX:197's block counters; no reference code). A workgroup owns 64
+// queries (8 per wave, 4 row blocks of (query, head) pairs) and a range of 256-key tiles. Per tile it
+// walks the KV heads: K_g of the tile's keys goes through LDS (the next head's rows in flight), the
+// wave's queries of that head come into registers a head ahead, and D = Q . K_g^T with pass 1's
+// normalisers raises a running maximum of the log2 probability per (query, key) and lane. After the
+// last head the lane's two head halves meet, then a block's keys (a butterfly over the low lane bits:
+// blocks of at most 64 aligned entries lie in a 64-key group), and only then, 2^x increasing with x,
+// one exponential per (query, block). Query i credits the whole blocks of keys < prefix_len + i + 1 -
+// delay: every other maximum is dropped there, so the heads' walk needs no mask. The waves' credits
+// meet in LDS and one thread per key adds them to the block's counter (KV head 0's score of its first
+// slot).
+// Bound by the matrix units beside vector issue: per 1024 logits 8 MFMAs (132 cycles), 16 FMAs and 8
+// three-way maxima. 2048 queries after 12,288 keys, blocks of 4: 630 us with a wave per KV head and
+// an LDS atomic maximum per lane and 16x16 block, 414 with plain LDS maxima and a barrier per 64
+// keys, 314 us so (2.1 GHz: the power limit).
 namespace pb {
-constexpr int QB = 16;          // queries per workgroup
-constexpr int RB = QB / 2;      // row-blocks per wave
-constexpr int WAVES = 8;        // wave g = KV head g
+constexpr int QB = pf::QB;      // queries per workgroup
+constexpr int QW = 8;           // queries per wave
+constexpr int WAVES = QB / QW;
 constexpr int THREADS = 64 * WAVES;
-constexpr int KT = 64;          // keys per tile
-constexpr int RING = 16;        // tiles of block credits held in LDS before they go to the scores
-constexpr int VALU_PER_MFMA = 3;  // vector instructions issued behind each MFMA in common tiles
+constexpr int KT = 256;         // keys per tile
+constexpr int KB = KT / 16;     // its 16-key blocks
+constexpr int MAX_HEADS = 64;   // query heads
+// Work items of a launch: some eight rounds of the one workgroup a CU holds.
+constexpr int ITEMS = 2048;
 }  // namespace pb
 
+GSE_DEVICE float vmax3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+// x of the lower and y of the upper lanes (by lane bit 5, resp. 4), each summed over that bit.
+GSE_DEVICE float join32(float x, float y) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+GSE_DEVICE float join16(float x, float y) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 template <typename IdxT>
-__global__ __launch_bounds__(pb::THREADS) void prefill_block_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(pb::THREADS, 2) void prefill_block_kernel(PrefillArgs a) {
   using namespace pb;
-  __shared__ uint32_t qk[2][QB][KT];
-  __shared__ float ring[RING][KT];  // block credits of RING tiles, added to the scores once per ring
+  using pf::KROW;
+  __shared__ __attribute__((aligned(16))) uint16_t ktile[2][KT * KROW];
+  // Negated normalisers of the workgroup's queries (-inf past the chunk), rows padded by 16 bytes.
+  __shared__ __attribute__((aligned(16))) float norms[QB][MAX_HEADS + 4];
+  __shared__ float cols[WAVES][KT];
   const int lane = threadIdx.x & 63;
-  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int col = lane & 15, grp = lane >> 4;
-  const int shift = a.block_shift;
+  const int shift = a.block_shift, block = 1 << shift;
   const IdxT* slots = static_cast<const IdxT*>(a.slots);
-  // Heaviest query blocks (longest causal range) first.
-  const int64_t nqb = (a.count + QB - 1) / QB;
-  const int64_t qb0 = (nqb - 1 - int64_t(blockIdx.x)) * QB;
-  const int64_t last_q = (qb0 + QB < a.count ? qb0 + QB : a.count) - 1;
-  auto limit = [&](int64_t i) {  // credited keys of query i
-    return i < a.count ? block_step_limit(int(a.prefix_len + i + 1), a.delay, shift) : 0;
+  const int count = int(a.count), heads = a.kv_heads;
+  // Block i: the query block from the end (the longest causal ranges first), then the key range.
+  const int nqb = (count + QB - 1) / QB;
+  const int split = blockIdx.x / nqb;
+  const int qb0 = (nqb - 1 - blockIdx.x % nqb) * QB;
+  auto limit = [&](int i) {  // credited keys of query i
+    return i < count ? block_step_limit(int(a.prefix_len) + i + 1, a.delay, shift) : 0;
   };
-  const int kend = limit(last_q);
-  if (kend <= 0) return;
-  for (int t = threadIdx.x; t < 2 * QB * KT; t += blockDim.x) (&qk[0][0][0])[t] = 0u;
-  for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) ring[t / KT][t % KT] = 0.f;
-  const bool live_wave = g < a.kv_heads;
-
-  // A fragments: row col of row-block rb is query qb0 + 2*rb + col/8, head g*8 + col%8, dims
-  // [8*grp, +8) and [32 + 8*grp, +8). This lane's D rows: query qb0 + 2*rb + grp/2, heads
-  // g*8 + 4*(grp%2) + r, with their normalisers (log2 units; +inf past the chunk) and limits.
-  bf16x8_t qa[RB][2];
-  f32x4_t nrm[RB];
-  int lim[RB];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    qa[rb][0] = bf16x8_t{};
-    qa[rb][1] = bf16x8_t{};
-    const int64_t qi = qb0 + 2 * rb + (col >> 3);
-    if (live_wave && qi < a.count) {
-      const uint16_t* qp = a.q + qi * a.q_st + int64_t(g * pf::GROUP + (col & 7)) * a.q_sh + 8 * grp;
-      qa[rb][0] = as_bf16x8(*reinterpret_cast<const uint4*>(qp));
-      qa[rb][1] = as_bf16x8(*reinterpret_cast<const uint4*>(qp + 32));
-    }
-    const int64_t qd = qb0 + 2 * rb + (grp >> 1);
-    lim[rb] = limit(qd);
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      nrm[rb][r] = live_wave && qd < a.count ? a.norm2[qd * a.q_heads + g * pf::GROUP + 4 * (grp & 1) + r] : INFINITY;
-  }
-  // The K rows of tile i + 1 are in flight while tile i computes, and their slot indices were
-  // read a tile before that, so a tile's K loads go out together and its compute waits on
-  // nothing issued during it. The two register sets alternate between tiles.
-  const auto kbase = as_global(a.k) + int64_t(live_wave ? g : 0) * a.kv_sh + 8 * grp;
-  // The indices stay as loaded until the next tile turns them into addresses (using them at
-  // once would make the compiler wait for every load in flight, K included).
-  auto load_idx = [&](int t0, IdxT (&s)[4]) {
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      const int key = t0 + 16 * st + col;
-      s[st] = slots[key < kend ? key : kend - 1];
-    }
-  };
-  auto load_k = [&](const IdxT (&s)[4], uint4 (&kf)[4][2]) {
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      const auto p = kbase + int64_t(s[st]) * a.kv_ss;
-      kf[st][0] = gload16(p);
-      kf[st][1] = gload16(p + 32);
-    }
-  };
+  const int kend = limit(min(qb0 + QB, count) - 1);
   const int ntiles = (kend + KT - 1) / KT;
-  uint4 ka[4][2], kb[4][2];
-  IdxT sidx[4];
-  load_idx(0, sidx);
-  if (live_wave) load_k(sidx, ka);
-  if (ntiles > 1) load_idx(KT, sidx);
-  __syncthreads();  // qk and the ring cleared
+  const int ranges = key_ranges(ntiles, a.tiles);
+  if (split >= ranges) return;
+  const int ti0 = int(int64_t(ntiles) * split / ranges), ti1 = int(int64_t(ntiles) * (split + 1) / ranges);
+  const int i0 = qb0 + QW * wave;
+  const bool live = i0 < count;
+  int lim[4];  // of this lane's D rows: query i0 + 2*rb + grp/2, heads 4*(grp%2) + r
+#pragma unroll
+  for (int rb = 0; rb < 4; ++rb) lim[rb] = limit(i0 + 2 * rb + (grp >> 1));
 
-  // Tile ti's maxima to the ring: wave w takes queries w and w + 8, lane = key.
-  auto reduce = [&](int ti) {
-    const int key = threadIdx.x & (KT - 1), q8 = threadIdx.x >> 6;
-    uint32_t(&m)[QB][KT] = qk[ti & 1];
-    float v0 = __uint_as_float(m[q8][key]), v1 = __uint_as_float(m[q8 + 8][key]);
-    m[q8][key] = 0u;
-    m[q8 + 8][key] = 0u;
-    for (int o = 1; o < (1 << shift); o <<= 1) {
-      v0 = fmaxf(v0, __shfl_xor(v0, o, kWave));
-      v1 = fmaxf(v1, __shfl_xor(v1, o, kWave));
+  // A fragments of head g: row col of block rb is query i0 + 2*rb + col/8, head g*8 + col%8.
+  auto load_q = [&](int g, uint4 (&q)[4][2]) {
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) {
+      const int qi = min(i0 + 2 * rb + (col >> 3), count - 1);  // past the chunk: any row, its normaliser is +inf
+      const auto qp = as_global(a.q) + qi * a.q_st + int64_t(g * pf::GROUP + (col & 7)) * a.q_sh + 8 * grp;
+      q[rb][0] = gload16(qp);
+      q[rb][1] = gload16(qp + 32);
     }
-    if ((key & ((1 << shift) - 1)) == 0 && v0 + v1 > 0.f) atomicAdd(&ring[ti % RING][key], v0 + v1);
   };
-  // Per row-block, the last key either of its queries credits (uniform).
-  int rb_lim[RB];
+  // Thread t stages 16 bytes of keys t/8 + 64*j. A tile's slots are read a tile ahead.
+  const int lk = threadIdx.x >> 3, lp = threadIdx.x & 7;
+  auto load_slots = [&](int ti, IdxT (&sl)[4]) {
 #pragma unroll
-  for (int rb = 0; rb < RB; ++rb) {
-    const int l0 = limit(qb0 + 2 * rb), l1 = limit(qb0 + 2 * rb + 1);
-    rb_lim[rb] = l0 > l1 ? l0 : l1;
+    for (int j = 0; j < 4; ++j) sl[j] = slots[min(ti * KT + 64 * j + lk, kend - 1)];
+  };
+  const auto kbase = as_global(a.k) + 8 * lp;
+  auto load_k = [&](int g, const IdxT (&sl)[4], uint4 (&x)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = gload16(kbase + int64_t(sl[j]) * a.kv_ss + int64_t(g) * a.kv_sh);
+  };
+  auto store_k = [&](int p, const uint4 (&x)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(&ktile[p][(lk + 64 * j) * KROW + 8 * lp]) = x[j];
+  };
+  IdxT sl[4], sn[4];
+  uint4 qf[4][2];
+  {
+    uint4 x[4];
+    load_slots(ti0, sl);
+    load_q(0, qf);
+    for (int t = threadIdx.x; t < QB * heads * pf::GROUP; t += THREADS) {
+      const int i = t / (heads * pf::GROUP), h = t % (heads * pf::GROUP);
+      norms[i][h] = qb0 + i < count ? -a.norm2[int64_t(qb0 + i) * a.q_heads + h] : -INFINITY;
+    }
+    load_k(0, sl, x);
+    store_k(0, x);
   }
-  // COMMON: a tile below the first query's limit, which every query of the workgroup credits
-  // whole (limits grow with the query), so no row-block or key needs its limit checked.
-  auto tile = [&](int ti, const uint4 (&cur)[4][2], uint4 (&nxt)[4][2], auto common) {
-    constexpr bool COMMON = decltype(common)::value;
-    const int t0 = ti * KT;
-    if (ti % RING != 0) reduce(ti - 1);  // a ring's last tile is reduced before its flush
-    if (live_wave) {
+  __syncthreads();
+
+  int p = 0;
+#pragma unroll 1
+  for (int ti = ti0; ti < ti1; ++ti) {
+    load_slots(ti + 1, sn);
+    float y[4][KB];  // the lane's maximum over its heads of query i0 + 2*rb + grp/2, key 16*kb + col
 #pragma unroll
-      for (int st = 0; st < 4; ++st) {
-        landed(cur[st][0]);
-        landed(cur[st][1]);
-      }
-      if (ti + 1 < ntiles) {
-        load_k(sidx, nxt);
-        if (ti + 2 < ntiles) load_idx(t0 + 2 * KT, sidx);
-      }
-      // The largest of the heads' probabilities is 2^(largest exponent): one exponential per
-      // lane instead of one per head. The two lanes of a (query, key) (heads 0-3 and 4-7) both
-      // fold their maximum into the same LDS cell, so the atomic takes the maximum over all 8.
-      auto credit = [&](const f32x4_t& d, int rb, int st, bool live) {
-        const float y0 = fmaf(d[0], a.scale2, -nrm[rb][0]);
-        const float y1 = fmaf(d[1], a.scale2, -nrm[rb][1]);
-        const float y2 = fmaf(d[2], a.scale2, -nrm[rb][2]);
-        const float y3 = fmaf(d[3], a.scale2, -nrm[rb][3]);
-        const float mx = fast_exp2(fmaxf(fmaxf(y0, y1), fmaxf(y2, y3)));
-        if (live) atomicMax(&qk[ti & 1][2 * rb + (grp >> 1)][16 * st + col], __float_as_uint(mx));
-      };
-      if constexpr (COMMON) {
-        // Row-block rb + 1's MFMAs are issued between rb's vector instructions (one MFMA, then
-        // VALU_PER_MFMA vector instructions): a SIMD overlaps an MFMA only with the independent
-        // vector work its own wave issues behind it.
-        f32x4_t dn[4];
+    for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          dn[st] = mfma16x16x32(qa[0][0], as_bf16x8(cur[st][0]), f32x4_t{0.f, 0.f, 0.f, 0.f});
-          dn[st] = mfma16x16x32(qa[0][1], as_bf16x8(cur[st][1]), dn[st]);
+      for (int kb = 0; kb < KB; ++kb) y[rb][kb] = -INFINITY;
+#pragma unroll 1
+    for (int g = 0; g < heads; ++g, p ^= 1) {
+      // The next head's rows and queries (the first of the next tile's after the last) go out.
+      const bool wrap = g + 1 == heads, more = !wrap || ti + 1 < ti1;
+      uint4 xn[4], qn[4][2];
+      if (wrap)
+        load_k(0, sn, xn);
+      else
+        load_k(g + 1, sl, xn);
+      load_q(wrap ? 0 : g + 1, qn);
+      if (live) {
+        bf16x8_t qa[4][2];
+        f32x4_t nn[4];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+          qa[rb][0] = as_bf16x8(qf[rb][0]);
+          qa[rb][1] = as_bf16x8(qf[rb][1]);
+          nn[rb] = *reinterpret_cast<const f32x4_t*>(&norms[QW * wave + 2 * rb + (grp >> 1)][g * pf::GROUP + 4 * (grp & 1)]);
         }
+        bf16x8_t kf[2][2];  // alternate by key block
+        fragments(ktile[p], 0, lane, kf[0]);
+        f32x4_t dn[2] = {dot64(qa[0], kf[0]), dot64(qa[1], kf[0])};
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          f32x4_t d[4];
-#pragma unroll
-          for (int st = 0; st < 4; ++st) d[st] = dn[st];
-          if (rb + 1 < RB) {
-#pragma unroll
-            for (int st = 0; st < 4; ++st) {
-              dn[st] = mfma16x16x32(qa[rb + 1][0], as_bf16x8(cur[st][0]), f32x4_t{0.f, 0.f, 0.f, 0.f});
-              dn[st] = mfma16x16x32(qa[rb + 1][1], as_bf16x8(cur[st][1]), dn[st]);
-            }
+        for (int u = 0; u < 2 * KB; ++u) {  // units of two row blocks against a key block
+          const int kb = u >> 1, rb = 2 * (u & 1), nkb = (u + 1) >> 1, nrb = 2 * ((u + 1) & 1);
+          const f32x4_t d[2] = {dn[0], dn[1]};
+          if ((u & 1) == 0 && kb + 1 < KB) fragments(ktile[p], kb + 1, lane, kf[(kb + 1) & 1]);
+          if (u + 1 < 2 * KB) {  // the next unit's MFMAs ahead of this one's vector work
+            dn[0] = dot64(qa[nrb], kf[nkb & 1]);
+            dn[1] = dot64(qa[nrb + 1], kf[nkb & 1]);
           }
 #pragma unroll
-          for (int st = 0; st < 4; ++st) credit(d[st], rb, st, true);
-          if (rb + 1 < RB) {
+          for (int j = 0; j < 2; ++j) {
+            float x[4];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-              __builtin_amdgcn_sched_group_barrier(0x002, VALU_PER_MFMA, 0);
-            }
+            for (int r = 0; r < 4; ++r) x[r] = fmaf(d[j][r], a.scale2, nn[rb + j][r]);
+            y[rb + j][kb] = vmax3(vmax3(y[rb + j][kb], x[0], x[1]), x[2], x[3]);
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-      } else {
+      }
+      if (more) {
+        store_k(p ^ 1, xn);
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-          if (rb_lim[rb] <= t0) continue;  // neither query credits this tile
-#pragma unroll
-          for (int st = 0; st < 4; ++st) {
-            f32x4_t d = mfma16x16x32(qa[rb][0], as_bf16x8(cur[st][0]), f32x4_t{0.f, 0.f, 0.f, 0.f});
-            d = mfma16x16x32(qa[rb][1], as_bf16x8(cur[st][1]), d);
-            credit(d, rb, st, t0 + 16 * st + col < lim[rb]);
-          }
+        for (int rb = 0; rb < 4; ++rb) {
+          qf[rb][0] = qn[rb][0];
+          qf[rb][1] = qn[rb][1];
         }
       }
-    }
-    __syncthreads();  // tile ti's maxima complete; tile ti - 1's reduction done
-    if ((ti + 1) % RING == 0 || ti + 1 == ntiles) {
-      // The ring's credits to the block counters: one atomic per credited block and workgroup.
-      reduce(ti);
       __syncthreads();
-      const int base = (ti - ti % RING) * KT;
-      for (int t = threadIdx.x; t < RING * KT; t += blockDim.x) {
-        const int key = base + t;
-        const float v = ring[t / KT][t % KT];
-        if ((key & ((1 << shift) - 1)) == 0 && key < kend && v > 0.f)
-          unsafeAtomicAdd(&a.scores[int64_t(slots[key]) * a.sss], v);
-        ring[t / KT][t % KT] = 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sl[j] = sn[j];
+
+    // Per (query, key) the maximum over all heads, of two key blocks at once: lane holds query i0 +
+    // 2*rb + grp/2 and key 32*kp + in_pair.
+    const int in_pair = 16 * (grp & 1) + col;
+    const bool leads = (in_pair & (block - 1)) == 0;
+#pragma unroll
+    for (int kp = 0; kp < KB / 2; kp += 2) {
+      float c[2] = {0.f, 0.f};
+#pragma unroll
+      for (int rb = 0; rb < 4; ++rb) {
+        float z[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(y[rb][2 * (kp + h)]),
+                                                          __float_as_uint(y[rb][2 * (kp + h) + 1]), false, false);
+          z[h] = vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
+          if (ti * KT + 32 * (kp + h) + in_pair >= lim[rb]) z[h] = -INFINITY;
+        }
+        for (int o = 1; o < block && o < 32; o <<= 1) {
+          z[0] = fmaxf(z[0], __shfl_xor(z[0], o, kWave));
+          z[1] = fmaxf(z[1], __shfl_xor(z[1], o, kWave));
+        }
+        if (block == 64) z[0] = fmaxf(z[0], z[1]);
+        c[0] += leads ? fast_exp2(z[0]) : 0.f;
+        c[1] += leads && block < 64 ? fast_exp2(z[1]) : 0.f;
       }
-      __syncthreads();
+      cols[wave][32 * kp + lane] = join32(c[0], c[1]);  // both queries of a row block
     }
-  };
-  // The common tiles in pairs (an even count, so the walk after them starts on set ka), then
-  // the rest. Each loop's body is unrolled by two so the K register sets alternate without copies.
-  const int n_common = ((limit(qb0) / KT) < ntiles ? limit(qb0) / KT : ntiles) & ~1;
-  int ti = 0;
-#pragma unroll 1
-  for (; ti < n_common; ti += 2) {
-    tile(ti, ka, kb, std::true_type{});
-    tile(ti + 1, kb, ka, std::true_type{});
-  }
-#pragma unroll 1
-  for (; ti < ntiles; ti += 2) {
-    tile(ti, ka, kb, std::false_type{});
-    if (ti + 1 < ntiles) tile(ti + 1, kb, ka, std::false_type{});
+    __syncthreads();
+    // The next tile's columns are written past its heads' barriers.
+    const int key = ti * KT + int(threadIdx.x);
+    if (int(threadIdx.x) < KT && key < kend && (key & (block - 1)) == 0) {
+      float v = 0.f;
+#pragma unroll
+      for (int w = 0; w < WAVES; ++w) v += cols[w][threadIdx.x];
+      if (v > 0.f) unsafeAtomicAdd(&a.scores[int64_t(slots[key]) * a.sss], v);
+    }
   }
 }
 
@@ -988,14 +979,6 @@ __global__ __launch_bounds__(p1::THREADS, NS == 0 ? 4 : 2) void diagnose_kernel(
       else
         rows(std::false_type{});
       // Lane l ends with key l: lane bit 4 selects the key block of a pair, bit 5 the pair.
-      auto join16 = [](float x, float y) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-      };
-      auto join32 = [](float x, float y) {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-      };
       tsum = join32(join16(cs[0], cs[1]), join16(cs[2], cs[3]));
       tmax = join32(cm[0], cm[1]);
     }
@@ -1114,11 +1097,18 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
                    prefix_len, sinks, sinks_dtype, kind, scores, scores_stride_g, scores_stride_s, q_heads, kv_heads,
                    sm_scale * kLog2e, static_cast<float*>(workspace), delay, block_shift};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (kind == GSE_SCORE_KIND_BLOCK_STEP && kv_heads > pb::WAVES)
+  if (kind == GSE_SCORE_KIND_BLOCK_STEP && q_heads > pb::MAX_HEADS)
     return gse_fail(GSE_ESHAPE, "prefill: block counters need kv_heads <= 8");
   if (int rc = launch_norms(a, workspace, s)) return rc;
   if (kind == GSE_SCORE_KIND_BLOCK_STEP) {
-    const dim3 bgrid(static_cast<uint32_t>((count + pb::QB - 1) / pb::QB));
+    const int64_t nqb = (count + pb::QB - 1) / pb::QB;
+    const int64_t first = prefix_len / pb::KT + 1, last = (total + pb::KT - 1) / pb::KT;
+    const int64_t work = (first + last + 1) / 2 * nqb;  // tiles of the launch
+    const int64_t tiles = std::max<int64_t>(1, (work + pb::ITEMS - 1) / pb::ITEMS);
+    a.tiles = int(tiles);  // of this pass's ranges (pass 1 and the merge are launched)
+    const int64_t items = nqb * ((last + tiles - 1) / tiles);
+    if (items >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
+    const dim3 bgrid{static_cast<uint32_t>(items)};
     if (slots_dtype == GSE_I64)
       hipLaunchKernelGGL(prefill_block_kernel<int64_t>, bgrid, dim3(pb::THREADS), 0, s, a);
     else
