@@ -237,6 +237,13 @@ struct KeyTiles {
   GSE_DEVICE void stage(int p, Tile (&tiles)[2]) { store(tiles[p], row[p]); }
 };
 
+// A row's normaliser (log2 units) from its one pair and the sink.
+GSE_DEVICE float row_norm(const PrefillArgs& a, int h, float ref, float sum) {
+  const float sink2 = load_float_dyn(a.sinks, a.sinks_dtype, h) * kLog2e;
+  const float m = fmaxf(ref, sink2);
+  return m + __log2f(sum * fast_exp2(ref - m) + fast_exp2(sink2 - m));
+}
+
 __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArgs a) {
   using namespace pf;
   using p1::QW;
@@ -344,12 +351,17 @@ __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArg
     const float nr = -xor32_max(xor16_max(-nref[rb]));
     const float total = xor32_sum(xor16_sum(sum[rb] * fast_exp2(nr - nref[rb])));
     const int64_t qi = i0 + 2 * rb + ((lane & 15) >> 3);
-    if (lane < 16 && qi < a.count)
-      a.part[(split * a.count + qi) * a.q_heads + g * GROUP + (lane & 7)] = float2{-nr, total};
+    if (lane < 16 && qi < a.count) {
+      const int h = g * GROUP + (lane & 7);
+      if (a.splits == 1)
+        a.norm2[qi * a.q_heads + h] = row_norm(a, h, -nr, total);
+      else
+        a.part[(split * a.count + qi) * a.q_heads + h] = float2{-nr, total};
+    }
   }
 }
 
-// Row normalisers in log2 units: thread = (query, head), joining the key ranges that hold keys of
+// Row normalisers in log2 units of several ranges: thread = (query, head), joining the key ranges that hold keys of
 // the row's query block and the sink.
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
   const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
@@ -1031,8 +1043,8 @@ __global__ __launch_bounds__(p1::THREADS, NS == 0 ? 4 : 2) void diagnose_kernel(
 
 using namespace gse;
 
-// Upper bound of pass 1's key ranges for a chunk of `count` queries: row_plan's item count divides
-// by the mean tiles of a query block, at least half of the last one's.
+// Upper bound of the key ranges pass 1 wants for a chunk of `count` queries: launch_norms divides the
+// item count by the mean tiles of a query block, at least half of the last one's.
 static int64_t max_splits(int64_t count, int kv_heads) {
   const int64_t blocks = (count + pf::QB - 1) / pf::QB * kv_heads;
   return blocks > 0 ? 2 * p1::ITEMS / blocks + 2 : 0;
@@ -1047,22 +1059,25 @@ extern "C" int64_t gse_prefill_workspace_bytes(int64_t count, int q_heads) {
 }
 
 // Pass 1 and the merge: row normalisers of a chunk into a.norm2. Fills in a's workspace pointers
-// and the key ranges.
-static int launch_norms(PrefillArgs& a, void* workspace, hipStream_t s) {
+// and the key ranges: as many as a workspace of at least the normalisers' bytes holds the pairs of
+// (one range leaves none).
+static int launch_norms(PrefillArgs& a, void* workspace, int64_t workspace_bytes, hipStream_t s) {
   a.norm2 = static_cast<float*>(workspace);
   a.part = reinterpret_cast<float2*>(static_cast<char*>(workspace) + norm_bytes(a.count, a.q_heads));
   const int64_t nqb = (a.count + pf::QB - 1) / pf::QB;
   const int64_t first = (a.prefix_len + (a.count < pf::QB ? a.count : pf::QB) + pf::KT - 1) / pf::KT;
   const int64_t last = (a.total + pf::KT - 1) / pf::KT;
   const int64_t work = (first + last + 1) / 2 * nqb * a.kv_heads;  // tiles of the launch
-  const int64_t tiles = std::max<int64_t>(p1::MIN_TILES, (work + p1::ITEMS - 1) / p1::ITEMS);
+  const int64_t room = (workspace_bytes - norm_bytes(a.count, a.q_heads)) / (a.count * a.q_heads * int64_t(sizeof(float2)));
+  int64_t tiles = std::max<int64_t>(p1::MIN_TILES, (work + p1::ITEMS - 1) / p1::ITEMS);
+  tiles = std::max(tiles, (last + std::max<int64_t>(room, 1) - 1) / std::max<int64_t>(room, 1));
   a.tiles = int(tiles);
   a.splits = int((last + tiles - 1) / tiles);
-  if (a.splits > max_splits(a.count, a.kv_heads)) return gse_fail(GSE_EINVAL, "prefill: key ranges past the workspace");
   const int64_t blocks = nqb * a.kv_heads * a.splits;
   if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
   hipLaunchKernelGGL(prefill_norm_kernel, dim3(uint32_t(blocks)), dim3(p1::THREADS), 0, s, a);
   if (int rc = gse_launch_check("prefill pass 1")) return rc;
+  if (a.splits == 1) return GSE_OK;
   const int64_t rows = a.count * a.q_heads;
   hipLaunchKernelGGL(prefill_merge_kernel, dim3(uint32_t((rows + 255) / 256)), dim3(256), 0, s, a);
   return gse_launch_check("prefill normalisers");
@@ -1090,8 +1105,7 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
   if (q_stride_t % 8 || q_stride_h % 8 || kv_stride_s % 8 || kv_stride_h % 8)
     return gse_fail(GSE_EINVAL, "prefill: strides must be multiples of 8 elements");
   if (!q || !k_pool || !slots || !sinks || !scores) return gse_fail(GSE_EINVAL, "prefill: null pointer");
-  if (workspace_bytes < gse_prefill_workspace_bytes(count, q_heads))
-    return gse_fail(GSE_EWORKSPACE, "prefill: workspace too small");
+  if (workspace_bytes < norm_bytes(count, q_heads)) return gse_fail(GSE_EWORKSPACE, "prefill: workspace too small");
   PrefillArgs a = {static_cast<const uint16_t*>(q), q_stride_t, q_stride_h, count,
                    static_cast<const uint16_t*>(k_pool), kv_stride_s, kv_stride_h, slots, slots_dtype, total,
                    prefix_len, sinks, sinks_dtype, kind, scores, scores_stride_g, scores_stride_s, q_heads, kv_heads,
@@ -1099,7 +1113,7 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (kind == GSE_SCORE_KIND_BLOCK_STEP && q_heads > pb::MAX_HEADS)
     return gse_fail(GSE_ESHAPE, "prefill: block counters need kv_heads <= 8");
-  if (int rc = launch_norms(a, workspace, s)) return rc;
+  if (int rc = launch_norms(a, workspace, workspace_bytes, s)) return rc;
   if (kind == GSE_SCORE_KIND_BLOCK_STEP) {
     const int64_t nqb = (count + pb::QB - 1) / pb::QB;
     const int64_t first = prefix_len / pb::KT + 1, last = (total + pb::KT - 1) / pb::KT;
@@ -1148,8 +1162,7 @@ extern "C" int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_s
     return gse_fail(GSE_EINVAL, "diagnose: null pointer");
   if (evicted_stride_g * 32 < ((total + 63) / 64) * 64)
     return gse_fail(GSE_EINVAL, "diagnose: evicted rows must cover the visible keys rounded up to 64");
-  if (workspace_bytes < gse_prefill_workspace_bytes(count, q_heads))
-    return gse_fail(GSE_EWORKSPACE, "diagnose: workspace too small");
+  if (workspace_bytes < norm_bytes(count, q_heads)) return gse_fail(GSE_EWORKSPACE, "diagnose: workspace too small");
   DiagArgs da;
   da.p = {static_cast<const uint16_t*>(q), q_stride_t, q_stride_h, count, static_cast<const uint16_t*>(k_pool),
           kv_stride_s, kv_stride_h, slots, slots_dtype, total, prefix_len, sinks, sinks_dtype, 1, score_sum,
@@ -1164,7 +1177,7 @@ extern "C" int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_s
   da.lost_ss = lost_stride_s;
   da.lost_scale = lost_scale;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (int rc = launch_norms(da.p, workspace, s)) return rc;
+  if (int rc = launch_norms(da.p, workspace, workspace_bytes, s)) return rc;
   // launch_norms has set the key ranges and checked the grid.
   const dim3 grid{static_cast<uint32_t>((count + pf::QB - 1) / pf::QB * kv_heads * da.p.splits)};
   static void (*const kernels[])(DiagArgs) = {diagnose_kernel<0>, diagnose_kernel<1>, diagnose_kernel<2>,

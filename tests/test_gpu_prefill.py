@@ -90,6 +90,22 @@ def test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, scal
     torch.testing.assert_close(st.scores[0][:, slots].double(), want, rtol=1e-5 + largest * 2 ** -22, atol=1e-7)
 
 
+@pytest.mark.parametrize("ranges", [1, 2, 5])
+def test_a_smaller_workspace_takes_fewer_key_ranges(ranges, monkeypatch):
+    """The normalisers' bytes alone are enough; each further range of pass 1 adds its pairs."""
+    count, prefix_len = 70, 3000
+    b, st, q, sinks, prefix, new = _case(count, prefix_len, seed=9)
+    keys = b.token_to_kv_pool.get_key_buffer(1)
+    slots = torch.cat((prefix, new)).long()
+    rows = count * 64
+    size = -(-rows * 4 // 256) * 256 + (rows * 8 * ranges if ranges > 1 else 0)
+    monkeypatch.setattr(st, "workspace", lambda name, nbytes: torch.empty(size, dtype=torch.uint8, device="cuda"))
+    st.scores.zero_()
+    ge._prefill_scores(st, 0, 1, layer(1), q, keys, sinks, prefix, new)
+    want = _exact_scores(1, q, keys, sinks, slots, prefix_len)
+    torch.testing.assert_close(st.scores[0][:, slots].double(), want, rtol=1e-4, atol=1e-7)
+
+
 def test_after_extend_scores_chunks_of_two_requests():
     """The hook path: CSR prefix per request, zeroed new slots, sum and max rows in one batch."""
     g = torch.Generator().manual_seed(21)

@@ -92,6 +92,26 @@ def test_layer_difference_matches_the_oracle(runtime, start, count, frontier, ke
     np.testing.assert_allclose(got, want, rtol=RTOL, atol=ATOL)
 
 
+# Chunks of one to 32 queries' blocks, whose key ranges run from 64 down to one, at the edges of the
+# blocks, tiles and ranges; each again in a workspace of the two outputs alone (one range).
+@pytest.mark.parametrize("start,count,frontier,kept", [
+    (2048, 1, 2048, 64), (2049, 31, 2048, 255), (4096, 33, 4096, 257), (2303, 65, 2048, 1000), (3000, 260, 2048, 100)])
+@pytest.mark.parametrize("small", [False, True])
+def test_layer_difference_over_key_ranges(runtime, monkeypatch, start, count, frontier, kept, small):
+    gen = torch.Generator().manual_seed(start + 3 * count)
+    k, v, direction = _shadow(start + count, gen)
+    q = _queries(count, direction, gen)
+    sinks = torch.randn(HEADS, generator=gen)
+    entry = {"frontier": frontier, "count": kept, "pos": _retained(frontier, kept, gen)}
+    if small:
+        st = runtime.state(backend(rows=2, width=64, slots=16, layers=2, full=(1,)))
+        size = 2 * -(-count * HEADS * DIM * 4 // 256) * 256
+        monkeypatch.setattr(type(st), "workspace", lambda self, name, nbytes: torch.empty(size, dtype=torch.uint8,
+                                                                                         device="cuda"))
+    got = _run(runtime, q, k, v, sinks, entry, start)
+    np.testing.assert_allclose(got, _oracle(q, k, v, sinks, entry, start), rtol=RTOL, atol=ATOL)
+
+
 def test_layer_difference_is_zero_before_any_eviction(runtime):
     gen = torch.Generator().manual_seed(9)
     k, v, direction = _shadow(700, gen)
