@@ -70,6 +70,14 @@ __global__ void zero_slots_kernel(float* scores, int layers, int64_t layer_strid
   scores[l * layer_stride + g * head_stride + int64_t(slots[s]) * slot_stride] = 0.f;
 }
 
+// out[i] = first[i] for i < n, then second[i - n].
+__global__ __launch_bounds__(256) void join_slots_kernel(const void* first, int first_dtype, int64_t n, const void* second,
+                                                       int second_dtype, int64_t total, int32_t* out) {
+  const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i < total)
+    out[i] = int32_t(i < n ? load_index_dyn(first, first_dtype, i) : load_index_dyn(second, second_dtype, i - n));
+}
+
 }  // namespace gse
 
 using namespace gse;
@@ -109,4 +117,16 @@ extern "C" int gse_zero_slots(float* scores, int layers, int64_t layer_stride, i
     hipLaunchKernelGGL(zero_slots_kernel<int32_t>, grid, dim3(256), 0, s, scores, layers, layer_stride, kv_heads,
                        head_stride, slot_stride, static_cast<const int32_t*>(slots), n);
   return gse_launch_check("zero_slots");
+}
+
+extern "C" int gse_join_slots(const void* first, int first_dtype, int64_t n, const void* second, int second_dtype,
+                              int64_t m, int32_t* out, gse_stream_t stream) {
+  if (n < 0 || m < 0) return gse_fail(GSE_EINVAL, "join_slots: negative size");
+  if (n + m == 0) return GSE_OK;
+  if ((n && !first) || (m && !second) || !out) return gse_fail(GSE_EINVAL, "join_slots: null pointer");
+  const int64_t blocks = (n + m + 255) / 256;
+  if (blocks >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "join_slots: too many slots");
+  hipLaunchKernelGGL(join_slots_kernel, dim3(uint32_t(blocks)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                     first, first_dtype, n, second, second_dtype, n + m, out);
+  return gse_launch_check("join_slots");
 }

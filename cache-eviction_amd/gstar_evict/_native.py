@@ -46,6 +46,7 @@ SIGNATURES = {
     "gse_last_error": (ctypes.c_char_p, []),
     "gse_fill": (_i, [_p, _l, _p, _l, _p, _i, _p, _i, _p, _p, _i, _l, _p, _p, _i, _p]),
     "gse_zero_slots": (_i, [_p, _i, _l, _i, _l, _l, _p, _i, _l, _p]),
+    "gse_join_slots": (_i, [_p, _i, _l, _p, _i, _l, _p, _p]),
     "gse_decode_workspace_bytes": (_l, [_i, _i, _i]),
     "gse_decode_fold_bytes": (_l, [_i, _i, _i]),
     "gse_decode": (_i, [_p, _l, _l, _p, _p, _l, _l, _p, _p, _i, _p, _i, _p, _p, _i, _p, _l, _l, _p, _l, _l, _p,

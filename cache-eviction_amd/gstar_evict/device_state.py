@@ -80,6 +80,7 @@ class State:
         self._pools = None
         self.pending = []  # boundaries queued on the device whose host part is still to do
         self._rows_host = self._rows_dev = self._rows_copied = None
+        self._ints_host = None  # read_ints' pinned buffer
 
     def workspace(self, name, nbytes):
         """A cached device byte buffer of at least nbytes (grows, never shrinks)."""
@@ -93,6 +94,23 @@ class State:
             self._ws.pop(name, None)
             buf = self._ws[name] = torch.empty(size, dtype=torch.uint8, device=self.device)
         return buf
+
+    def read_ints(self, *tensors):
+        """The values of small integer tensors as lists, with one wait for all of them: their copies
+        to a pinned buffer are queued together on the current stream."""
+        if any(t.device.type != "cuda" for t in tensors):
+            return [t.tolist() for t in tensors]
+        views, end = [], 0
+        for t in tensors:
+            views.append((end, end + t.numel() * t.element_size()))
+            end = -(-views[-1][1] // 8) * 8
+        if self._ints_host is None or self._ints_host.numel() < end:
+            self._ints_host = torch.empty(max(end, 4096), dtype=torch.uint8, pin_memory=True)
+        host = [self._ints_host[a:b].view(t.dtype).view(t.shape) for (a, b), t in zip(views, tensors)]
+        for h, t in zip(host, tensors):
+            h.copy_(t, non_blocking=True)
+        torch.cuda.current_stream(self.device).synchronize()
+        return [h.tolist() for h in host]
 
     def status_block(self, count=0):
         """A pinned host block of status rows ([rows, 16] int32, the first ``count`` for one

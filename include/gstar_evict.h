@@ -144,6 +144,11 @@ int gse_fill(const int32_t* table, int64_t table_stride, const int32_t* req_to_t
 int gse_zero_slots(float* scores, int layers, int64_t layer_stride, int kv_heads, int64_t head_stride,
                    int64_t slot_stride, const void* slots, int slots_dtype, int64_t n, gse_stream_t stream);
 
+/* A key list of two parts as int32 slots: out[0..n) = first, out[n..n+m) = second (each int32
+ * or int64, contiguous). */
+int gse_join_slots(const void* first, int first_dtype, int64_t n, const void* second, int second_dtype, int64_t m,
+                   int32_t* out, gse_stream_t stream);
+
 /* Workspace bytes gse_decode needs for bs sequences. */
 int64_t gse_decode_workspace_bytes(int bs, int q_heads, int head_dim);
 
