@@ -48,6 +48,39 @@ GSE_DEVICE uint4 ld16(const uint16_t* p) { return *reinterpret_cast<const uint4*
 // Keys per workgroup for P workgroups over T keys (0 when T == 0).
 GSE_DEVICE int fused_chunk(int T, int P) { return (T + P - 1) / P; }
 
+// The other partition, for batches of few sequences: every workgroup's keys lie in one sequence. With
+// C = ceil(T / (P - bs)) keys per workgroup, sequence b takes ceil(len_b / C) of them, at most P in
+// all; lane b of a wave counts sequence b's. A workgroup that crosses into a second sequence starts
+// its load pipeline again (some 3 us) and ends last; here the others' chunks grow by bs / P instead,
+// which a stream bound by HBM hardly shows; and the bounds come in one vector load instead of a chain
+// of scalar ones. A replayed step of 12 layers: 4 sequences of 7,850 to 8,020 keys 303 -> 273 us, 8 of
+// 3000 to 10,200 404 -> 363, 32 of up to 4096 604 -> 545 (with 16 workgroups or more per sequence
+// only: 596), 4 of up to 1500 180 -> 147. One sequence keeps the scalar form (140 us against 147 at
+// 2252 keys).
+struct Share {
+  int chunk;         // keys per workgroup
+  int start, end;    // the lane's sequence's list
+  int mine, before;  // its workgroups, and those of the sequences before it
+};
+GSE_DEVICE Share sequence_shares(const int32_t* indptr, int bs, int P, int lane) {
+  Share sh;
+  sh.start = lane < bs ? indptr[lane] : 0;
+  sh.end = lane < bs ? indptr[lane + 1] : 0;
+  const int T = __builtin_amdgcn_readlane(sh.end, bs - 1);
+  sh.chunk = max(1, (T + P - bs - 1) / (P - bs));
+  sh.mine = (sh.end - sh.start + sh.chunk - 1) / sh.chunk;
+  int upto = sh.mine;  // a scan over 32 lanes by row shifts, then lane 15's into the second row
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
+  upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);
+  sh.before = upto - sh.mine;
+  return sh;
+}
+constexpr int SHARE_MAX_BS = 32;
+constexpr int SHARE_MIN_WG = 8;  // workgroups per sequence: chunks grow by at most a seventh
+
 // Largest b in [0, bs) with indptr[b] <= p (indptr non-decreasing, indptr[0] = 0 <= p).
 GSE_DEVICE int seq_of(const int32_t* indptr, int bs, int p) {
   int lo = 0, hi = bs - 1;
@@ -84,6 +117,11 @@ struct FusedArgs {
   // queue q [rows, cap, q_heads, D], norm [rows, cap, q_heads], lim [rows, cap], count [rows]
   // into scores[g * ssg + slot * sss].
   int P;
+  bool whole_seq;  // workgroups by sequence_shares
+  // Queue mode: the queue counts this launch advances for the merge's append (null otherwise), and
+  // the rows' score words.
+  int32_t* step_count;
+  const int32_t* step_mode;
   const int32_t* fold_seq;
   int n_fold;
   const int32_t* mode;
@@ -101,11 +139,6 @@ struct FusedArgs {
   int fold_stride;
 };
 
-// A queue count word: the count in the low 24 bits; the merge's arrival tickets above them (at
-// most q_heads = 64 head workgroups per sequence, so the word stays below 2^31).
-constexpr int32_t QUEUE_TICKET = 1 << 24;
-constexpr int32_t QUEUE_COUNT_MASK = QUEUE_TICKET - 1;
-
 // The list entries of fold sequence i that its queue scores: [0, the largest scored length),
 // within the sequence's list and the totals buffer's stride; 0 when the row's kind is not 1 or 2
 // or its queue is empty.
@@ -115,8 +148,7 @@ GSE_DEVICE int fold_extent(const FusedArgs& a, int i) {
   const int64_t row = load_index_dyn(a.rows, a.rows_dtype, b);
   const int word = a.mode[row];
   const int md = score_kind(word);
-  int m = a.qcount[row] & QUEUE_COUNT_MASK;
-  m = m < a.cap ? m : a.cap;
+  const int m = min(a.qcount[row], a.cap);
   if ((md != 1 && md != 2) || m <= 0) return 0;
   int ext = 0;
   for (int q = 0; q < m; ++q) ext = max(ext, a.qlim[row * a.cap + q] - score_delay(word));
@@ -165,8 +197,7 @@ GSE_DEVICE void fold_role(const FusedArgs& a, uint16_t* qs, float* ns) {
       staged_g = g;
       const int word = a.mode[row];
       md = score_kind(word);
-      int m = a.qcount[row] & QUEUE_COUNT_MASK;
-      m = m < a.cap ? m : a.cap;
+      const int m = min(a.qcount[row], a.cap);
       maxlim = 0;
       if ((md == 1 || md == 2) && m > 0) {
         __syncthreads();  // the previous item's tiles have read the staged queue
@@ -191,6 +222,24 @@ GSE_DEVICE void fold_role(const FusedArgs& a, uint16_t* qs, float* ns) {
       fold_tiles<true>(qs, ns, lims, pmin, pmax, npairs, c0, wave, maxlim, a.scale2, kp, a.kv_ss, slot_of, put);
     else
       fold_tiles<false>(qs, ns, lims, pmin, pmax, npairs, c0, wave, maxlim, a.scale2, kp, a.kv_ss, slot_of, put);
+  }
+}
+
+// Advances the queue count of sequence w's row (and of sequences w + P, ...) by this step, for the
+// merge to append at count - 1: the launch boundary orders it before the merge's reads, which took an
+// arrival ticket per head group when the merge advanced the count itself (0.65 us per layer). A row
+// whose queue this launch folds restarts in the merge instead.
+GSE_DEVICE void count_steps(const FusedArgs& a, int w, int64_t row, int word) {
+  if (!a.step_count || threadIdx.x != 0) return;
+  for (int b = w; b < a.bs; b += a.P) {
+    if (b != w) {
+      row = load_index_dyn(a.rows, a.rows_dtype, b);
+      word = a.step_mode[row];
+    }
+    const int md = score_kind(word);
+    bool folded = false;
+    for (int i = 0; i < a.n_fold; ++i) folded |= a.fold_seq[i] == b;
+    if (scoring_kind(md) && !(folded && (md == 1 || md == 2))) atomicAdd(a.step_count + row, 1);
   }
 }
 
@@ -228,12 +277,36 @@ __global__ __launch_bounds__(FUSED_THREADS) void decode_fused_kernel(FusedArgs a
   // Key positions are CSR offsets (int32 in the CSR itself).
   const int P = a.P;
   const int w = blockIdx.x;
-  const int T = a.indptr[a.bs];
-  const int C = fused_chunk(T, P);
-  int p = w * C;
-  const int p_end = p + C < T ? p + C : T;
-  if (p >= p_end) return;
-  int b = seq_of(a.indptr, a.bs, p);
+  // Workgroup w counts the step of sequence w (and w + P, ...): its row's score word is on its way
+  // while the keys stream, and the count moves when they have.
+  const bool counts = a.step_count && w < a.bs;
+  const int64_t own_row = counts ? load_index_dyn(a.rows, a.rows_dtype, w) : 0;
+  int p, p_end, b, seq_end;
+  int64_t slot0 = w;  // the partial of this workgroup's segment in sequence b is slot0 + b
+  if (a.whole_seq) {
+    const Share sh = sequence_shares(a.indptr, a.bs, P, lane);
+    const uint64_t own = __builtin_amdgcn_ballot_w64(sh.before <= w && w < sh.before + sh.mine);
+    if (!own) {
+      count_steps(a, w, own_row, counts ? a.step_mode[own_row] : 0);
+      return;
+    }
+    b = __builtin_ctzll(own);
+    seq_end = __builtin_amdgcn_readlane(sh.end, b);
+    p = __builtin_amdgcn_readlane(sh.start, b) + (w - __builtin_amdgcn_readlane(sh.before, b)) * sh.chunk;
+    p_end = min(p + sh.chunk, seq_end);
+    slot0 -= b;  // one segment: slot w
+  } else {
+    const int T = a.indptr[a.bs];
+    const int C = fused_chunk(T, P);
+    p = w * C;
+    p_end = p + C < T ? p + C : T;
+    if (p >= p_end) {
+      count_steps(a, w, own_row, counts ? a.step_mode[own_row] : 0);
+      return;
+    }
+    b = seq_of(a.indptr, a.bs, p);
+    seq_end = a.indptr[b + 1];
+  }
 
   // Load i of a tile: lane l reads 16-byte piece l % 8 of the wave's head row of key 8 * i + l / 8.
   const int krow = lane >> 3, piece = lane & 7;
@@ -248,10 +321,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void decode_fused_kernel(FusedArgs a
     uint4 k[8], v[8];
   };
 
+  const int own_word = counts ? a.step_mode[own_row] : 0;
   while (p < p_end) {
-    while (a.indptr[b + 1] <= p) ++b;  // skip empty sequences
+    while (seq_end <= p) seq_end = a.indptr[++b + 1];  // the next sequence, skipping empty ones
     const int s0 = p;
-    const int s1 = a.indptr[b + 1] < p_end ? a.indptr[b + 1] : p_end;
+    const int s1 = seq_end < p_end ? seq_end : p_end;
 
     // B operand: column col supplies dims [8*grp, 8*grp + 8) and [32 + 8*grp, ...) of its head.
     bf16x8_t qf0 = {}, qf1 = {};
@@ -431,7 +505,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void decode_fused_kernel(FusedArgs a
     // This segment's partial: O^T rows 4*grp + r of dim block j, column col; m and l.
     const float lt = xor32_sum(xor16_sum(l_run));
     if (live_col) {
-      float* pp = a.part + ((int64_t(w) + b) * a.q_heads + hq) * PART;
+      float* pp = a.part + ((slot0 + b) * a.q_heads + hq) * PART;
 #pragma unroll
       for (int j = 0; j < 4; ++j) *reinterpret_cast<f32x4_t*>(pp + 16 * j + 4 * grp) = oacc[j];
       if (grp == 0) {
@@ -440,8 +514,8 @@ __global__ __launch_bounds__(FUSED_THREADS) void decode_fused_kernel(FusedArgs a
       }
     }
     p = s1;
-    ++b;
   }
+  count_steps(a, w, own_row, own_word);
 }
 
 // ---------------------------------------------------------------------------
@@ -455,9 +529,9 @@ struct MergeArgs {
   uint16_t* o;
   int64_t o_sb, o_sh;
   float* norm_out;  // [bs, q_heads]
-  // Score queue (GSE_SCORE_QUEUE): for rows whose score mode is 1 or 2, entry n = qcount[row] gets
-  // the step's query, normaliser and list length if n < cap, and qcount[row] = n + 1 (a count
-  // above cap records dropped steps).
+  // Score queue (GSE_SCORE_QUEUE): for rows whose score mode is 1 or 2, entry n = qcount[row] - 1
+  // (the fused kernel has counted the step) gets its query, normaliser and list length if n < cap (a
+  // count above cap records dropped steps).
   const uint16_t* q;
   int64_t q_sb, q_sh;
   const int32_t* mode;
@@ -469,6 +543,7 @@ struct MergeArgs {
   int32_t* qcount;  // [rows]
   int cap;
   int bs, q_heads, nparts;  // nparts = P, the fused kernel's attention workgroup count
+  bool whole_seq;           // its workgroups by sequence_shares
   // Sequences whose queue the fused kernel folded (score kinds 1 and 2): their step goes to
   // entry 0 and their count becomes 1, and their totals (the fused kernel's fold_buf / fold_hdr,
   // over the CSR list `indices`) are added to scores[g * ssg + slot * sss].
@@ -518,10 +593,6 @@ GSE_DEVICE void fold_scatter(const MergeArgs& a) {
 // eight), so a sequence's partials cost ceil(count / (8 * SPLIT)) rounds of loads. Instances:
 // <1, 8> for batches whose sequences span at most 8 workgroups, <8, 8> up to 64, <64, 1> past
 // that (a single long sequence: one head per workgroup, 64 groups).
-// A sequence's head groups run in separate workgroups, so its queue count is advanced by the
-// last of them to finish: each adds one arrival ticket (bit 24 up) to the count word after it
-// has read the count, and the one that sees every other ticket there removes the tickets and
-// adds the step. The count's low 24 bits never change while a group can still read them.
 constexpr int MERGE_BATCH = 8;
 constexpr int MERGE_SCATTER_ROWS = 8;  // grid rows of the merge launch that scatter the fold's totals
 template <int SPLIT, int HEADS>
@@ -546,7 +617,7 @@ __global__ __launch_bounds__(16 * HEADS * SPLIT) void decode_merge_kernel(MergeA
   if (a.qq) {
     row = load_index_dyn(a.rows, a.rows_dtype, b);
     const int md = score_kind(a.mode[row]);
-    slot = a.qcount[row] & QUEUE_COUNT_MASK;
+    slot = a.qcount[row] - 1;  // the fused kernel has counted the step
     queue = scoring_kind(md);
     bool listed = false;
     for (int i = 0; i < a.n_fold; ++i) listed |= a.fold_seq[i] == b;
@@ -556,11 +627,15 @@ __global__ __launch_bounds__(16 * HEADS * SPLIT) void decode_merge_kernel(MergeA
   const bool live = h < a.q_heads;
   const int hh = live ? h : 0;
   const uint2 qv = *reinterpret_cast<const uint2*>(a.q + int64_t(b) * a.q_sb + int64_t(hh) * a.q_sh + 4 * j);
-  const int T = a.indptr[a.bs];
-  const int C = fused_chunk(T, a.nparts);
   const int start = a.indptr[b], end = a.indptr[b + 1];
-  int wf = 1, wl = 0;
-  if (end > start) {
+  int wf = 1, wl = 0, slot0 = b;  // workgroup w's partial of this sequence is slot0 + w
+  if (a.whole_seq) {
+    const Share sh = sequence_shares(a.indptr, a.bs, a.nparts, threadIdx.x & 63);
+    wf = __builtin_amdgcn_readlane(sh.before, b);
+    wl = wf + __builtin_amdgcn_readlane(sh.mine, b) - 1;
+    slot0 = 0;
+  } else if (end > start) {
+    const int C = fused_chunk(a.indptr[a.bs], a.nparts);
     wf = start / C;
     wl = (end - 1) / C;
   }
@@ -573,7 +648,7 @@ __global__ __launch_bounds__(16 * HEADS * SPLIT) void decode_merge_kernel(MergeA
 #pragma unroll
     for (int k = 0; k < MERGE_BATCH; ++k) {
       const int w = w0 + k <= wl ? w0 + k : wl;
-      const float* ps = a.part + ((int64_t(w) + b) * a.q_heads + hh) * PART;
+      const float* ps = a.part + ((int64_t(w) + slot0) * a.q_heads + hh) * PART;
       pm[k] = w0 + k <= wl ? ps[D] : -INFINITY;
       pl[k] = ps[D + 1];
       po[k] = *reinterpret_cast<const f32x4_t*>(ps + 4 * j);
@@ -639,16 +714,7 @@ __global__ __launch_bounds__(16 * HEADS * SPLIT) void decode_merge_kernel(MergeA
       if (threadIdx.x == 0 && blockIdx.y == 0) a.qlim[e] = end - start;
     }
   }
-  if (!queue) return;
-  // Every thread of this group has read the count before its ticket goes in.
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int groups = a.head_groups;
-    const int32_t before = atomicAdd(a.qcount + row, QUEUE_TICKET);
-    // A folded queue restarts: the count goes from its old value to 1.
-    const int32_t step = folded ? 1 - (before & QUEUE_COUNT_MASK) : 1;
-    if ((before >> 24) == groups - 1) atomicAdd(a.qcount + row, step - groups * QUEUE_TICKET);
-  }
+  if (folded && threadIdx.x == 0 && blockIdx.y == 0) a.qcount[row] = 1;  // the folded queue restarts
 }
 
 // ---------------------------------------------------------------------------
@@ -1005,6 +1071,11 @@ int decode_run(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void
     f.lcap = logit_cap;
   }
   f.P = P;
+  if (score_mode == GSE_SCORE_QUEUE) {
+    f.step_count = queue_count;
+    f.step_mode = mode_by_row;
+  }
+  f.whole_seq = bs > 1 && bs <= SHARE_MAX_BS && bs * SHARE_MIN_WG <= P;
   if (n_fold > 0) {
     f.fold_seq = fold_seq;
     f.n_fold = n_fold;
@@ -1061,6 +1132,7 @@ int decode_run(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void
   m.bs = bs;
   m.q_heads = q_heads;
   m.nparts = P;
+  m.whole_seq = f.whole_seq;
   m.fold_seq = fold_seq;
   m.n_fold = n_fold;
   m.fold_buf = f.fold_buf;

@@ -411,8 +411,7 @@ def test_full_queues_flush_before_the_step(monkeypatch, mode):
 def test_merge_of_empty_short_and_long_sequences_over_a_reused_workspace():
     """The merge of a batch with empty sequences (all mass on the sink: o = 0, normaliser =
     sink, queued with list length 0), one inside a single workgroup and one across many; then a
-    smaller batch on the same workspace. Each row's queue count is exactly one step after its
-    head groups' arrival tickets are taken back."""
+    smaller batch on the same workspace. Each row's queue count is exactly one step."""
     for call, lengths in enumerate(([0, 5, 4000, 0, 1], [300, 2])):
         b, st, q, sinks, perm, indptr, rows = _decode_setup(lengths, seed=20 + call)
         if call:
@@ -444,6 +443,46 @@ def test_merge_of_empty_short_and_long_sequences_over_a_reused_workspace():
             np.testing.assert_allclose(st.qnorm[index, row, 0].cpu().numpy(), want_norm, rtol=1e-5, atol=1e-4)
         assert torch.equal(st.qq[index, rows, 0], q)
         ge.STATE = None
+
+
+# Batches whose workgroups each keep to one sequence (2 to 32 sequences, at least 8 workgroups per
+# sequence), at the edges of that rule and of the shares: empty lists, one key, all of the keys in one
+# list; then more sequences than workgroups (one tile in all), where a workgroup counts several rows.
+@pytest.mark.parametrize("lengths", [
+    [1, 1], [0, 5000], [6000, 0], [700] * 3 + [1], [2047, 2049, 0, 64, 63], [513] * 8, [300] * 31 + [0],
+    [600] * 32, [600] * 33, [1] * 40, [0] * 20 + [3] + [0] * 20])
+def test_workgroups_of_one_sequence_each(lengths):
+    bs = len(lengths)
+    b, st, q, sinks, perm, indptr, rows = _decode_setup(lengths, seed=bs + sum(lengths), slots=24000)
+    st.score_mode = "queue"
+    kinds = torch.tensor([i % 3 for i in range(bs)], dtype=torch.int32, device="cuda")  # kind 0: not queued
+    st.mode[:] = 0
+    st.mode[rows] = kinds
+    b.forward_metadata = SimpleNamespace(kv_indptr=indptr, kv_indices=perm)
+    fb = SimpleNamespace(out_cache_loc=torch.zeros(bs, dtype=torch.int64, device="cuda"), req_pool_indices=rows,
+                         seq_lens_cpu=torch.tensor(lengths))
+    o = torch.full_like(q, float("nan"))
+    for step in range(2):
+        assert ge.decode(b, q.reshape(bs, -1), layer(1), fb, sinks, o.reshape(bs, -1))
+    index = st.index[1]
+    keys, values = (f(1) for f in (b.token_to_kv_pool.get_key_buffer, b.token_to_kv_pool.get_value_buffer))
+    counts = torch.where(kinds > 0, 2, 0).to(torch.int32)
+    assert torch.equal(st.qcount[index, rows], counts)
+    assert int(st.qcount[index].sum()) == int(counts.sum())  # no other row's moved
+    for i, n in enumerate(lengths):
+        slots = perm[indptr[i]:indptr[i + 1]].long()
+        x = torch.matmul(q[i].double().view(8, 8, 64), keys[slots].double().permute(1, 2, 0).contiguous()) * 0.125
+        sink = sinks.double().view(8, 8)
+        norm = torch.logaddexp(torch.logsumexp(x, -1), sink) if n else sink
+        want = torch.matmul(torch.exp(x - norm[..., None]), values[slots].double().transpose(0, 1).contiguous())
+        # Probabilities and outputs are rounded to bf16 (2^-9 each); values are N(0, 1).
+        torch.testing.assert_close(o[i].double(), want.reshape(64, 64), rtol=8e-3, atol=8e-3)
+        if kinds[i]:
+            for entry in range(2):
+                torch.testing.assert_close(st.qnorm[index, rows[i], entry].double(), norm.reshape(64), rtol=1e-6,
+                                           atol=4e-6)
+                assert int(st.qlim[index, rows[i], entry]) == n
+                assert torch.equal(st.qq[index, rows[i], entry], q[i])
 
 
 @pytest.mark.parametrize("bs", [40, 5, 3, 1, 300])
