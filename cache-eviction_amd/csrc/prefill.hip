@@ -78,13 +78,17 @@ constexpr int QW = 8;                // queries per wave: two column blocks of 4
 constexpr int WAVES = 8;
 constexpr int THREADS = 64 * WAVES;
 static_assert(QW * WAVES == pf::QB, "a workgroup's queries");
-// Work items of a launch: about three rounds of the 512 workgroups the chip holds (2 per CU), at
-// least MIN_TILES tiles each (an item's start, its query and first key loads, costs some 3 us).
-// Both passes, 2048 tokens without a prefix: 97 us; twice the items or half the tiles 117, a third
-// fewer items 94. 190 tokens after 7000: 59 against 64. Past 2048 tokens after 28,672 the split no
-// longer matters (1231 us, 1241 with twice the items, 1271 with a third fewer).
-constexpr int ITEMS = 1536;
-constexpr int MIN_TILES = 8;
+// Work items of a launch: about three rounds of the SLOTS workgroups the chip holds (2 per CU). Where
+// these have FEW_TILES tiles or less each to do, whole rounds count: then the item length (at least
+// MIN_TILES tiles) whose rounds take least, with the start of an item (its query and first key loads,
+// some 4 us) counted as START tiles. Both passes, 2048 tokens without a prefix: 96 us with items of 8
+// tiles (1.25 rounds), 88 in one round; 60 after 1000 33 -> 29; 190 after 7000 61 -> 56. Past that the
+// rounds' count no longer decides (8192 after 28,672: 5.45 ms, 5.8 with the fewest rounds).
+constexpr int SLOTS = 512;
+constexpr int ITEMS = 3 * SLOTS;
+constexpr int FEW_TILES = 16;
+constexpr int MIN_TILES = 4;
+constexpr double START = 2.3;
 }  // namespace p1
 
 // Key ranges of a query block that sees ntiles tiles (equal ones, of at most `tiles` tiles).
@@ -404,11 +408,14 @@ constexpr int WAVES = 4;
 constexpr int KB = KW * WAVES;
 constexpr int THREADS = 64 * WAVES;
 constexpr int QT = 8;  // queries per tile (64 rows)
-// Work items of a launch (as p1::ITEMS), the fewest queries per item, and the most: a sum takes at
-// most MAX_QUERIES / 4 additions in one register, so its rounding error stays near that of a sum
-// over 64-query blocks.
-constexpr int ITEMS = 2048;
-constexpr int MIN_QUERIES = 64;
+// Work items of a launch and the rule for few tiles as in p1 (4 workgroups per CU), the fewest queries
+// of an item, and the most: a sum takes at most MAX_QUERIES / 4 additions in one register, so its
+// rounding error stays near that of a sum over 64-query blocks.
+constexpr int SLOTS = 1024;
+constexpr int ITEMS = 2 * SLOTS;
+constexpr int FEW_TILES = 20;
+constexpr double START = 1.5;
+constexpr int MIN_QUERIES = 32;
 constexpr int MAX_QUERIES = 512;
 }  // namespace p2
 
@@ -1065,12 +1072,26 @@ static int launch_norms(PrefillArgs& a, void* workspace, int64_t workspace_bytes
   a.norm2 = static_cast<float*>(workspace);
   a.part = reinterpret_cast<float2*>(static_cast<char*>(workspace) + norm_bytes(a.count, a.q_heads));
   const int64_t nqb = (a.count + pf::QB - 1) / pf::QB;
-  const int64_t first = (a.prefix_len + (a.count < pf::QB ? a.count : pf::QB) + pf::KT - 1) / pf::KT;
   const int64_t last = (a.total + pf::KT - 1) / pf::KT;
-  const int64_t work = (first + last + 1) / 2 * nqb * a.kv_heads;  // tiles of the launch
   const int64_t room = (workspace_bytes - norm_bytes(a.count, a.q_heads)) / (a.count * a.q_heads * int64_t(sizeof(float2)));
-  int64_t tiles = std::max<int64_t>(p1::MIN_TILES, (work + p1::ITEMS - 1) / p1::ITEMS);
-  tiles = std::max(tiles, (last + std::max<int64_t>(room, 1) - 1) / std::max<int64_t>(room, 1));
+  const int64_t most = std::max<int64_t>(1, std::min({max_splits(a.count, a.kv_heads), room, last / p1::MIN_TILES}));
+  // Tiles that query block b sees, and the launch's (by the mean block).
+  auto sees = [&](int64_t b) { return (a.prefix_len + std::min((b + 1) * pf::QB, a.count) + pf::KT - 1) / pf::KT; };
+  const int64_t work = (sees(0) + last + 1) / 2 * nqb * a.kv_heads;
+  int64_t tiles = std::max<int64_t>((work + p1::ITEMS - 1) / p1::ITEMS, (last + most - 1) / most);
+  if (work <= p1::FEW_TILES * p1::SLOTS) {
+    double best = 0;
+    for (int64_t n = 1; n <= most; n += 1 + n / 16) {
+      const int64_t t = (last + n - 1) / n;
+      int64_t items = 0;
+      for (int64_t b = 0; b < nqb; ++b) items += (sees(b) + t - 1) / t;
+      const double cost = double((items * a.kv_heads + p1::SLOTS - 1) / p1::SLOTS) * (double(t) + p1::START);
+      if (n == 1 || cost < best) {
+        best = cost;
+        tiles = t;
+      }
+    }
+  }
   a.tiles = int(tiles);
   a.splits = int((last + tiles - 1) / tiles);
   const int64_t blocks = nqb * a.kv_heads * a.splits;
@@ -1130,9 +1151,28 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
     return gse_launch_check("prefill block counters");
   }
   const int64_t nkb = (total + p2::KB - 1) / p2::KB;
-  const int64_t want = std::max<int64_t>(1, p2::ITEMS / (nkb * kv_heads));
-  const int64_t nq = std::min(want, (count + p2::MIN_QUERIES - 1) / p2::MIN_QUERIES);
-  a.qblock = int(std::min<int64_t>(((count + nq - 1) / nq + p2::QT - 1) / p2::QT * p2::QT, p2::MAX_QUERIES));
+  const int64_t bound0 = prefix_len - delay;  // query i credits keys up to bound0 + i
+  auto block_of = [&](int64_t n) {  // queries of one of n blocks
+    return std::min<int64_t>(((count + n - 1) / n + p2::QT - 1) / p2::QT * p2::QT, p2::MAX_QUERIES);
+  };
+  const int64_t nqmax = (count + p2::MIN_QUERIES - 1) / p2::MIN_QUERIES;
+  a.qblock = int(block_of(std::min(std::max<int64_t>(1, p2::ITEMS / (nkb * kv_heads)), (nqmax + 1) / 2)));
+  // As for pass 1, few tiles per workgroup: the query block whose rounds take least. The key blocks that
+  // only part of the chunk credits have fewer query blocks.
+  if (nkb * kv_heads * ((count + p2::QT - 1) / p2::QT) <= p2::FEW_TILES * p2::SLOTS) {
+    double best = 0;
+    for (int64_t n = (count + p2::MAX_QUERIES - 1) / p2::MAX_QUERIES, first = n; n <= nqmax; n += 1 + n / 16) {
+      const int64_t qblock = block_of(n), nq = (count + qblock - 1) / qblock;
+      int64_t live = 0;
+      for (int64_t k = 0; k < nkb; ++k)
+        live += std::max<int64_t>(0, nq - std::max<int64_t>(0, k * p2::KB - bound0) / qblock);
+      const double cost = double((live * kv_heads + p2::SLOTS - 1) / p2::SLOTS) * (double(qblock) / p2::QT + p2::START);
+      if (n == first || cost < best) {
+        best = cost;
+        a.qblock = int(qblock);
+      }
+    }
+  }
   const int64_t items = nkb * ((count + a.qblock - 1) / a.qblock) * kv_heads;
   if (items >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
   if (kind == 2)
