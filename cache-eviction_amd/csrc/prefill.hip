@@ -71,7 +71,7 @@ struct PrefillArgs {
 // mix alone runs at 2.2 GHz, 139 ns per 1024 logits; 32x32x16 MFMAs take fewer issue slots but
 // more power (156 ns), and the FMA with a vector instead of a scalar scale 147 ns. Against rows
 // spread over 16 lanes (a running maximum per row and lane) with 2 waves per SIMD and whole causal
-// ranges: 87 -> 42 us for the first 2048 tokens of a prompt, 816 -> 640 us for 1896 tokens after
+// ranges: 87 -> 43 us for the first 2048 tokens of a prompt, 816 -> 640 us for 1896 tokens after
 // 30,720, 3.36 -> 2.75 ms for 8192 after 28,672.
 namespace p1 {
 constexpr int QW = 8;                // queries per wave: two column blocks of 4 queries x 8 heads
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 // a sum per key), max mode S = Q . K^T (a lane holds 4 heads of a query for one key: the maximum
 // over the heads is in the lane and its neighbouring group). 4 waves per SIMD. Bound as pass 1;
 // max mode takes one exponential per (query, key). Against query blocks of 64 walking the keys (column sums through LDS rings, two
-// waves per SIMD): sums 77 -> 52 us for the first 2048 tokens of a prompt, 3.4 -> 2.5 ms for 8192
+// waves per SIMD): sums 77 -> 44 us for the first 2048 tokens of a prompt, 3.4 -> 2.5 ms for 8192
 // tokens after 28,672; maxima 1120 -> 450 us for 1896 after 30,720.
 namespace p2 {
 constexpr int KW = 64;  // keys per wave: two 32-key blocks
