@@ -90,6 +90,18 @@ def test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, scal
     torch.testing.assert_close(st.scores[0][:, slots].double(), want, rtol=1e-5 + largest * 2 ** -22, atol=1e-7)
 
 
+@pytest.mark.parametrize("n,m,first,second", [
+    (0, 1, torch.int32, torch.int64), (255, 1, torch.int32, torch.int64), (1, 256, torch.int64, torch.int32),
+    (300, 0, torch.int64, torch.int64), (257, 513, torch.int16, torch.int32)])
+def test_visible_slots_of_any_index_width(n, m, first, second):
+    from gstar_evict import attention
+    prefix = torch.arange(3, 3 + 2 * n, 2, device="cuda").to(first)
+    new = torch.arange(10 * m, 0, -5, device="cuda").to(second)[::2]  # a strided view
+    got = attention.visible_slots(prefix, new)
+    assert got.dtype == torch.int32
+    assert got.tolist() == prefix.tolist() + new.tolist()
+
+
 @pytest.mark.parametrize("ranges", [1, 2, 5])
 def test_a_smaller_workspace_takes_fewer_key_ranges(ranges, monkeypatch):
     """The normalisers' bytes alone are enough; each further range of pass 1 adds its pairs."""
