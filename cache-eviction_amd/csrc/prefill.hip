@@ -219,8 +219,8 @@ struct KeyTiles {
       : a(a_), kend(kend_), lk(threadIdx.x >> 3), lp(threadIdx.x & 7),
         base(as_global(a_.k) + int64_t(g) * a_.kv_sh + 8 * (threadIdx.x & 7)) {}
   GSE_DEVICE int32_t slot_at(int ti) const {
-    const int key = ti * pf::KT + lk;
-    return key < kend ? int32_t(load_index_dyn(a.slots, a.slots_dtype, key)) : 0;
+    const uint32_t key = uint32_t(ti) * pf::KT + lk;  // up to four tiles past kend < 2^31
+    return key < uint32_t(kend) ? int32_t(load_index_dyn(a.slots, a.slots_dtype, key)) : 0;
   }
   GSE_DEVICE uint4 load(int32_t s) const { return gload16(base + int64_t(s) * a.kv_ss); }
   GSE_DEVICE void store(Tile& tile, const uint4& x) const { *reinterpret_cast<uint4*>(&tile[lk * pf::KROW + 8 * lp]) = x; }
@@ -532,7 +532,7 @@ __global__ __launch_bounds__(p2::THREADS, 4) void prefill_score_kernel(PrefillAr
   bf16x8_t kf[4][2];
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) {
-    const int key = min(kw + 16 * kb + (lane & 15), int(a.total) - 1);
+    const uint32_t key = min(uint32_t(kw) + 16 * kb + (lane & 15), uint32_t(a.total) - 1);
     const int64_t s = load_index_dyn(a.slots, a.slots_dtype, key);
     const auto kp = as_global(a.k) + s * a.kv_ss + int64_t(g) * a.kv_sh + 8 * (lane >> 4);
     kf[kb][0] = as_bf16x8(gload16(kp));
@@ -710,7 +710,7 @@ __global__ __launch_bounds__(pb::THREADS, 2) void prefill_block_kernel(PrefillAr
   const int lk = threadIdx.x >> 3, lp = threadIdx.x & 7;
   auto load_slots = [&](int ti, IdxT (&sl)[4]) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sl[j] = slots[min(ti * KT + 64 * j + lk, kend - 1)];
+    for (int j = 0; j < 4; ++j) sl[j] = slots[min(uint32_t(ti) * KT + 64 * j + lk, uint32_t(kend) - 1)];
   };
   const auto kbase = as_global(a.k) + 8 * lp;
   auto load_k = [&](int g, const IdxT (&sl)[4], uint4 (&x)[4]) {

@@ -250,14 +250,14 @@ __global__ __launch_bounds__(64 * rp::WAVES, 4) void replay_output_kernel(Replay
   // until its tile's rows are loaded, so the index load is not waited for where it is issued.
   const int n_retained = int(sd.n_retained), tail0 = int(sd.tail0) - n_retained;
   auto row_at = [&](int t0) -> int32_t {
-    const int c = t0 + lk;
-    return c < kend && c < n_retained ? sd.retained[g * sd.ret_sg + c] : 0;
+    const uint32_t c = uint32_t(t0) + lk;  // up to two tiles past kend < 2^31
+    return c < uint32_t(kend) && c < uint32_t(n_retained) ? sd.retained[g * sd.ret_sg + c] : 0;
   };
   const int rows = int(a.rows < INT32_MAX ? a.rows : INT32_MAX);
   const auto base = as_global(src) + int64_t(g) * a.kv_sh + 16 * lp;
   auto load_rows = [&](int32_t retained_row, int t0, uint4 (&x)[2]) {
-    const int c = t0 + lk;
-    const int32_t row = c >= kend ? 0 : c < n_retained ? retained_row : tail0 + c;
+    const uint32_t c = uint32_t(t0) + lk;
+    const int32_t row = c >= uint32_t(kend) ? 0 : c < uint32_t(n_retained) ? retained_row : tail0 + int32_t(c);
     const auto p = base + (uint32_t(row) < uint32_t(rows) ? row : 0) * a.kv_ss;
     x[0] = gload16(p);
     x[1] = gload16(p + 8);
