@@ -178,3 +178,18 @@ def test_csr_check_runs_before_the_decode_launch(hooks, monkeypatch):
     with pytest.raises(ValueError, match="kv_indices holds 3"):
         attention.fused_decode(st, b, q, lay, SimpleNamespace(out_cache_loc=torch.zeros(1, dtype=torch.int64)),
                                torch.zeros(64), torch.zeros_like(q))
+
+
+def test_a_batch_without_an_opted_in_row_needs_no_bounds(hooks):
+    """after_extend of rows that opted out returns while another request is live, whatever its
+    metadata holds; a batch with an opted-in row is refused without bounds."""
+    from fakes import layer
+    ge, st, _ = hooks
+    _extend(ge, _req("a", 1, 0, 2048, {"gstar_eviction": CFG}))
+    out = SimpleNamespace(req_pool_indices=torch.tensor([2, 3]))
+    for b in (SimpleNamespace(), SimpleNamespace(forward_metadata=None),
+              SimpleNamespace(forward_metadata=SimpleNamespace(qo_indptr=None)),
+              SimpleNamespace(forward_metadata=SimpleNamespace(kv_indptr=torch.tensor([0, 5, 9])))):
+        assert ge.after_extend(b, None, layer(0), out, None) is None
+        with pytest.raises((ValueError, AttributeError)):
+            ge.after_extend(b, None, layer(0), SimpleNamespace(req_pool_indices=torch.tensor([2, 1])), None)
