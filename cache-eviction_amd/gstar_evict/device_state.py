@@ -7,6 +7,7 @@ workspaces and the per-layer K/V pointer tables of the boundary kernels.
 from __future__ import annotations
 
 import os
+import threading
 
 import torch
 
@@ -80,7 +81,7 @@ class State:
         self._pools = None
         self.pending = []  # boundaries queued on the device whose host part is still to do
         self._rows_host = self._rows_dev = self._rows_copied = None
-        self._ints_host = None  # read_ints' pinned buffer
+        self._ints_host = threading.local()  # read_ints' pinned buffer, one per thread
 
     def workspace(self, name, nbytes):
         """A cached device byte buffer of at least nbytes (grows, never shrinks)."""
@@ -97,16 +98,17 @@ class State:
 
     def read_ints(self, *tensors):
         """The values of small integer tensors as lists, with one wait for all of them: their copies
-        to a pinned buffer are queued together on the current stream."""
+        to the thread's pinned buffer are queued together on the current stream."""
         if any(t.device.type != "cuda" for t in tensors):
             return [t.tolist() for t in tensors]
         views, end = [], 0
         for t in tensors:
             views.append((end, end + t.numel() * t.element_size()))
             end = -(-views[-1][1] // 8) * 8
-        if self._ints_host is None or self._ints_host.numel() < end:
-            self._ints_host = torch.empty(max(end, 4096), dtype=torch.uint8, pin_memory=True)
-        host = [self._ints_host[a:b].view(t.dtype).view(t.shape) for (a, b), t in zip(views, tensors)]
+        buf = getattr(self._ints_host, "buf", None)
+        if buf is None or buf.numel() < end:
+            buf = self._ints_host.buf = torch.empty(max(end, 4096), dtype=torch.uint8, pin_memory=True)
+        host = [buf[a:b].view(t.dtype).view(t.shape) for (a, b), t in zip(views, tensors)]
         for h, t in zip(host, tensors):
             h.copy_(t, non_blocking=True)
         torch.cuda.current_stream(self.device).synchronize()

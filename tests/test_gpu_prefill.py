@@ -172,3 +172,26 @@ def test_prefill_mass_is_conserved_at_8k_chunk():
         sink_p = torch.exp(sinks.float().view(8, 8, 1) - norm)
         total += (1 - sink_p).sum((1, 2)).double().cpu()
     torch.testing.assert_close(got.cpu(), total, rtol=1e-4, atol=1e-3)
+
+
+def test_index_reads_of_two_threads_do_not_meet(monkeypatch):
+    """A second thread reads its vectors between the first one's wait and its copy to lists: each
+    gets its own values."""
+    import threading
+    from concurrent.futures import ThreadPoolExecutor
+    st = ge.state(backend())
+    mine = [torch.tensor([3, 1], device="cuda"), torch.tensor([0, 5, 9], dtype=torch.int32, device="cuda")]
+    other = [torch.tensor([7, 8], device="cuda"), torch.tensor([0, 2, 4], dtype=torch.int32, device="cuda")]
+    stream_of, main, read = torch.cuda.current_stream, threading.current_thread(), []
+    with ThreadPoolExecutor(1) as pool:
+        def current_stream(device=None):
+            stream = stream_of(device)
+
+            def synchronize():
+                stream.synchronize()
+                if threading.current_thread() is main:
+                    read.append(pool.submit(st.read_ints, *other).result())
+            return SimpleNamespace(synchronize=synchronize)
+        monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+        assert st.read_ints(*mine) == [[3, 1], [0, 5, 9]]
+    assert read == [[[7, 8], [0, 2, 4]]]
