@@ -1195,6 +1195,7 @@ extern "C" int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_s
   if (n_specs < 0 || n_specs > DIAG_MAX_SPECS) return gse_fail(GSE_EINVAL, "diagnose: 0..8 policy specs");
   if (count < 0 || prefix_len < 0 || total != prefix_len + count)
     return gse_fail(GSE_EINVAL, "diagnose: total must equal prefix_len + count");
+  if (total >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "diagnose: too many keys");  // 32-bit key indexes
   if (count == 0) return GSE_OK;
   if (q_stride_t % 8 || q_stride_h % 8 || kv_stride_s % 8 || kv_stride_h % 8)
     return gse_fail(GSE_EINVAL, "diagnose: strides must be multiples of 8 elements");

@@ -499,7 +499,7 @@ int gse_boundary_live_batch(float* scores, int layers, int64_t scores_stride_l, 
  * covers every key k <= prefix_len + i). Kind 4 (block counters, GSE_SCORE_KIND_BLOCK_STEP)
  * instead adds, per query i and whole block of keys < prefix_len + i + 1 - delay, the block's
  * maximum over its keys and all query heads of p to the block's counter (KV head 0's score of
- * the block's first slot); kv_heads <= 8 and a total below 2^31 keys.
+ * the block's first slot); kv_heads <= 8. total must be below 2^31 keys.
  * q [count, q_heads, head_dim] bf16, keys gathered through slots (int64 or
  * int32, prefix slots then the chunk's own) from the pool. head_dim = 64,
  * q_heads = 8 * kv_heads. MFMA 16x16x32 bf16 tiles, two passes (row
@@ -524,7 +524,7 @@ int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_stride_h, in
  * evicted: bit k%32 of word k/32 of row (s, g) (rows evicted_stride_g words,
  * covering total rounded up to 64); lost points at the chunk's first query
  * column; lost_scale = 1 / (q_heads * full layers). n_specs <= 8; same shape
- * limits and workspace as prefill_scores.
+ * limits, key limit and workspace as prefill_scores.
  */
 int gse_diagnose_chunk(const void* q, int64_t q_stride_t, int64_t q_stride_h, int64_t count,
                        const void* k_pool, int64_t kv_stride_s, int64_t kv_stride_h,

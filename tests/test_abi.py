@@ -183,3 +183,20 @@ def test_row_descriptors_match_the_header_layout(tmp_path):
         assert got[(cname, "size")] == ctypes.sizeof(mirror), cname
         for field, _ in mirror._fields_:
             assert got[(cname, field)] == getattr(mirror, field).offset, (cname, field)
+
+
+def test_prefill_entries_refuse_key_counts_of_2_to_the_31_without_a_gpu():
+    """Their kernels index keys in 32 bits: both entries refuse a longer list before any launch (the
+    pointers are host buffers)."""
+    if not os.path.exists(_native.LIB_PATH):
+        pytest.skip("library not built")
+    lib = _native.lib()
+    buf = ctypes.create_string_buffer(256)
+    p = ctypes.addressof(buf)
+    total, count = 1 << 31, 10
+    rc = lib.gse_prefill_scores(p, 0, 0, count, p, 0, 0, p, 0, total, total - count, p, 0, 1, p, 0, 0, 64, 8, 64,
+                                0.125, p, 1 << 30, None)
+    assert rc == 1 and b"too many keys" in lib.gse_last_error()  # GSE_EINVAL
+    rc = lib.gse_diagnose_chunk(p, 0, 0, count, p, 0, 0, p, 0, total, total - count, p, 0, p, p, 0, 0, p, 2, 0,
+                                total // 32, p, 0, 1.0, 64, 8, 64, 0.125, p, 1 << 30, None)
+    assert rc == 1 and b"too many keys" in lib.gse_last_error()
