@@ -49,36 +49,54 @@ GSE_DEVICE uint4 ld16(const uint16_t* p) { return *reinterpret_cast<const uint4*
 GSE_DEVICE int fused_chunk(int T, int P) { return (T + P - 1) / P; }
 
 // The other partition, for batches of few sequences: every workgroup's keys lie in one sequence. With
-// C = ceil(T / (P - bs)) keys per workgroup, sequence b takes ceil(len_b / C) of them, at most P in
-// all; lane b of a wave counts sequence b's. A workgroup that crosses into a second sequence starts
-// its load pipeline again (some 3 us) and ends last; here the others' chunks grow by bs / P instead,
-// which a stream bound by HBM hardly shows; and the bounds come in one vector load instead of a chain
-// of scalar ones. A replayed step of 12 layers: 4 sequences of 7,850 to 8,020 keys 303 -> 273 us, 8 of
-// 3000 to 10,200 404 -> 363, 32 of up to 4096 604 -> 545 (with 16 workgroups or more per sequence
-// only: 596), 4 of up to 1500 180 -> 147. One sequence keeps the scalar form (140 us against 147 at
-// 2252 keys).
+// C keys per workgroup, sequence b takes ceil(len_b / C) of them, at most P in all; lane b of a wave
+// counts sequence b's. A workgroup that crosses into a second sequence starts its load pipeline again
+// (some 3 us) and ends last; here the others' chunks grow by bs / P at most instead, which a stream
+// bound by HBM hardly shows; and the bounds come in one vector load instead of a chain of scalar ones.
+// C = ceil(T / (P - bs)) always fits. Where the even cut gives a workgroup at most one tile, a few keys
+// more would cost it a second tile step (4 us): there C is one tile, or, if the lists' last tiles make
+// that more than P workgroups, the cut is even (C = ceil(T / P), bounds from the lanes too).
+// Replayed steps of 12 layers, cut evenly with the bounds from scalar loads -> so: 3 lists of 720 to
+// 1200 keys 163 -> 137 us, 2 of 4000 181 -> 160 (202 in chunks of 66 keys), 8 of 3900 to 9200 387 ->
+// 359, 16 of 2047 287 -> 269, 32 of 4097 634 -> 604, 2 of 32,765 393 -> 384. Not faster: the even cut of
+// 4 lists of 16,379 keys in all 217 -> 221 (236 in chunks of 66), and lists of whole tiles, where no
+// even chunk crosses (2 of 512: 122.5 -> 125.2; 560: 155 -> 130). One sequence keeps the scalar form (140 us against 147
+// at 2252 keys).
+constexpr int SHARE_MAX_BS = 32;
 struct Share {
+  bool even;         // the even cut: workgroup w has keys [w * chunk, + chunk) of all lists
   int chunk;         // keys per workgroup
+  int total;         // keys of all lists
   int start, end;    // the lane's sequence's list
-  int mine, before;  // its workgroups, and those of the sequences before it
+  int mine, before;  // (not even) its workgroups, and those of the sequences before it
 };
 GSE_DEVICE Share sequence_shares(const int32_t* indptr, int bs, int P, int lane) {
   Share sh;
   sh.start = lane < bs ? indptr[lane] : 0;
   sh.end = lane < bs ? indptr[lane + 1] : 0;
-  const int T = __builtin_amdgcn_readlane(sh.end, bs - 1);
-  sh.chunk = max(1, (T + P - bs - 1) / (P - bs));
-  sh.mine = (sh.end - sh.start + sh.chunk - 1) / sh.chunk;
-  int upto = sh.mine;  // a scan over 32 lanes by row shifts, then lane 15's into the second row
-  upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
-  upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
-  upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
-  upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
-  upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);
-  sh.before = upto - sh.mine;
+  const int T = sh.total = __builtin_amdgcn_readlane(sh.end, bs - 1);
+  auto cut = [&](int chunk) {  // the workgroups that chunks of this many keys take
+    sh.chunk = chunk;
+    sh.mine = (sh.end - sh.start + chunk - 1) / chunk;
+    int upto = sh.mine;  // a scan over 32 lanes by row shifts, then lane 15's into the second row
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xf, 0xf, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xa, 0xf, false);
+    sh.before = upto - sh.mine;
+    return __builtin_amdgcn_readlane(upto, 31);
+  };
+  sh.even = false;
+  const int fits = max(1, (T + P - bs - 1) / (P - bs));
+  if (fits <= TILE || T > TILE * P) {
+    cut(fits);
+  } else if (cut(TILE) > P) {
+    sh.even = true;
+    sh.chunk = fused_chunk(T, P);
+  }
   return sh;
 }
-constexpr int SHARE_MAX_BS = 32;
 constexpr int SHARE_MIN_WG = 8;  // workgroups per sequence: chunks grow by at most a seventh
 
 // Largest b in [0, bs) with indptr[b] <= p (indptr non-decreasing, indptr[0] = 0 <= p).
@@ -283,27 +301,31 @@ __global__ __launch_bounds__(FUSED_THREADS) void decode_fused_kernel(FusedArgs a
   const int64_t own_row = counts ? load_index_dyn(a.rows, a.rows_dtype, w) : 0;
   int p, p_end, b, seq_end;
   int64_t slot0 = w;  // the partial of this workgroup's segment in sequence b is slot0 + b
+  auto idle = [&]() { count_steps(a, w, own_row, counts ? a.step_mode[own_row] : 0); };
   if (a.whole_seq) {
     const Share sh = sequence_shares(a.indptr, a.bs, P, lane);
-    const uint64_t own = __builtin_amdgcn_ballot_w64(sh.before <= w && w < sh.before + sh.mine);
-    if (!own) {
-      count_steps(a, w, own_row, counts ? a.step_mode[own_row] : 0);
-      return;
+    if (sh.even) {
+      p = w * sh.chunk;
+      p_end = min(p + sh.chunk, sh.total);
+      if (p >= p_end) return idle();
+      // The lists that start at or before p: the last of them holds it (lane 0's starts at 0).
+      b = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < a.bs && sh.start <= p)) - 1;
+      seq_end = __builtin_amdgcn_readlane(sh.end, b);
+    } else {
+      const uint64_t own = __builtin_amdgcn_ballot_w64(sh.before <= w && w < sh.before + sh.mine);
+      if (!own) return idle();
+      b = __builtin_ctzll(own);
+      seq_end = __builtin_amdgcn_readlane(sh.end, b);
+      p = __builtin_amdgcn_readlane(sh.start, b) + (w - __builtin_amdgcn_readlane(sh.before, b)) * sh.chunk;
+      p_end = min(p + sh.chunk, seq_end);
+      slot0 -= b;  // one segment: slot w
     }
-    b = __builtin_ctzll(own);
-    seq_end = __builtin_amdgcn_readlane(sh.end, b);
-    p = __builtin_amdgcn_readlane(sh.start, b) + (w - __builtin_amdgcn_readlane(sh.before, b)) * sh.chunk;
-    p_end = min(p + sh.chunk, seq_end);
-    slot0 -= b;  // one segment: slot w
   } else {
     const int T = a.indptr[a.bs];
     const int C = fused_chunk(T, P);
     p = w * C;
     p_end = p + C < T ? p + C : T;
-    if (p >= p_end) {
-      count_steps(a, w, own_row, counts ? a.step_mode[own_row] : 0);
-      return;
-    }
+    if (p >= p_end) return idle();
     b = seq_of(a.indptr, a.bs, p);
     seq_end = a.indptr[b + 1];
   }
@@ -629,13 +651,20 @@ __global__ __launch_bounds__(16 * HEADS * SPLIT) void decode_merge_kernel(MergeA
   const uint2 qv = *reinterpret_cast<const uint2*>(a.q + int64_t(b) * a.q_sb + int64_t(hh) * a.q_sh + 4 * j);
   const int start = a.indptr[b], end = a.indptr[b + 1];
   int wf = 1, wl = 0, slot0 = b;  // workgroup w's partial of this sequence is slot0 + w
+  int C = 0;  // keys per workgroup of the even cut
   if (a.whole_seq) {
     const Share sh = sequence_shares(a.indptr, a.bs, a.nparts, threadIdx.x & 63);
-    wf = __builtin_amdgcn_readlane(sh.before, b);
-    wl = wf + __builtin_amdgcn_readlane(sh.mine, b) - 1;
-    slot0 = 0;
+    if (sh.even) {
+      C = sh.chunk;
+    } else {
+      wf = __builtin_amdgcn_readlane(sh.before, b);
+      wl = wf + __builtin_amdgcn_readlane(sh.mine, b) - 1;
+      slot0 = 0;
+    }
   } else if (end > start) {
-    const int C = fused_chunk(a.indptr[a.bs], a.nparts);
+    C = fused_chunk(a.indptr[a.bs], a.nparts);
+  }
+  if (C && end > start) {
     wf = start / C;
     wl = (end - 1) / C;
   }
@@ -1042,7 +1071,11 @@ int decode_run(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void
   // at most bs * max_len keys (a small batch's launch is bound by each workgroup's load latency,
   // and every extra workgroup adds a partial to the merge).
   const int64_t tiles = (int64_t(bs) * std::max(max_len, 1) + TILE - 1) / TILE;
-  const int P = int(std::min<int64_t>(P_all - F, std::max<int64_t>(tiles, 1)));
+  int P = int(std::min<int64_t>(P_all - F, std::max<int64_t>(tiles, 1)));
+  // By sequence every list's last tile counts, so that chunks of one tile fit. SHARE_MIN_WG workgroups
+  // per sequence leave P - bs > 0 for its divisions.
+  const bool whole_seq = bs > 1 && bs <= SHARE_MAX_BS && bs * SHARE_MIN_WG <= P;
+  if (whole_seq) P = int(std::min<int64_t>(P_all - F, bs * ((int64_t(max_len) + TILE - 1) / TILE)));
   float* part = static_cast<float*>(workspace);
   float* norm_ws = part + (int64_t(P_all) + bs) * q_heads * PART;
   float* norm = norm_out ? norm_out : norm_ws;
@@ -1075,7 +1108,7 @@ int decode_run(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void
     f.step_count = queue_count;
     f.step_mode = mode_by_row;
   }
-  f.whole_seq = bs > 1 && bs <= SHARE_MAX_BS && bs * SHARE_MIN_WG <= P;
+  f.whole_seq = whole_seq;
   if (n_fold > 0) {
     f.fold_seq = fold_seq;
     f.n_fold = n_fold;
@@ -1132,7 +1165,7 @@ int decode_run(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void
   m.bs = bs;
   m.q_heads = q_heads;
   m.nparts = P;
-  m.whole_seq = f.whole_seq;
+  m.whole_seq = whole_seq;
   m.fold_seq = fold_seq;
   m.n_fold = n_fold;
   m.fold_buf = f.fold_buf;

@@ -485,6 +485,38 @@ def test_workgroups_of_one_sequence_each(lengths):
                 assert torch.equal(st.qq[index, rows[i], entry], q[i])
 
 
+# A workgroup's chunk never takes more 64-key tile steps than an even cut of the batch over the same
+# grid would: lists whose shares fit in whole tiles, and a batch whose shares would not (its last
+# tiles exceed the chip's workgroups) and is cut evenly.
+@pytest.mark.parametrize("lengths", [[4000] * 2, [4000] * 4, [8000, 7980], [16084, 100, 100, 100], [0, 8192, 0, 8191]])
+def test_shares_by_sequence_take_no_more_tile_steps_than_an_even_cut(lengths):
+    bs, total = len(lengths), sum(lengths)
+    b, st, q, sinks, perm, indptr, rows = _decode_setup(lengths, seed=total)
+    b.forward_metadata = SimpleNamespace(kv_indptr=indptr, kv_indices=perm)
+    fb = SimpleNamespace(out_cache_loc=torch.zeros(bs, dtype=torch.int64, device="cuda"), req_pool_indices=rows,
+                         seq_lens_cpu=torch.tensor(lengths))
+    o = torch.empty_like(q)
+    ge.decode(b, q.reshape(bs, -1), layer(1), fb, sinks, o.reshape(bs, -1))  # the workspace is there
+    ws = st._ws["decode"]
+    ws.fill_(255)  # NaN partials
+    ge.decode(b, q.reshape(bs, -1), layer(1), fb, sinks, o.reshape(bs, -1))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    grid = min(cus, -(-bs * max(lengths) // 64))
+    steps = -(-(-(-total // grid)) // 64)
+    partials = ws[:(cus + bs) * 64 * 68 * 4].view(torch.float32).view(-1, 64, 68)  # o[64], m, l, pad per head
+    used = int((~partials[:, 0, 64].isnan()).sum())
+    assert used * 64 * steps >= total
+    keys, values = (f(1) for f in (b.token_to_kv_pool.get_key_buffer, b.token_to_kv_pool.get_value_buffer))
+    for i, n in enumerate(lengths):
+        slots = perm[indptr[i]:indptr[i + 1]].long()
+        x = torch.matmul(q[i].double().view(8, 8, 64), keys[slots].double().permute(1, 2, 0).contiguous()) * 0.125
+        sink = sinks.double().view(8, 8)
+        norm = torch.logaddexp(torch.logsumexp(x, -1), sink) if n else sink
+        want = torch.matmul(torch.exp(x - norm[..., None]), values[slots].double().transpose(0, 1).contiguous())
+        # As above: bf16 probabilities and outputs.
+        torch.testing.assert_close(o[i].double(), want.reshape(64, 64), rtol=8e-3, atol=8e-3)
+
+
 @pytest.mark.parametrize("bs", [40, 5, 3, 1, 300])
 def test_merge_paths_for_many_and_few_sequences(bs):
     """The merge folds a sequence's partials in one group when there are at least 32 sequences
