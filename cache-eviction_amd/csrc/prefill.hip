@@ -81,9 +81,10 @@ static_assert(QW * WAVES == pf::QB, "a workgroup's queries");
 // Work items of a launch: about three rounds of the SLOTS workgroups the chip holds (2 per CU). Where
 // these have FEW_TILES tiles or less each to do, whole rounds count: then the item length (at least
 // MIN_TILES tiles) whose rounds take least, with the start of an item (its query and first key loads,
-// some 4 us) counted as START tiles. Both passes, 2048 tokens without a prefix: 96 us with items of 8
-// tiles (1.25 rounds), 88 in one round; 60 after 1000 33 -> 29; 190 after 7000 61 -> 56. Past that the
-// rounds' count no longer decides (8192 after 28,672: 5.45 ms, 5.8 with the fewest rounds).
+// some 4 us) counted as START tiles. Both passes of sums, without the rule -> with it, us: 2047 tokens
+// without a prefix 87.2 -> 86.1, 1000 after 1000 67.8 -> 63.3, 400 after 4096 70.4 -> 64.9, 400 after 9000
+// 120 -> 111; 1000 without a prefix 45.0 -> 44.9. Past that the rounds' count no longer decides (8192
+// after 28,672: 5.45 ms, 5.8 with the fewest rounds).
 constexpr int SLOTS = 512;
 constexpr int ITEMS = 3 * SLOTS;
 constexpr int FEW_TILES = 16;
@@ -408,13 +409,23 @@ constexpr int WAVES = 4;
 constexpr int KB = KW * WAVES;
 constexpr int THREADS = 64 * WAVES;
 constexpr int QT = 8;  // queries per tile (64 rows)
-// Work items of a launch and the rule for few tiles as in p1 (4 workgroups per CU), the fewest queries
-// of an item, and the most: a sum takes at most MAX_QUERIES / 4 additions in one register, so its
-// rounding error stays near that of a sum over 64-query blocks.
-constexpr int SLOTS = 1024;
+// Query blocks: about ITEMS workgroups, of at least 64 queries and at most MAX_QUERIES: a sum takes at
+// most MAX_QUERIES / 4 additions in one register, so its rounding error stays near that of a sum over
+// 64-query blocks. Two exceptions, by the workgroups that have keys to credit:
+// - Fewer than FEW (7 for 4 CUs): a workgroup has its CU nearly to itself and its walk is the launch, so
+//   the blocks shrink (to MIN_QUERIES, by a quarter at least) as long as there are no more than FEW. Both
+//   passes, sums / maxima, us: 60 tokens without a prefix 24.0 -> 17.9 / 20.2 -> 15.8, 850 without one
+//   38.3 -> 34.1 / 33.7 -> 31.8, 190 after 1000 32.8 -> 28.4 / 30.1 -> 27.9. With more of them shorter
+//   walks no longer pay for their starts and atomics: 1000 without a prefix, 640 workgroups instead of
+//   320, 44.6 -> 45.3 / 40.4 -> 45.4.
+// - Blocks of 64 in up to 13/8 rounds of the SLOTS workgroups that run at once: longer ones in one round,
+//   if they fill it (7/8): 2047 without a prefix 92.6 -> 86.4, 1000 after 2500 100.5 -> 95.9 / 90.7 -> 86.4;
+//   not 300 after 9000 (872 workgroups) 85.2 -> 91.5. Maxima only from 5/4 rounds on: at 1152 workgroups
+//   79.0 -> 80.1, at 1048 69.2 -> 70.5.
+constexpr int SLOTS = 1024;  // 4 workgroups per CU
 constexpr int ITEMS = 2 * SLOTS;
-constexpr int FEW_TILES = 20;
-constexpr double START = 1.5;
+constexpr int FEW = 448;
+constexpr int ROUND = SLOTS * 13 / 8;
 constexpr int MIN_QUERIES = 32;
 constexpr int MAX_QUERIES = 512;
 }  // namespace p2
@@ -1155,24 +1166,28 @@ extern "C" int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_s
   auto block_of = [&](int64_t n) {  // queries of one of n blocks
     return std::min<int64_t>(((count + n - 1) / n + p2::QT - 1) / p2::QT * p2::QT, p2::MAX_QUERIES);
   };
+  // Workgroups that credit keys: the key blocks that only part of the chunk credits have fewer query blocks.
+  auto live = [&](int64_t qblock) {
+    const int64_t nq = (count + qblock - 1) / qblock;
+    int64_t n = 0;
+    for (int64_t k = 0; k < nkb && k * p2::KB - bound0 < count; ++k)
+      n += std::max<int64_t>(0, nq - std::max<int64_t>(0, k * p2::KB - bound0) / qblock);
+    return n * kv_heads;
+  };
   const int64_t nqmax = (count + p2::MIN_QUERIES - 1) / p2::MIN_QUERIES;
-  a.qblock = int(block_of(std::min(std::max<int64_t>(1, p2::ITEMS / (nkb * kv_heads)), (nqmax + 1) / 2)));
-  // As for pass 1, few tiles per workgroup: the query block whose rounds take least. The key blocks that
-  // only part of the chunk credits have fewer query blocks.
-  if (nkb * kv_heads * ((count + p2::QT - 1) / p2::QT) <= p2::FEW_TILES * p2::SLOTS) {
-    double best = 0;
-    for (int64_t n = (count + p2::MAX_QUERIES - 1) / p2::MAX_QUERIES, first = n; n <= nqmax; n += 1 + n / 16) {
-      const int64_t qblock = block_of(n), nq = (count + qblock - 1) / qblock;
-      int64_t live = 0;
-      for (int64_t k = 0; k < nkb; ++k)
-        live += std::max<int64_t>(0, nq - std::max<int64_t>(0, k * p2::KB - bound0) / qblock);
-      const double cost = double((live * kv_heads + p2::SLOTS - 1) / p2::SLOTS) * (double(qblock) / p2::QT + p2::START);
-      if (n == first || cost < best) {
-        best = cost;
-        a.qblock = int(qblock);
-      }
-    }
+  const int64_t common = std::min(std::max<int64_t>(1, p2::ITEMS / (nkb * kv_heads)), (nqmax + 1) / 2);
+  const int64_t wgs = nkb * kv_heads <= p2::ROUND ? live(block_of(common)) : p2::ROUND + 1;
+  int64_t blocks = common;
+  if (wgs < p2::FEW) {
+    for (int64_t n = nqmax; n > blocks && block_of(n) * 4 <= block_of(common) * 3; --n)
+      if (live(block_of(n)) <= p2::FEW) blocks = n;
+  } else if (common == (nqmax + 1) / 2 && wgs > (kind == 2 ? p2::SLOTS * 5 / 4 : p2::SLOTS) && wgs <= p2::ROUND) {
+    int64_t n = common - 1;
+    while (n > 1 && live(block_of(n)) > p2::SLOTS) --n;
+    const int64_t one = n > 0 ? live(block_of(n)) : 0;
+    if (one <= p2::SLOTS && one * 8 >= p2::SLOTS * 7) blocks = n;
   }
+  a.qblock = int(block_of(blocks));
   const int64_t items = nkb * ((count + a.qblock - 1) / a.qblock) * kv_heads;
   if (items >= (int64_t(1) << 31)) return gse_fail(GSE_EINVAL, "prefill: chunk too large");
   if (kind == 2)

@@ -90,6 +90,16 @@ def test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, scal
     torch.testing.assert_close(st.scores[0][:, slots].double(), want, rtol=1e-5 + largest * 2 ** -22, atol=1e-7)
 
 
+# Both sides of pass 2's query-block rules: shorter blocks while few workgroups have work (60 and 850
+# queries, not 1000), and longer ones in one round instead of a part of a second (2047, 1000 after
+# 2500; 300 after 9000 would not fill it).
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("count,prefix_len", [(60, 0), (850, 0), (1000, 0), (780, 300), (2047, 0), (1000, 2500),
+                                              (300, 9000)])
+def test_prefill_scores_by_query_block_rule(count, prefix_len, mode):
+    test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, 1, mode)
+
+
 @pytest.mark.parametrize("n,m,first,second", [
     (0, 1, torch.int32, torch.int64), (255, 1, torch.int32, torch.int64), (1, 256, torch.int64, torch.int32),
     (300, 0, torch.int64, torch.int64), (257, 513, torch.int16, torch.int32)])
