@@ -26,13 +26,6 @@ HIPCC_FLAGS = [
 ]
 
 
-# Per-source additions. prefill.hip: keep MFMA results in ordinary VGPRs. With the compiler's
-# own choice the pass-2 tile kept them in accumulation registers and paid one v_accvgpr_read per
-# logit (a fifth vector issue slot beside the FMA, the exp2 and the add); forcing the VGPR form
-# removed them without spills (measured: 290 -> 302 TFLOP/s at the 79,720-token prompt).
-SOURCE_FLAGS = {"prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
-
-
 def hipcc() -> str:
     path = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(path):
@@ -41,7 +34,7 @@ def hipcc() -> str:
 
 
 def _compile(src: Path, obj: Path, verbose: bool) -> None:
-    cmd = [hipcc(), *HIPCC_FLAGS, *SOURCE_FLAGS.get(src.name, []), "-c", str(src), "-o", str(obj)]
+    cmd = [hipcc(), *HIPCC_FLAGS, "-c", str(src), "-o", str(obj)]
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, capture_output=True, text=True)
