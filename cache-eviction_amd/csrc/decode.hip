@@ -60,8 +60,8 @@ GSE_DEVICE int fused_chunk(int T, int P) { return (T + P - 1) / P; }
 // 1200 keys 163 -> 137 us, 2 of 4000 181 -> 160 (202 in chunks of 66 keys), 8 of 3900 to 9200 387 ->
 // 359, 16 of 2047 287 -> 269, 32 of 4097 634 -> 604, 2 of 32,765 393 -> 384. Not faster: the even cut of
 // 4 lists of 16,379 keys in all 217 -> 221 (236 in chunks of 66), and lists of whole tiles, where no
-// even chunk crosses (2 of 512: 122.5 -> 125.2; 560: 155 -> 130). One sequence keeps the scalar form (140 us against 147
-// at 2252 keys).
+// even chunk crosses (2 of 512: 122.5 -> 125.2; 560: 155 -> 130). One sequence keeps the scalar form
+// (140 us against 147 at 2252 keys).
 constexpr int SHARE_MAX_BS = 32;
 struct Share {
   bool even;         // the even cut: workgroup w has keys [w * chunk, + chunk) of all lists
@@ -1294,11 +1294,10 @@ extern "C" int gse_decode_scores_from_lse(const void* q, int64_t q_stride_b, int
                                           const void* sinks, int sinks_dtype, const int32_t* mode_by_row,
                                           const void* rows, int rows_dtype, float* scores,
                                           int64_t scores_stride_g, int64_t scores_stride_s, int bs, int q_heads,
-                                          int kv_heads, int head_dim, float sm_scale, int max_len, void* workspace,
-                                          int64_t workspace_bytes, gse_stream_t stream) {
+                                          int kv_heads, int head_dim, float sm_scale, int max_len, void*, int64_t,
+                                          gse_stream_t stream) {
   if (int rc = check_decode_shape(q_heads, kv_heads, head_dim)) return rc;
   if (bs <= 0) return bs < 0 ? gse_fail(GSE_EINVAL, "scores_from_lse: bs < 0") : GSE_OK;
-  if (workspace_bytes < int64_t(bs) * q_heads * 4) return gse_fail(GSE_EWORKSPACE, "scores_from_lse: workspace");
   if (max_kv_splits < 1 || min_block_kv < 1) return gse_fail(GSE_EINVAL, "scores_from_lse: split layout");
   if (!q || !k_pool || !kv_indptr || !kv_indices || !attn_lse || !num_kv_splits || !sinks || !mode_by_row || !rows ||
       !scores)

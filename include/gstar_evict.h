@@ -329,7 +329,8 @@ int gse_score_flush_logits(void* const* k_pools, int layers, int64_t kv_stride_s
  * max_kv_splits] (strides in elements) over the valid splits of SGLang's layout
  * per = cdiv(cdiv(len, num_kv_splits[b]), min_block_kv) * min_block_kv, started
  * at (sink, 1) (R:180-188), then every resident key's probability is added.
- * max_len bounds every sequence's list length; workspace holds bs * q_heads floats.
+ * max_len bounds every sequence's list length (it sizes the grid). The pass forms the normalisers
+ * itself: workspace is not used and may be null.
  */
 int gse_decode_scores_from_lse(const void* q, int64_t q_stride_b, int64_t q_stride_h,
                                const void* k_pool, int64_t kv_stride_s, int64_t kv_stride_h,
@@ -503,7 +504,10 @@ int gse_boundary_live_batch(float* scores, int layers, int64_t scores_stride_l, 
  * q [count, q_heads, head_dim] bf16, keys gathered through slots (int64 or
  * int32, prefix slots then the chunk's own) from the pool. head_dim = 64,
  * q_heads = 8 * kv_heads. MFMA 16x16x32 bf16 tiles, two passes (row
- * log-sum-exp, then column sums). Needs workspace for the row normalisers.
+ * log-sum-exp, then column sums). The workspace holds the row normalisers
+ * (count * q_heads floats, rounded up to 256 bytes: the least that is accepted)
+ * and pass 1's (reference, sum) pairs of each row and key range; one smaller
+ * than gse_prefill_workspace_bytes takes fewer key ranges.
  */
 int64_t gse_prefill_workspace_bytes(int64_t count, int q_heads);
 int gse_prefill_scores(const void* q, int64_t q_stride_t, int64_t q_stride_h, int64_t count,
@@ -553,7 +557,10 @@ int gse_pack_evicted(const void* resident, int64_t resident_stride_s, int64_t re
  * retained_stride_g apart) lie below frontier <= start. retained_count = 0
  * (nothing evicted yet) gives error 0. head_dim = 64, q_heads = 8 * kv_heads.
  * MFMA 16x16x32 bf16 tiles with a single-pass online softmax; probabilities
- * enter the value product as bf16 hi + lo parts.
+ * enter the value product as bf16 hi + lo parts. retained_count + start + count
+ * must be below 2^31. The workspace holds both outputs, per key range where a
+ * short chunk's keys are split; a smaller one than gse_replay_workspace_bytes
+ * takes fewer ranges, down to the two outputs alone.
  */
 int64_t gse_replay_workspace_bytes(int64_t count, int q_heads);
 int gse_replay_layer_difference(const void* q, int64_t q_stride_t, int64_t q_stride_h, int64_t count,
