@@ -100,6 +100,29 @@ def test_prefill_scores_by_query_block_rule(count, prefix_len, mode):
     test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, 1, mode)
 
 
+# The hooks build 32-bit slot lists; the entry also takes 64-bit ones, for every kind (sums, maxima,
+# block counters of 4 keys 100 entries late) and more than one key range.
+@pytest.mark.parametrize("mode", [1, 2, 4 | 2 << 4 | 100 << 8])
+@pytest.mark.parametrize("count,prefix_len", [(70, 1500), (513, 0)])
+def test_prefill_scores_of_64_bit_slot_lists(count, prefix_len, mode):
+    from gstar_evict import _native as N
+    b, st, q, sinks, prefix, new = _case(count, prefix_len, seed=31)
+    keys = b.token_to_kv_pool.get_key_buffer(1)
+    ws = torch.empty(N.lib().gse_prefill_workspace_bytes(count, 64), dtype=torch.uint8, device="cuda")
+    got = []
+    for slots in (torch.cat((prefix, new)).int(), torch.cat((prefix, new)).long()):
+        sc = torch.zeros_like(st.scores[0])
+        N.call("gse_prefill_scores", N.ptr(q), q.stride(0), q.stride(1), count, N.ptr(keys), keys.stride(0),
+               keys.stride(1), N.ptr(slots), N.idx_code(slots), slots.numel(), prefix_len, N.ptr(sinks),
+               N.float_code(sinks), mode, N.ptr(sc), sc.stride(0), sc.stride(1), 64, 8, 64, 0.125, N.ptr(ws),
+               ws.numel(), N.stream())
+        got.append(sc)
+    assert float(got[0].sum()) > 0
+    # The same sums, added in another order by the atomics: at most 2^-24 of the sum for each of the
+    # query blocks (one per 32 queries at most).
+    torch.testing.assert_close(got[1], got[0], rtol=17 * 2 ** -24, atol=0)
+
+
 @pytest.mark.parametrize("n,m,first,second", [
     (0, 1, torch.int32, torch.int64), (255, 1, torch.int32, torch.int64), (1, 256, torch.int64, torch.int32),
     (300, 0, torch.int64, torch.int64), (257, 513, torch.int16, torch.int32)])
