@@ -242,11 +242,20 @@ struct KeyTiles {
   GSE_DEVICE void stage(int p, Tile (&tiles)[2]) { store(tiles[p], row[p]); }
 };
 
+// m + log2(l), rounded once: the exponent of l joins m without loss and only the mantissa's logarithm,
+// in [-1, 0), is inexact (log2(l) itself, 6 to 16 for the sums here, is rounded to 2^-21 or 2^-20).
+GSE_DEVICE float add_log2(float m, float l) {
+  const float e = float(__builtin_amdgcn_frexp_expf(l));
+  const float s = m + e, t = s - m;
+  const float lost = (m - (s - t)) + (e - t);
+  return s + (__log2f(__builtin_amdgcn_frexp_mantf(l)) + lost);
+}
+
 // A row's normaliser (log2 units) from its one pair and the sink.
 GSE_DEVICE float row_norm(const PrefillArgs& a, int h, float ref, float sum) {
   const float sink2 = load_float_dyn(a.sinks, a.sinks_dtype, h) * kLog2e;
   const float m = fmaxf(ref, sink2);
-  return m + __log2f(sum * fast_exp2(ref - m) + fast_exp2(sink2 - m));
+  return add_log2(m, sum * fast_exp2(ref - m) + fast_exp2(sink2 - m));
 }
 
 __global__ __launch_bounds__(p1::THREADS, 4) void prefill_norm_kernel(PrefillArgs a) {
@@ -388,7 +397,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
     for (int j = 0; j < 8; ++j) l += s0 + j < ranges ? p[j].y * fast_exp2(p[j].x - mn) : 0.f;
     m = mn;
   }
-  a.norm2[t] = m + __log2f(l);
+  a.norm2[t] = add_log2(m, l);
 }
 
 // ---------------------------------------------------------------------------

@@ -100,6 +100,22 @@ def test_prefill_scores_by_query_block_rule(count, prefix_len, mode):
     test_prefill_scores_at_the_edges_of_tiles_and_ranges(count, prefix_len, 1, mode)
 
 
+@pytest.mark.parametrize("count,prefix_len", [(300, 0), (1000, 2500), (500, 9000)])
+def test_normalisers_are_rounded_once(count, prefix_len):
+    """A column sums thousands of rows' probabilities. One rounding of each normaliser (at most 2^-21
+    in log2 units here) is as often up as down and all but cancels in it, as the exponentials' do, so
+    what is left lies below 2^-23 in relative 2-norm; a logarithm with an error of its own does not
+    cancel (2e-7)."""
+    b, st, q, sinks, prefix, new = _case(count, prefix_len, seed=41)
+    keys = b.token_to_kv_pool.get_key_buffer(1)
+    slots = torch.cat((prefix, new)).long()
+    st.scores.zero_()
+    ge._prefill_scores(st, 0, 1, layer(1), q / 1.5, keys, sinks, prefix, new)
+    want = _exact_scores(1, q / 1.5, keys, sinks, slots, prefix_len)
+    got = st.scores[0][:, slots].double()
+    assert float((got - want).norm() / want.norm()) < 2 ** -23
+
+
 # The hooks build 32-bit slot lists; the entry also takes 64-bit ones, for every kind (sums, maxima,
 # block counters of 4 keys 100 entries late) and more than one key range.
 @pytest.mark.parametrize("mode", [1, 2, 4 | 2 << 4 | 100 << 8])
