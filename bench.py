@@ -699,7 +699,7 @@ def prefill_bench(args, torch, ge):
                    "causal_pairs_per_layer": pairs},
         "roofline": {"bound": "mfma", "achieved": round(tflops, 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / PEAK_BF16_TFLOPS, 4), "issued_frac": round(2 * tflops / PEAK_BF16_TFLOPS, 4),
-                     # HBM bytes per (chunk, layer) score launch pair, from the committed profile of the
+                     # HBM bytes per (chunk, layer) of the score launches, from the committed profile of the
                      # default --prefill workload.
                      "traffic": measured_traffic("prefill_kernel_79720.md") if prefill_default(args) else None},
         "cpu_baseline": baseline,

@@ -811,9 +811,10 @@ GSE_DEVICE float norm_from_lse(const ScoreArgs& a, int b, int g, int len) {
 // Kind 4 (block counters): per key the maximum over the KV heads and per block the maximum over its
 // keys (lane swaps: blocks of at most 64 entries are aligned lane groups of a wave), added to KV
 // head 0's score of the block's first slot.
-// Bound by HBM; 8 lists of 4 to 18 thousand keys (115 MB), with the clearing of the new slots: 46.9
-// us (a kernel of its own for the normalisers, workgroups sized by the batch's longest possible
-// list, a wave's share of a score row at a time) -> 29.0 us; 32 lists, 1.1 GB: 376 -> 235 us.
+// Bound by HBM where a batch exceeds the 256 MB last-level cache: 32 lists, 1.1 GB: 375 -> 237 us with the
+// clearing of the new slots (a kernel of its own for the normalisers, workgroups sized by the batch's
+// longest possible list, a wave's share of a score row at a time), 4.6 TB/s. 8 lists of 4 to 18 thousand
+// keys (115 MB): 52.8 -> 36.1 us among other batches (four in turn), 47.3 -> 29.1 us over the same one.
 template <typename IdxT>
 __global__ __launch_bounds__(512) void decode_score_kernel(ScoreArgs a) {
   __shared__ float totals[2][SCORE_TILE][MAX_KVH + 1];

@@ -71,14 +71,16 @@ struct PrefillArgs {
 // mix alone runs at 2.2 GHz, 139 ns per 1024 logits; 32x32x16 MFMAs take fewer issue slots but
 // more power (156 ns), and the FMA with a vector instead of a scalar scale 147 ns. Against rows
 // spread over 16 lanes (a running maximum per row and lane) with 2 waves per SIMD and whole causal
-// ranges: 87 -> 43 us for the first 2048 tokens of a prompt, 816 -> 640 us for 1896 tokens after
-// 30,720, 3.36 -> 2.75 ms for 8192 after 28,672.
+// ranges, means of 20 traced calls in a row, the join of the ranges included: 82 -> 51 us for the first
+// 2048 tokens of a prompt, 738 -> 652 us for 1896 tokens after 30,720, 2.91 -> 2.54 ms for 8192 after
+// 28,672. Single calls between waits run at another clock (790 us for the second), and another card's
+// power limit made the passes 6 % slower.
 namespace p1 {
 constexpr int QW = 8;                // queries per wave: two column blocks of 4 queries x 8 heads
 constexpr int WAVES = 8;
 constexpr int THREADS = 64 * WAVES;
 static_assert(QW * WAVES == pf::QB, "a workgroup's queries");
-// Work items of a launch: about three rounds of the SLOTS workgroups the chip holds (2 per CU). Where
+// Work items of a launch: about three rounds of the SLOTS workgroups that 256 CUs hold (2 each). Where
 // these have FEW_TILES tiles or less each to do, whole rounds count: then the item length (at least
 // MIN_TILES tiles) whose rounds take least, with the start of an item (its query and first key loads,
 // some 4 us) counted as START tiles. Both passes of sums, without the rule -> with it, us: 2047 tokens
@@ -408,10 +410,10 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
 // whole walk and reaches the score table with one atomic per (key, query block), and no key index
 // is read inside it. Sum mode forms S^T = K . Q^T (a lane holds 16 keys of one row: one normaliser,
 // a sum per key), max mode S = Q . K^T (a lane holds 4 heads of a query for one key: the maximum
-// over the heads is in the lane and its neighbouring group). 4 waves per SIMD. Bound as pass 1;
-// max mode takes one exponential per (query, key). Against query blocks of 64 walking the keys (column sums through LDS rings, two
-// waves per SIMD): sums 77 -> 44 us for the first 2048 tokens of a prompt, 3.4 -> 2.5 ms for 8192
-// tokens after 28,672; maxima 1120 -> 450 us for 1896 after 30,720.
+// over over the heads is in the lane and its neighbouring group). 4 waves per SIMD. Bound as pass 1;
+// max mode takes one exponential per (query, key). Against query blocks of 64 walking the keys (column
+// sums through LDS rings, two waves per SIMD), traced as pass 1: sums 74 -> 44 us for the first 2048
+// tokens of a prompt, 3.01 -> 2.65 ms for 8192 after 28,672; maxima 1053 -> 494 us for 1896 after 30,720.
 namespace p2 {
 constexpr int KW = 64;  // keys per wave: two 32-key blocks
 constexpr int WAVES = 4;
@@ -431,7 +433,7 @@ constexpr int QT = 8;  // queries per tile (64 rows)
 //   if they fill it (7/8): 2047 without a prefix 92.6 -> 86.4, 1000 after 2500 100.5 -> 95.9 / 90.7 -> 86.4;
 //   not 300 after 9000 (872 workgroups) 85.2 -> 91.5. Maxima only from 5/4 rounds on: at 1152 workgroups
 //   79.0 -> 80.1, at 1048 69.2 -> 70.5.
-constexpr int SLOTS = 1024;  // 4 workgroups per CU
+constexpr int SLOTS = 1024;  // 4 workgroups on each of 256 CUs
 constexpr int ITEMS = 2 * SLOTS;
 constexpr int FEW = 448;
 constexpr int ROUND = SLOTS * 13 / 8;
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(p2::THREADS, 4) void prefill_score_kernel(PrefillAr
 // Bound by the matrix units beside vector issue: per 1024 logits 8 MFMAs (132 cycles), 16 FMAs and 8
 // three-way maxima. 2048 queries after 12,288 keys, blocks of 4: 630 us with a wave per KV head and
 // an LDS atomic maximum per lane and 16x16 block, 414 with plain LDS maxima and a barrier per 64
-// keys, 314 us so (2.1 GHz: the power limit).
+// keys, 314 us so (2.1 GHz: the power limit; 287 in a row, 597 the first form).
 namespace pb {
 constexpr int QB = pf::QB;      // queries per workgroup
 constexpr int QW = 8;           // queries per wave
@@ -899,7 +901,7 @@ __global__ __launch_bounds__(256) void pack_evicted_kernel(const uint8_t* reside
 // swaps, then through a column per wave in LDS (float atomics there took 194 cycles each, half the
 // kernel). NS, the number of specs, is a template argument: a run-time bound on
 // the unrolled spec loop cost a branch per (spec, 16x16 block). Vector issue bound as pass 1; 2048
-// queries after 14,336 keys, 4 specs: 1292 -> 684 us, 65 % of the cycles issuing (2 waves per SIMD).
+// queries after 14,336 keys, 4 specs: 1249 -> 619 us (20 calls in a row), 65 % of the cycles issuing (2 waves per SIMD).
 template <int NS>
 __global__ __launch_bounds__(p1::THREADS, NS == 0 ? 4 : 2) void diagnose_kernel(DiagArgs da) {
   using namespace pf;

@@ -17,7 +17,7 @@
 // are read from LDS where they are used, which leaves 128 registers and 4 waves per SIMD, so that
 // one wave's MFMAs run beside another's vector work. Bound by the card's power: 24 MFMAs per 1024
 // logits cost 200 ns per SIMD by themselves, their exponentials and splits 140 (1.95 GHz). Both
-// outputs and the errors, 2048 queries after 16,384 keys (2048 retained): 1066 -> 969 us; 150
+// outputs and the errors, 2048 queries after 16,384 keys (2048 retained): 1107 -> 1029 us (20 calls in a row); 150
 // queries after 8192, whose 40 workgroups now split their keys: 276 -> 80 us; 17 after 28,672: 770 -> 66.
 //
 // Key columns: column c < n_retained is key row retained[g][c]; column c >= n_retained is key
