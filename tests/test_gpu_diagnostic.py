@@ -179,3 +179,20 @@ def test_chunk_of_any_spec_count_against_64_bits(runtime, specs, count, start):
     torch.testing.assert_close(entry["score_sum"][0].double(), sums, **tol)
     torch.testing.assert_close(entry["score_max"][0].double(), maxes, **tol)
     torch.testing.assert_close(entry["lost"].double(), lost, **tol)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 300])
+@pytest.mark.parametrize("form", ["bool", "table", "transposed", "int32"])
+def test_evicted_words_of_any_mask(runtime, n, form):
+    """Masks of any layout and type pack alike: one that ends before its table does, one whose
+    positions are not side by side, one of 32-bit numbers."""
+    from gstar_evict import diagnostics
+    g = torch.Generator(device="cuda").manual_seed(n)
+    held = torch.rand((3, 8, n), generator=g, device="cuda") < 0.5
+    mask = {"bool": held, "table": torch.cat((held, torch.ones((3, 8, 77), dtype=torch.bool, device="cuda")), -1)[..., :n],
+            "transposed": held.transpose(0, 2).contiguous().transpose(0, 2), "int32": held.to(torch.int32) * 256}[form]
+    words = diagnostics.evicted_words(mask).cpu().numpy().view(np.uint8)
+    bits = np.unpackbits(words, axis=-1, bitorder="little")
+    assert words.shape[-1] == -(-n // 64) * 8
+    assert np.array_equal(bits[..., :n].astype(bool), ~held.cpu().numpy())
+    assert not bits[..., n:].any()
