@@ -119,7 +119,8 @@ GSE_DEVICE void replay_tile(const bf16x8_t (&qa)[rp::RB][2], const uint16_t* kt,
   for (int rb = 0; rb < RB; ++rb) {
     // p = 2^(x*scale2 - ref). A lane whose 16 values sum past kRescaleSum may hold one 2^8 above
     // the reference: then (rarely, wave-uniform) the reference moves to the column's maximum over
-    // the tile, and the terms are formed again from the products.
+    // the tile, and the terms are formed again from the products. References are whole numbers, so
+    // that what a move or the join of key ranges scales by is a power of two and exact.
     auto expo = [&]() {
       float t[4];
 #pragma unroll
@@ -140,7 +141,7 @@ GSE_DEVICE void replay_tile(const bf16x8_t (&qa)[rp::RB][2], const uint16_t* kt,
         s[rb][kb] = dot(kf, rb, kb);
         tmax = fmaxf(fmaxf(tmax, fmaxf(s[rb][kb][0], s[rb][kb][1])), fmaxf(s[rb][kb][2], s[rb][kb][3]));
       }
-      tmax = xor32_max(xor16_max(tmax)) * scale2;  // the column's maximum over the tile (scale > 0)
+      tmax = rintf(xor32_max(xor16_max(tmax)) * scale2);  // the column's maximum over the tile (scale > 0)
       const float nr = fmaxf(ref[rb], tmax);
       const float corr = fast_exp2(ref[rb] - nr);
       ref[rb] = nr;
@@ -350,7 +351,7 @@ __global__ __launch_bounds__(64 * rp::WAVES, 4) void replay_output_kernel(Replay
 GSE_DEVICE float4 replay_join(const ReplayArgs& a, const ReplaySide& sd, int64_t i, int h, int piece) {
   if (a.splits == 1) return *reinterpret_cast<const float4*>(sd.o + (i * a.q_heads + h) * rp::D + 4 * piece);
   const int ranges = replay_ranges(replay_tiles(sd, a.count, i / rp::QB * rp::QB), a.splits);
-  float m = load_float_dyn(a.sinks, a.sinks_dtype, h) * kLog2e, l = 1.f;
+  float m = -1e30f, l = 0.f;
   float4 o = {0.f, 0.f, 0.f, 0.f};
   constexpr int B = 8;
   for (int s0 = 0; s0 < ranges; s0 += B) {
@@ -376,7 +377,8 @@ GSE_DEVICE float4 replay_join(const ReplayArgs& a, const ReplaySide& sd, int64_t
     }
     m = mn;
   }
-  const float inv = 1.f / l;
+  // The sink joins last: the ranges' weights stay whole powers of two.
+  const float inv = 1.f / (l + fast_exp2(load_float_dyn(a.sinks, a.sinks_dtype, h) * kLog2e - m));
   return {o.x * inv, o.y * inv, o.z * inv, o.w * inv};
 }
 

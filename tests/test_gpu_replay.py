@@ -112,6 +112,29 @@ def test_layer_difference_over_key_ranges(runtime, monkeypatch, start, count, fr
     np.testing.assert_allclose(got, _oracle(q, k, v, sinks, entry, start), rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("start,count,kept", [(6144, 700, 4096), (4096, 1000, 2048), (8192, 300, 2048)])
+def test_joining_key_ranges_adds_no_error(runtime, monkeypatch, start, count, kept):
+    """Ranges' references are whole numbers, so the weights that join them are exact: the errors over
+    two to six ranges and over one (a workspace of the two outputs alone) differ by the order of the
+    32-bit sums only."""
+    gen = torch.Generator().manual_seed(start + count)
+    k, v = (torch.randn((start + count, KV_HEADS, DIM), generator=gen).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn((count, HEADS, DIM), generator=gen).to(torch.bfloat16)
+    sinks = torch.randn(HEADS, generator=gen)
+    entry = {"frontier": start, "count": kept, "pos": _retained(start, kept, gen)}
+    many = _run(runtime, q, k, v, sinks, dict(entry), start)
+    st = runtime.state(backend(rows=2, width=64, slots=16, layers=2, full=(1,)))
+    size = 2 * -(-count * HEADS * DIM * 4 // 256) * 256
+    monkeypatch.setattr(type(st), "workspace", lambda self, name, nbytes: torch.empty(size, dtype=torch.uint8,
+                                                                                     device="cuda"))
+    one = _run(runtime, q, k, v, sinks, dict(entry), start)
+    # What the order of the sums leaves: an output is some hundred tiles' products in 32 bits, 2^-24 of it
+    # each and as often up as down, beside errors |b - a| of some tenths of |a|, whose norm over 4096
+    # values averages it again (0.8e-7 seen). Weights off by 2^-24 for a whole range do not average (2.5e-7).
+    difference = float(np.linalg.norm(many.astype(np.float64) - one) / np.linalg.norm(one))
+    assert difference < 2 ** -23, difference
+
+
 def test_layer_difference_is_zero_before_any_eviction(runtime):
     gen = torch.Generator().manual_seed(9)
     k, v, direction = _shadow(700, gen)
